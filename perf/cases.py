@@ -537,12 +537,13 @@ def _attenuated_exact(case, problem):
         it = torch.round(((r * 1000.0) / cp - problem["delay"][p]) / step)
         ai = (case["step"] ** 2) / (2 * math.pi * r) / dt * 1000.0
         ok = (it >= 0) & (it < nt)
-        r, it, ai = r[ok] * 1e-3, it[ok] * dt_s, ai[ok]
+        r, it, ai = r[ok] * 1e-3, it[ok], ai[ok]
         spec[p, 0] = ai.sum()
         for c0 in range(0, r.numel(), 1 << 16):
-            rc, tc, ac = (v[c0:c0 + (1 << 16), None] for v in (r, it, ai))
+            rc, ic, ac = (v[c0:c0 + (1 << 16), None] for v in (r, it, ai))
             mag = ac * torch.exp(-rc * al * w / (2 * math.pi))
-            arg = -w * rc * al / math.pi ** 2 * b - tc * w
+            # The delay's phase 2 pi it k / nt, reduced before it is rounded.
+            arg = -w * rc * al / math.pi ** 2 * b - (ic * k % nt) * (2 * math.pi / nt)
             spec[p, 1:] += torch.complex((mag * torch.cos(arg)).sum(0),
                                          (mag * torch.sin(arg)).sum(0))
     return torch.fft.irfft(spec, n=nt)
