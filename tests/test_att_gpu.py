@@ -124,3 +124,27 @@ def test_device_entry_point_with_attenuation(gpu, oracle):
                                         nthreads=2, alpha=4.0)
     H, code, n_oob = sir_attenuated(dict(base, shape="circ", R=0.5), 4.0)
     assert _close(H.cpu().numpy().T, ref) and code == e and n_oob == oob
+
+
+@pytest.mark.parametrize("alpha,delay,nt", [
+    (0.5, None, 160),       # 8 moments, the per-sample table
+    (20.0, None, 161),      # 12 moments
+    (60.0, None, 160),      # two sub-cells per sample, no table
+    (900.0, None, 160),     # many sub-cells, everything but near samples gone
+    (40.0, -45.0, 1200),    # a far negative delay: factors evaluated per cell
+    (5.0, 2.0, 700),        # an element over more than one window of 256 samples
+])
+def test_attenuated_moments(gpu, oracle, alpha, delay, nt):
+    """The moment expansion's terms, sub-cells, windows and table rule."""
+    from dream_amd.dreamrect import dreamrect
+    wide = nt == 700
+    No = 3 if wide else 40
+    rng = np.random.default_rng(37)
+    Ro = np.c_[rng.uniform(-2, 2, No), rng.uniform(-1, 1, No), rng.uniform(4, 7, No)]
+    dt = 0.02 if wide else 0.05
+    geom, step = ([16.0, 4.0], 0.4) if wide else ([0.8, 1.2], 0.1)
+    d = Ro[:, 2] * 1000.0 / CP - 1.0 if delay is None else delay
+    H = dreamrect(Ro, geom, [step, step, dt, nt], d, [1.0, CP, alpha], "ignore")
+    ref, _, _ = oracle.dreamrect(Ro, *geom, step, step, dt, nt, d, 1.0, CP, err_level="ignore",
+                                 nthreads=4, alpha=alpha)
+    assert _close(H, ref)
