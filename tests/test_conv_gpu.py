@@ -148,3 +148,33 @@ def test_fftconv_p_long_filters_take_the_fft_path(gpu, oracle, conv_path):
     Y = fftconv_p(H, h)
     ref = oracle.fftconv_p(H, h)
     assert np.max(np.abs(Y - ref)) <= 1e-11 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("dtype,logs,tol", [(torch.float64, (10, 11, 12, 13), 1e-13),
+                                            (torch.float32, (10, 11, 12, 13, 14), 2e-6)])
+@pytest.mark.parametrize("kind", ["vec", "layer", "col"])
+def test_every_transform_length(gpu, conv_path, dtype, logs, tol, kind):
+    """Each built transform length at its largest and just past the one
+    below, one column (no imaginary part) and enough columns for a work-group
+    to serve several pairs; longer ones than a kind takes (they go through
+    the direct sum, another kernel) are left out."""
+    from dream_amd.torch_ops import conv_sum
+    rng = np.random.default_rng(93)
+    conv_path("fft")
+    logs = logs[:{"vec": None, "layer": -1, "col": -2}[kind]]
+    for lg in logs:
+        for MY in ((1 << lg), (1 << (lg - 1)) + 1):
+            MB = MY // 3
+            MA = MY - MB + 1
+            for N in ((1, 3) if kind != "vec" or lg > 11 else (1, 6001)):
+                L = 3 if kind == "layer" else 1
+                A = rng.standard_normal((L, N, MA))
+                B = rng.standard_normal({"vec": (MB,), "layer": (L, MB), "col": (N, MB)}[kind])
+                n = 1 << (MY - 1).bit_length()
+                fB = np.fft.rfft(B, n)
+                fB = {"vec": lambda: fB, "layer": lambda: fB[:, None], "col": lambda: fB}[kind]()
+                ref = np.fft.irfft((np.fft.rfft(A, n) * fB).sum(axis=0), n)[:, :MY]
+                Y = conv_sum(torch.tensor(A if L > 1 else A[0], dtype=dtype, device="cuda"),
+                             torch.tensor(B, dtype=dtype, device="cuda"))
+                err = np.max(np.abs(Y.double().cpu().numpy() - ref)) / np.abs(ref).max()
+                assert err <= tol, (lg, MY, N, kind, err)
