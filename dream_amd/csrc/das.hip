@@ -122,19 +122,11 @@ __device__ __forceinline__ GT delay_ms_of(GT d)
   return (GT) ((double) d / 1000.0);
 }
 
-__device__ __forceinline__ float wave_sum_f(float v)
-{
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
 __device__ __forceinline__ double wave_sum_d(double v)
 {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
 }
-// Wave sum in the data type: FP64 plans reduce in FP64 all the way.
-__device__ __forceinline__ float wave_sum_t(float v) { return wave_sum_f(v); }
-__device__ __forceinline__ double wave_sum_t(double v) { return wave_sum_d(v); }
 
 __device__ __forceinline__ int64_t pixel_of(const int32_t *perm, int64_t idx)
 {
@@ -1145,18 +1137,75 @@ das_adj_region_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int
   }
 }
 
+// Sum over the wave, left in lane 63: adds along DPP rows of 16 lanes, then
+// across the rows.  No LDS traffic and no waits between the steps, unlike
+// shuffles.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_get(float v)
+{
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_get(double v)
+{
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false));
+}
+template <typename T>
+__device__ __forceinline__ T wave_total(T v)
+{
+  v += dpp_get<0x111, 0xf>(v);               // row_shr 1, 2, 4, 8
+  v += dpp_get<0x112, 0xf>(v);
+  v += dpp_get<0x114, 0xf>(v);
+  v += dpp_get<0x118, 0xf>(v);
+  v += dpp_get<0x142, 0xa>(v);               // row_bcast 15, 31
+  v += dpp_get<0x143, 0xc>(v);
+  return v;
+}
+
+__device__ __forceinline__ float fma_d(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_d(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// <g, v> of a lane: one frame's product, or (FR = 4) a record's four.
+__device__ __forceinline__ float weigh(float g, float v) { return g * v; }
+__device__ __forceinline__ double weigh(double g, double v) { return g * v; }
+__device__ __forceinline__ float weigh(frames4 g, frames4 v)
+{
+  return __builtin_fmaf(g[3], v[3], __builtin_fmaf(g[2], v[2], __builtin_fmaf(g[1], v[1], g[0] * v[0])));
+}
+
 // Pixel-major adjoint for two-leg modes without gY: accumulates
 // z_t[i] = sum_p g_p sum_j w_j v(p,i,j), z_r[j] = sum_p g_p sum_i w_i v(p,i,j)
-// and z_cp, in LDS per work-group, flushed once.  Grid-stride over
-// (frame, 256-pixel tile); gathers as in the forward kernel.  FR = 4: over
-// (frame group, tile), each gather bringing four frames' samples, which
-// the lane weights with its four g values (nearest-lower sampling).
+// and z_cp, in LDS per work-group, flushed once.  FR = 4: over frame groups,
+// each gather bringing four frames' samples, which the lane weights with its
+// four g values.
+//
+// A work item is (frame or frame group, 64-pixel tile, part of the tile's
+// jobs), one wave each, strided over a grid that fills the device; a job is a
+// block of `tb` transmits x 16 receivers, so that a small image is split over
+// many waves.  As in the forward a group of kG gathers
+// is issued before any is used, a row out of range for the whole wave is
+// skipped, and the bound is the address path of the gathers (25 L1 lookups
+// per 64-lane gather of a 16-byte record).  A wave that ran all transmits of
+// a chunk and reduced every row by shuffles spent 81 % of its cycles
+// waiting: 64 x 64 elements, 2^19 voxels, 8 frames, nearest-lower took 6.25 ms,
+// now 3.0 (the forward 2.33); one FP32 frame of 48 x 48 over 30720 pixels,
+// linear, 330 us, now 95.
+// Waves per SIMD of the pixel adjoint, near what its registers allow: FP32
+// nearest-lower groups of four frames fit four waves (3.0 ms; three 3.6, five
+// spill and take 7.3), linear sampling is fastest with all it asks for
+// (eight frames of 2^18 voxels 2.9 ms, held to two waves 3.2).
+template <typename DT, int INTERP>
+constexpr int kAdjWaves = INTERP == DREAM_HIP_LINEAR ? 1 : (sizeof(DT) == 4 ? 4 : 3);
+
 template <typename DT, typename GT, int TYPE, int INTERP, bool APOD, int FR = 1>
 __global__ void __launch_bounds__(kThreads)
-das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t n_tiles)
+__attribute__((amdgpu_waves_per_eu(kAdjWaves<DT, INTERP>)))
+das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_end, int split,
+                     int tb)
 {
-  static_assert(FR == 1 || (INTERP == DREAM_HIP_NEAREST && std::is_same<DT, float>::value),
-                "frame groups: FP32, nearest-lower sampling");
+  static_assert(FR == 1 || std::is_same<DT, float>::value, "frame groups: FP32");
+  using VT = lane_t<DT, FR>;
   extern __shared__ __align__(16) unsigned char smem[];
   double *zt = reinterpret_cast<double *>(smem);
   double *zr = zt + A.Lt;
@@ -1168,121 +1217,131 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t n_tile
   const GT *Gt = (const GT *) A.Gt;
   const GT *Gr = (const GT *) A.Gr;
   const GT fs = (GT) A.fs_khz, inv_cp = (GT) A.inv_cp, dl = (GT) A.delay_ms;
-  const double cpd = A.cp;
   const DT *at = (const DT *) A.apod_t;
   const DT *ar = (const DT *) A.apod_r;
   const int K = (int) A.K;
-  const int64_t tiles_per_frame = (A.No + kThreads - 1) / kThreads;
+  const unsigned KB = (unsigned) K * (unsigned) sizeof(VT);      // bytes per A-scan
+  const int64_t tiles_per_row = (A.No + 63) / 64;
   const GT y_lo = Gr[Lt], y_hi = Gr[2 * Lt - 1], x_lo = Gt[0], x_hi = Gt[Lr - 1];
   const GT tmax = (GT) A.leg_max;
+  const int nchunks = (Lr + kRC - 1) / kRC;
+  const int J = nchunks * ((Lt + tb - 1) / tb);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t stride = (int64_t) gridDim.x * (kThreads / 64);
   double zcp = 0.0;
-  const bool lane0 = (threadIdx.x & 63) == 0;
 
-  for (int64_t tile = A.block0 + blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-    const int64_t frame = tile / tiles_per_frame;
-    const int64_t idx = (tile - frame * tiles_per_frame) * kThreads + threadIdx.x;
+  for (int64_t item = A.block0 * split + (int64_t) blockIdx.x * (kThreads / 64) + wave;
+       item < tile_end * split; item += stride) {
+    const int64_t tile = item / split;
+    const int part = (int) (item - tile * split);
+    const int64_t row = tile / tiles_per_row;      // frame or frame group
+    const int64_t idx = (tile - row * tiles_per_row) * 64 + lane;
     const bool valid = idx < A.No;
+    const bool all_valid = __all(valid) != 0;
     const int64_t p = valid ? pixel_of(perm, idx) : 0;
     const GT xo = Ro[p], yo = Ro[p + A.No], zo = Ro[p + 2 * A.No];
-    // `frame` is the frame group when FR = 4: its g values in gp4, and gp
-    // (the weight of the per-row sums) 1.
     const DT *gv = (const DT *) A.g;
-    DT gp = DT(0);
-    frames4 gp4 = frames4{};
+    VT gp;
+    const VT *Yf;
     if constexpr (FR == 4) {
-      gp = DT(1);
 #pragma unroll
       for (int q = 0; q < 4; q++)
-        gp4[q] = valid && 4 * frame + q < A.n_frames ? gv[(4 * frame + q) * A.im_stride + p] : 0.0f;
+        gp[q] = valid && 4 * row + q < A.n_frames ? gv[(4 * row + q) * A.im_stride + p] : 0.0f;
+      Yf = (const VT *) A.Yg + row * A.yg_stride;
     } else {
-      gp = valid ? gv[frame * A.im_stride + p] : DT(0);
+      gp = valid ? gv[row * A.im_stride + p] : DT(0);
+      Yf = (const VT *) A.Y + row * A.y_stride;
     }
-    const DT *Yf = (const DT *) A.Y + (FR == 4 ? 0 : frame * A.y_stride);
-    const __amdgpu_buffer_rsrc_t ry =
-        FR == 4 ? ascan_rsrc((const frames4 *) A.Yg + frame * A.yg_stride, K, 16)
-                : ascan_rsrc(Yf, K, (int) sizeof(DT));
-    const __amdgpu_buffer_rsrc_t rf = frame_rsrc(Yf, A.y_stride * (int64_t) sizeof(DT));
-    const unsigned KB = (unsigned) K * (unsigned) (FR == 4 ? 16 : sizeof(DT));
+    const __amdgpu_buffer_rsrc_t ry = ascan_rsrc(Yf, K, (int) sizeof(VT));
     GT gy_c = GT(0), gx_r = GT(0);
     if (TYPE != DAS_TFM) {
       gy_c = stripe_gap<GT>(yo, y_lo, y_hi);
       gx_r = stripe_gap<GT>(xo, x_lo, x_hi);
     }
-    for (int j0 = 0; j0 < Lr; j0 += kRC) {
+    for (int job = part; job < J; job += split) {
+      const int c = job % nchunks, b = job / nchunks;
+      const int j0 = c * kRC, i0 = b * tb, i1 = min(i0 + tb, Lt);
       GT tr[kRC];
       DT zj[kRC];
+      GT trmin, trmax;
 #pragma unroll
       for (int jj = 0; jj < kRC; jj++) {
         const int j = min(j0 + jj, Lr - 1);
         if (TYPE == DAS_TFM)
-          tr[jj] = leg3<GT>(Gr[j] - xo, Gr[j + Lr] - yo, Gr[j + 2 * Lr] - zo) * inv_cp;
+          tr[jj] = leg3_wave<GT>(Gr[j] - xo, Gr[j + Lr] - yo, Gr[j + 2 * Lr] - zo) * inv_cp;
         else
-          tr[jj] = leg3<GT>(gx_r, Gr[j + Lr] - yo, Gr[j + 2 * Lr] - zo) * inv_cp;
+          tr[jj] = leg3_wave<GT>(gx_r, Gr[j + Lr] - yo, Gr[j + 2 * Lr] - zo) * inv_cp;
         zj[jj] = DT(0);
+        // The linear rule's cp gradient weighs with the unclamped travel time.
+        const GT t = clamp_leg<GT>(tr[jj], tmax);
+        if (INTERP == DREAM_HIP_NEAREST) tr[jj] = t;
+        trmin = jj ? fmin(trmin, t) : t;
+        trmax = jj ? fmax(trmax, t) : t;
       }
-      for (int i = 0; i < Lt; i++) {
-        GT tt;
-        if (TYPE == DAS_TFM)
-          tt = leg3<GT>(Gt[i] - xo, Gt[i + Lt] - yo, Gt[i + 2 * Lt] - zo) * inv_cp;
-        else
-          tt = leg3<GT>(Gt[i] - xo, gy_c, Gt[i + 2 * Lt] - zo) * inv_cp;
-        const GT tt0 = tt;
-        tt += dl;
-        const DT wi = APOD ? at[i] : DT(1);
-        // Nearest-lower taps through the structured view of the frame (0
-        // outside [0, K) and for pairs that are not live); linear ones
-        // through the frame view with their own bounds tests (fewer
-        // registers there).
-        DT y0[kRC], y1[kRC], f[kRC];
+      auto rows = [&](auto all_live) {
+        constexpr bool ALL_LIVE = decltype(all_live)::value;
+        for (int i = i0; i < i1; i++) {
+          GT tt;
+          if (TYPE == DAS_TFM)
+            tt = leg3_wave<GT>(Gt[i] - xo, Gt[i + Lt] - yo, Gt[i + 2 * Lt] - zo) * inv_cp;
+          else
+            tt = leg3_wave<GT>(Gt[i] - xo, gy_c, Gt[i + 2 * Lt] - zo) * inv_cp;
+          const GT tt0 = tt;
+          tt = clamp_leg<GT>(tt + dl, tmax);
+          const GT lo = (tt + trmin) * fs, hi = (tt + trmax) * fs;
+          if (__all(!valid || !(lo < (GT) K) || !(hi > GT(-1)))) continue;
+          const DT wi = APOD ? at[i] : DT(1);
+          constexpr int kG = (INTERP == DREAM_HIP_NEAREST ? kRC : kRC / 2) / (FR == 4 ? 2 : 1);
+          DT zi = DT(0), zc = DT(0);
 #pragma unroll
-        for (int jj = 0; jj < kRC; jj++) {
-          const int j = min(j0 + jj, Lr - 1);
-          const int a = (TYPE == DAS_RCA_ROWTX) ? j * Lt + i : i * Lr + j;
-          const GT u = (clamp_leg<GT>(tt, tmax) + clamp_leg<GT>(tr[jj], tmax)) * fs;
-          const bool live = valid && j0 + jj < Lr;
-          if (INTERP == DREAM_HIP_NEAREST) {
-            unsigned i0, i1;
-            int kk;
-            gather_index<DT, GT, INTERP, false>(u, live, i0, i1, f[jj], kk);
-            if constexpr (FR == 4) {
-              const frames4 v = sload<frames4>(ry, i0, (unsigned) a * KB);
-              y0[jj] = gp4[0] * v[0] + gp4[1] * v[1] + gp4[2] * v[2] + gp4[3] * v[3];
-            } else {
-              y0[jj] = sload<DT>(ry, i0, (unsigned) a * KB);
+          for (int g0 = 0; g0 < kRC; g0 += kG) {
+            unsigned o0[kG], o1[kG];
+            DT f[kG];
+            VT y0[kG], y1[kG];
+#pragma unroll
+            for (int jj = 0; jj < kG; jj++) {
+              const GT t = INTERP == DREAM_HIP_NEAREST ? tr[g0 + jj] : clamp_leg<GT>(tr[g0 + jj], tmax);
+              int k;
+              gather_index<DT, GT, INTERP, ALL_LIVE>((tt + t) * fs, valid && j0 + g0 + jj < Lr,
+                                                     o0[jj], o1[jj], f[jj], k);
             }
-            y1[jj] = y0[jj];
-            f[jj] = DT(0);
-          } else {
-            int kk;
-            fetch_taps<DT, GT, INTERP>(rf, (unsigned) a * (unsigned) K, K, u, live, y0[jj],
-                                       y1[jj], f[jj], kk);
-          }
-        }
-        DT zi = DT(0), zc = DT(0);
 #pragma unroll
-        for (int jj = 0; jj < kRC; jj++) {
-          const DT wj = APOD ? ar[min(j0 + jj, Lr - 1)] : DT(1);
-          const DT slope = INTERP == DREAM_HIP_LINEAR ? y1[jj] - y0[jj] : DT(0);
-          const DT val = y0[jj] + f[jj] * slope;
-          zi += wj * val;
-          zj[jj] += wi * val;
-          if (INTERP == DREAM_HIP_LINEAR) zc += wi * wj * slope * (DT) (tt0 + tr[jj]);
+            for (int jj = 0; jj < kG; jj++) {
+              const int j = min(j0 + g0 + jj, Lr - 1);
+              const unsigned soff = (unsigned) (TYPE == DAS_RCA_ROWTX ? j * Lt + i : i * Lr + j) * KB;
+              y0[jj] = sload<VT>(ry, o0[jj], soff);
+              if (INTERP != DREAM_HIP_NEAREST) y1[jj] = sload<VT>(ry, o1[jj], soff);
+            }
+#pragma unroll
+            for (int jj = 0; jj < kG; jj++) {
+              const DT wj = APOD ? ar[min(j0 + g0 + jj, Lr - 1)] : DT(1);
+              DT val = weigh(gp, y0[jj]);
+              if (INTERP == DREAM_HIP_LINEAR) {
+                const DT slope = weigh(gp, y1[jj] - y0[jj]);
+                val += f[jj] * slope;
+                zc += wj * slope * (DT) (tt0 + tr[g0 + jj]);
+              }
+              zi = fma_d(wj, val, zi);
+              zj[g0 + jj] = fma_d(wi, val, zj[g0 + jj]);
+            }
+          }
+          const DT total = wave_total(zi);
+          if (lane == 63 && total != DT(0)) lds_atomic_add(&zt[i], (double) total);
+          if (INTERP == DREAM_HIP_LINEAR) zcp += (double) (wi * zc);
         }
-        const DT zsum = wave_sum_t(gp * zi);
-        if (lane0 && zsum != DT(0)) atomicAdd(&zt[i], (double) zsum);
-        if (INTERP == DREAM_HIP_LINEAR) zcp += (double) (gp * zc);
-      }
+      };
+      if (all_valid && j0 + kRC <= Lr) rows(std::true_type{});
+      else rows(std::false_type{});
 #pragma unroll
       for (int jj = 0; jj < kRC; jj++) {
-        if (j0 + jj < Lr) {
-          const DT zsum = wave_sum_t(gp * zj[jj]);
-          if (lane0 && zsum != DT(0)) atomicAdd(&zr[j0 + jj], (double) zsum);
-        }
+        const DT total = wave_total(zj[jj]);
+        if (lane == 63 && j0 + jj < Lr && total != DT(0)) lds_atomic_add(&zr[j0 + jj], (double) total);
       }
     }
   }
-  zcp = wave_sum_d(zcp) * (-(double) A.fs_khz / cpd);
-  if (lane0) s_cp[threadIdx.x >> 6] = zcp;
+  zcp = wave_sum_d(zcp) * (-(double) A.fs_khz / A.cp);
+  if (lane == 0) s_cp[wave] = zcp;
   __syncthreads();
   for (int q = threadIdx.x; q < Lt + Lr; q += kThreads) {
     const double v = zt[q];
@@ -1693,26 +1752,37 @@ void adj_launch(const DasArgs &a, const int32_t *perm, bool want_gy, hipStream_t
     }
     run(subs_cand[pick], false, s, gate);
   } else {
-    // Grid-stride over (frame or frame group, 256-pixel tile); a chunk is a
-    // range of tiles.
-    constexpr bool kGroups = std::is_same<DT, float>::value && INTERP == DREAM_HIP_NEAREST;
+    // Wave items over (frame or frame group, 64-pixel tile, part of its
+    // jobs); a chunk is a range of tiles.  Tiles are split into parts until
+    // there are kItems items per wave slot, so the last round is short.
+    constexpr bool kGroups = std::is_same<DT, float>::value;
     const bool groups = kGroups && a.Yg != nullptr;
     const int64_t rows = groups ? (a.n_frames + 3) / 4 : a.n_frames;
-    const int64_t tiles = ((a.No + kThreads - 1) / kThreads) * rows;
+    const int64_t tiles = ((a.No + 63) / 64) * rows;
+    constexpr int64_t kItems = 4;
+    const int64_t slots = (int64_t) cu_count() * 4 * (kThreads / 64);
+    // Blocks of 16 transmits amortise a job's 16 receive legs best; images
+    // that leave the device idle take shorter blocks, down to 4.
+    int tb = kTB;
+    auto jobs_of = [&](int n) { return (int64_t) ((a.Lr + kRC - 1) / kRC) * ((a.Lt + n - 1) / n); };
+    while (tb > 4 && tiles * jobs_of(tb) < slots) tb /= 2;
+    const int64_t jobs = jobs_of(tb);
+    const int split = (int) std::max<int64_t>(1, std::min(jobs, (kItems * slots + tiles - 1) / std::max<int64_t>(tiles, 1)));
     const size_t lds = (size_t) (a.Lt + a.Lr) * sizeof(double);
-    run_chunked(tiles, 1,
-                (int64_t) kThreads * pairs_per_pixel(TYPE, a.Lt, a.Lr) * (groups ? 4 : 1), gate,
+    run_chunked(tiles, 1, (int64_t) 64 * pairs_per_pixel(TYPE, a.Lt, a.Lr) * (groups ? 4 : 1), gate,
                 [&](int64_t b0, int64_t nb, int64_t, int64_t) {
                   DasArgs c = a;
                   c.block0 = b0;
-                  const int grid = (int) std::min<int64_t>(nb, (int64_t) cu_count() * 4);
+                  const int64_t items = nb * split;
+                  const int grid = (int) std::min<int64_t>((items + kThreads / 64 - 1) / (kThreads / 64),
+                                                           (int64_t) cu_count() * 4);
                   if (groups) {
                     if constexpr (kGroups)
                       hipLaunchKernelGGL((das_adj_pixel_kernel<DT, GT, TYPE, INTERP, APOD, 4>),
-                                         dim3(grid), dim3(kThreads), lds, s, c, perm, b0 + nb);
+                                         dim3(grid), dim3(kThreads), lds, s, c, perm, b0 + nb, split, tb);
                   } else {
                     hipLaunchKernelGGL((das_adj_pixel_kernel<DT, GT, TYPE, INTERP, APOD>),
-                                       dim3(grid), dim3(kThreads), lds, s, c, perm, b0 + nb);
+                                       dim3(grid), dim3(kThreads), lds, s, c, perm, b0 + nb, split, tb);
                   }
                   DREAM_HIP_CHECK(hipGetLastError());
                 });
@@ -2291,9 +2361,9 @@ void DasHandle::adjoint_dev(const void *Y, const void *Ro, const void *Gt, const
   const bool channel = type_ == DAS_SAFT || gY != nullptr;
   a.z_t = channel ? (void *) Z : (void *) zt;
   a.z_r = zr;
-  // The pixel kernel's nearest-lower taps read frames in groups of four
-  // (not in the allocation-free call).
-  if (No_ > 0 && !channel && !fixed_z && interp == DREAM_HIP_NEAREST)
+  // The pixel kernel reads frames in groups of four (not in the
+  // allocation-free call).
+  if (No_ > 0 && !channel && !fixed_z)
     group_frames(a, Y, y_stride, n_frames, s);
   ChunkGate gate(s);
   if (No_ > 0) {

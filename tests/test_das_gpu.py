@@ -324,6 +324,36 @@ def test_frame_groups_match_single_frames(gpu, method):
     assert rel_l2(gar.double().cpu().numpy(), sar) <= 1e-5
 
 
+@pytest.mark.parametrize("method", ["tfm", "rca_coltx", "rca_rowtx"])
+@pytest.mark.parametrize("No,L", [(1, 5), (63, 16), (65, 17), (700, 33)])
+def test_pixel_adjoint_edges(gpu, oracle, method, No, L):
+    """The pixel-major adjoint (no Y gradient) at partial tiles, receive
+    chunks and transmit blocks, one frame and frame groups with padding
+    frames, both sampling rules, against the FP64 oracle summed over the
+    frames."""
+    from dream_amd.torch_ops import DasPlan
+    Y, Gt, Gr, Ro, rng = _setup(method, L=L, seed=14, No=No)
+    F = 5
+    Yf = np.stack([Y.T * (1 + f) for f in range(F)])
+    g = rng.standard_normal((F, No))
+    at, ar = rng.uniform(0.5, 1.5, L), rng.uniform(0.5, 1.5, L)
+    for interp in ("nearest", "linear"):
+        ref = [oracle.das_ext_adjoint(Yf[f].T, Gt, Gr, Ro, 0.02, 0.1, 1500.0, g[f], method,
+                                      interp, at, ar) for f in range(F)]
+        for prec, dt_, tol in (("f64", torch.float64, 1e-10), ("f32", torch.float32, 5e-5)):
+            plan = DasPlan(method, Y.shape[0], Ro, Gt, Gr, precision=prec)
+            for n in (1, F):
+                t = [torch.tensor(v, dtype=dt_, device="cuda").contiguous()
+                     for v in (Yf[:n], g[:n], at, ar)]
+                _, gat, gar, gcp = plan.adjoint(t[0], t[1], 0.02, 0.1, 1500.0, t[2], t[3], interp,
+                                                want_gy=False)
+                assert rel_l2(gat.double().cpu().numpy(), sum(r[1] for r in ref[:n])) <= tol
+                assert rel_l2(gar.double().cpu().numpy(), sum(r[2] for r in ref[:n])) <= tol
+                if interp == "linear":
+                    rcp = sum(r[3] for r in ref[:n])
+                    assert abs(float(gcp) - rcp) <= (1e-9 if prec == "f64" else 1e-3) * abs(rcp)
+
+
 def test_autograd_function(gpu, oracle):
     from dream_amd.torch_ops import DasPlan, das_diff
     method = "saft"
