@@ -22,8 +22,16 @@
 // The LDS atomics of those flushes bound the kernel, and along x the bin
 // changes about every other step when the element lies to the side of the
 // point; for flat rectangles a point may instead walk columns (y inner, in
-// row segments), where |ry| <= b/2 keeps the bin for several steps.  Each
-// point takes the walk its run-length model prices lower.
+// row segments), where |ry| <= b/2 keeps the bin for several steps.  Where
+// the bin lasts, a rectangle's columns and a disc's rows are walked run by
+// run (sir_runs.hpp): a bin's edge and a closed-form sum of 1/r per run, about
+// 75 FP64-rate instructions whatever its length, against 19.5 for each
+// sub-element.  Each point takes the walk its run-length model prices lowest.
+// FP64 instruction issue bounds all three.  Measured, steps -> runs: 16384
+// points x 32 elements of 0.4 x 10 mm (7 sub-elements a run, 80 % of issue
+// slots) 630 -> 410 us; 24 uneven problems of 5 .. 15 mm elements, FP32 out,
+// 3.70 -> 2.45 ms; 9 discs of 3.5 .. 7.5 mm over 4096 points (18 a run) 1.20 ->
+// 0.83 ms.
 //
 // Sample index.  The index must equal the reference's FP64 sequence bit for
 // bit.  A fast estimate u = r*c1 - d/dt (r from the hardware rsqrt, about
@@ -46,6 +54,7 @@
 #include <type_traits>
 
 #include "sir.hpp"
+#include "sir_runs.hpp"
 #include "tune.hpp"
 
 namespace dream {
@@ -53,7 +62,6 @@ namespace dream {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
 // Sub-elements per block of independent index computations.
 constexpr int kBlock = 4;
 constexpr double kBoundScale = 0x1p-36;
@@ -156,55 +164,52 @@ __device__ __forceinline__ int find_problem(const SirDev *P, int n, int64_t item
   return lo;
 }
 
-// Double sum over the wave, in a fixed order (the same on every work-group).
-__device__ __forceinline__ double wave_sum_d(double v)
-{
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
+// How point (xo, yo, zo) walks its sub-elements: WALK_ROWS (x inner, index by
+// index), WALK_COLUMNS (y inner; rectangles) or WALK_RUNS (run by run, see
+// sir_runs.hpp: a rectangle's columns, a disc's rows).  A lane flushes its
+// run into the histogram when the bin changes, which along x happens at a
+// rate of about min(1, |rx|/r dx/l) per step (l = cp dt/1000, one sample of
+// path) and along y at min(1, |ry|/r dy/l); with up to 256 elements' mean
+// offsets for rx and ry, the cheapest walk is taken: a stepped flush counts
+// as 4 contributions, a run as 6 (75 instructions against 19.5 for a
+// contribution, and its flush), a line's set-up for runs as 8, and each walk
+// pays for its partly filled lane rounds.  Every wave of the point computes
+// the same sums in the same order, so all its items agree.
+enum { WALK_ROWS = 0, WALK_COLUMNS = 1, WALK_RUNS = 2 };
 
-// Whether point (xo, yo, zo) of a rectangle problem walks columns (y inner)
-// rather than rows (x inner).  A lane flushes its run into the histogram
-// when the bin changes, which along x happens at a rate of about
-// min(1, |rx|/r dx/l) per step (l = cp dt/1000, one sample of path) and
-// along y at min(1, |ry|/r dy/l); with each element's mean offsets for rx
-// and ry, the cheaper walk counts a flush as 4 contributions and charges
-// each walk its partly filled lane rounds.  Every work-group of the point
-// computes the same sums in the same order, so all its items agree.
-__device__ __forceinline__ bool walk_columns(const SirDev &P, double xo, double yo, double zo, double *red)
+__device__ __forceinline__ int pick_walk(const SirDev &P, double xo, double yo, double zo)
 {
   gdouble *el = (gdouble *) P.el;
-  const int L = P.L;
-  double fx = 0.0, fy = 0.0;
-  for (int e = threadIdx.x; e < L; e += kThreads) {
-    const double mx = __builtin_fmax(__builtin_fabs(xo - el[e]), P.wx);
-    const double my = __builtin_fmax(__builtin_fabs(yo - el[L + e]), P.wy);
-    const double mz = zo - el[2 * L + e];
-    const double r = __builtin_sqrt(mx * mx + my * my + mz * mz);
-    if (r > 0.0) {
-      fx += __builtin_fmin(1.0, mx / r * P.sx);
-      fy += __builtin_fmin(1.0, my / r * P.sy);
-    }
+  const int L = P.L, every = (L + 255) / 256;
+  float fx = 0.0f, fy = 0.0f, n = 0.0f;
+  for (int e = (int) (threadIdx.x & 63) * every; e < L; e += 64 * every) {
+    const float mx = __builtin_fmaxf(__builtin_fabsf((float) (xo - el[e])), P.wx);
+    const float my = __builtin_fmaxf(__builtin_fabsf((float) (yo - el[L + e])), P.wy);
+    const float mz = (float) (zo - el[2 * L + e]);
+    const float q = __builtin_amdgcn_rsqf(mx * mx + my * my + mz * mz);
+    fx += __builtin_fminf(1.0f, mx * q * P.sx);       // NaN (all zero) counts as 1
+    fy += __builtin_fminf(1.0f, my * q * P.sy);
+    n += 1.0f;
   }
-  fx = wave_sum_d(fx);
-  fy = wave_sum_d(fy);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) { red[w] = fx; red[kWaves + w] = fy; }
-  __syncthreads();
-  fx = red[0];
-  fy = red[kWaves];
-  for (int k = 1; k < kWaves; k++) {
-    fx += red[k];
-    fy += red[kWaves + k];
+  for (int off = 32; off > 0; off >>= 1) {
+    fx += __shfl_xor(fx, off, 64);
+    fy += __shfl_xor(fy, off, 64);
+    n += __shfl_xor(n, off, 64);
   }
-  fx /= L;
-  fy /= L;
-  const double nx = P.nx, S = P.seg_len;
-  const double rounds_r = __builtin_ceil((double) L * P.ny / P.chunks / kThreads);
-  const double rounds_c = __builtin_ceil((double) L * P.nx * P.nseg / P.chunks / kThreads);
-  const double cost_r = rounds_r * nx * (1.0 + 4.0 * (1.0 + (nx - 1.0) * fx) / nx);
-  const double cost_c = rounds_c * S * (1.0 + 4.0 * (1.0 + (S - 1.0) * fy) / S);
-  return __builtin_amdgcn_readfirstlane((int) (cost_c < cost_r)) != 0;
+  fx /= n;
+  fy /= n;
+  const float nx = (float) P.nx, S = (float) P.seg_len;
+  int walk;
+  if (P.shape == SIR_CIRC) {
+    walk = 8.0f + 6.0f * (1.0f + nx * fx) < nx * (1.0f + 4.0f * fx) ? WALK_RUNS : WALK_ROWS;
+  } else {
+    const float cost_r = P.rounds_r * (nx + 4.0f + 4.0f * (nx - 1.0f) * fx);
+    const float cost_c = P.rounds_c * (S + 4.0f + 4.0f * (S - 1.0f) * fy);
+    const float cost_u = P.rounds_c * (8.0f + 6.0f * (1.0f + (S - 1.0f) * fy));
+    walk = cost_c < cost_r ? WALK_COLUMNS : WALK_ROWS;
+    if (P.runs && cost_u < __builtin_fminf(cost_c, cost_r)) walk = WALK_RUNS;
+  }
+  return __builtin_amdgcn_readfirstlane(walk);
 }
 
 // One work item: observation point n of problem P, chunk c of its rows (or
@@ -213,7 +218,7 @@ __device__ __forceinline__ bool walk_columns(const SirDev &P, double xo, double 
 // times faster than its FP32 one, and the column is rounded to T once, when
 // it is written.
 template <typename T, bool ANY_GLOBAL>
-__device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double *hist, double *red)
+__device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double *hist)
 {
   const int64_t n = local / P.chunks;
   const int c = (int) (local - n * P.chunks);
@@ -227,10 +232,18 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
   // Plans without a global-mode problem compile the LDS path only.
   const bool use_lds = !ANY_GLOBAL || P.mode != SIR_GLOBAL;
   constexpr bool REFINE_H = !std::is_same<T, float>::value;
-  const bool columns = P.nseg > 0 && (P.walk == 1 || walk_columns(P, xo, yo, zo, red));
+  // A choice of walks only where the plan offers one.
+  int walk = WALK_ROWS;
+  if (P.walk >= 0) walk = P.walk;
+  else if (P.shape == SIR_CIRC ? P.runs != 0 : P.nseg > 0) walk = pick_walk(P, xo, yo, zo);
+  const bool columns = P.shape == SIR_RECT && walk != WALK_ROWS;
 
+  // Copies of the histogram, one per group of lanes.
+  const int pitch = (int) nt + 1;
+  double *const copy0 = hist;
   if (use_lds) {
-    for (int i = threadIdx.x; i < nt; i += kThreads) hist[i] = 0.0;
+    for (int i = threadIdx.x; i < P.copies * pitch; i += kThreads) hist[i] = 0.0;
+    hist += (threadIdx.x & (P.copies - 1)) * pitch;
     __syncthreads();
   }
 
@@ -297,6 +310,22 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
     if (lane == __ffsll((long long) act) - 1) oob_s += cnt_w;
     return ((out_mask >> lane) & 1ull) != 0;
   };
+  // Sub-elements [k0, k1) of a usable line, run by run; step(k) adds one
+  // that no run certifies.  Runs outside [0, nt) add to the spare bin.
+  auto walk_line = [&](const RunLine &line, int k0, int k1, double amp, auto step) {
+#pragma clang loop unroll(disable)
+    for (int half = 0; half < 2; half++) {
+      int len;
+      const int first = half_of(line, half, k0, k1, len);
+      int m = walk_half<REFINE_H>(line, half, first, len, [&](int b, int n, double v) {
+        const bool in = (unsigned) b < (unsigned) nt;
+        if (use_lds) lds_add(hist + min((unsigned) b, (unsigned) nt), amp * v);
+        else if (in) global_add(out + b, (T) (amp * v));
+        oob += in ? 0 : n;
+      });
+      for (; m < len; m++) step(half ? first - m : first + m);
+    }
+  };
   if (!columns) {
     const int Q = L * ny;
     const int q0 = (int) ((int64_t) c * Q / P.chunks);
@@ -313,7 +342,10 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
       const double ye = yo - el[L + e];
       const double ze = zo - el[2 * L + e];
       const double d = (dlay - el[3 * L + e]) - el[4 * L + e];
-      const double ry = ye - ys[row];
+      // Discs: part j / rows of a row, a wave's lanes mostly of one part.
+      const int part = P.shape == SIR_CIRC ? j / P.rows : 0;
+      const int line_row = P.shape == SIR_CIRC ? j - part * P.rows : row;
+      const double ry = ye - ys[line_row];
       const double ryy = ry * ry;
       // Cylinders: the row's depth on the curved surface (ze - 0.0 == ze
       // for flat elements).
@@ -328,10 +360,31 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
       unsigned cnt_w = 0;
       unsigned long long out_mask = 0;
       if (P.shape == SIR_CIRC) {
-        // A disc row: the reference's accumulated walk from this row's start.
-        double x = ((gdouble *) P.row_x0)[row];
-        const int cnt = (int) ((gdouble *) P.row_n)[row];
-        for (int i = 0; i < cnt; i++) {
+        // One part of a disc row: run by run, or the reference's
+        // accumulated walk from the row's start.
+        const int cnt = (int) ((gdouble *) P.row_n)[line_row];
+        const double x0 = ((gdouble *) P.row_x0)[line_row];
+        const double len = (double) cnt * P.part_len;
+        int k = (int) (len * (double) part);
+        const int k1 = part + 1 == P.nseg ? cnt : (int) (len * (double) (part + 1));
+        if (walk == WALK_RUNS && k < k1) {
+          RunLine line{xe - x0, ((gdouble *) P.row_dx)[line_row], ((gdouble *) P.row_idx)[line_row],
+                       ryz, P.c1, P.ic1, c2, 0.5 - lim};
+          if (runs_ready<REFINE_H>(line, cnt)) {
+            walk_line(line, k, k1, el[5 * L + e] * P.amp, [&](int i) {
+              double x = x0, h;
+              for (int m = 0; m < i; m++) x += P.dx;
+              const double ru = sir_index<REFINE_H>(xe - x, ryy, rzz, ryz, c1h, c2, lim, P.cp, d,
+                                                    P.dt, h);
+              accumulate(sat_i32(ru), h);
+            });
+            k = k1;
+          }
+        }
+        double x = x0;
+        if (k < k1)
+          for (int m = 0; m < k; m++) x += P.dx;
+        for (; k < k1; k++) {
           double h;
           const double ru = sir_index<REFINE_H>(xe - x, ryy, rzz, ryz, c1h, c2, lim, P.cp, d,
                                                 P.dt, h);
@@ -400,13 +453,27 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
       const unsigned oob_unit = oob;
       unsigned cnt_w = 0;
       unsigned long long out_mask = 0;
-      const int j0 = sg * P.seg_len;
+      int j0 = sg * P.seg_len;
       const int j1 = min(j0 + P.seg_len, ny);
+      if (walk == WALK_RUNS) {
+        RunLine line{ye - P.line_p0, P.line_dv, P.line_inv_dv, rxz, P.c1, P.ic1, c2, 0.5 - lim};
+        if (runs_ready<REFINE_H>(line, ny)) {
+          walk_line(line, j0, j1, el[5 * L + e] * P.amp, [&](int k) {
+            const double ry = ye - ys[k];
+            double r, h;
+            if (!sir_fast<REFINE_H>(ry, rxz, c1h, c2, lim, r, h))
+              sir_exact<REFINE_H>(rx, ry * ry, rzz, P.cp, d, P.dt, r, h);
+            accumulate(sat_i32(r), h);
+          });
+          j0 = j1;
+        }
+      }
       // Every segment has seg_len rows but the last, so the wave's whole
       // blocks of kBlock rows are a uniform count: the shorter length's when
       // any of its lanes holds a last segment.
       const int last_len = ny - (P.nseg - 1) * P.seg_len;
-      const int nb = (__ballot(j1 - j0 < P.seg_len) ? last_len : P.seg_len) / kBlock;
+      const int nb = walk == WALK_RUNS ? 0
+                   : (__ballot(j1 - j0 < P.seg_len) ? last_len : P.seg_len) / kBlock;
       int j = j0;
       for (int blk = 0; blk < nb; blk++, j += kBlock) {
         double yv[kBlock], r[kBlock], w[kBlock];
@@ -455,13 +522,11 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
 
   if (use_lds) {
     __syncthreads();
-    if (P.mode == SIR_LDS_STORE) {
-      for (int i = threadIdx.x; i < nt; i += kThreads) out[i] = (T) hist[i];
-    } else {
-      for (int i = threadIdx.x; i < nt; i += kThreads) {
-        const double v = hist[i];
-        if (v != 0.0) global_add(out + i, (T) v);
-      }
+    for (int i = threadIdx.x; i < nt; i += kThreads) {
+      double v = copy0[i];
+      for (int c = 1; c < P.copies; c++) v += copy0[c * pitch + i];
+      if (P.mode == SIR_LDS_STORE) out[i] = (T) v;
+      else if (v != 0.0) global_add(out + i, (T) v);
     }
     __syncthreads();
   }
@@ -478,13 +543,12 @@ sir_kernel(const SirDev *__restrict__ probs, int n_probs, int64_t item_lo, int64
 {
   extern __shared__ __align__(16) unsigned char smem[];
   double *hist = reinterpret_cast<double *>(smem);
-  __shared__ double red[2 * kWaves];
   // This launch serves items [item_lo, item_hi) (a chunk of a long plan).
   if (counter == nullptr) {
     const int64_t item = item_lo + blockIdx.x;
     if (item >= item_hi) return;
     const int p = find_problem(probs, n_probs, item);
-    sir_item<T, ANY_GLOBAL>(probs[p], item - probs[p].item_begin, hist, red);
+    sir_item<T, ANY_GLOBAL>(probs[p], item - probs[p].item_begin, hist);
     return;
   }
   // Persistent: pull items from counter[0]; the last work-group to leave
@@ -497,7 +561,7 @@ sir_kernel(const SirDev *__restrict__ probs, int n_probs, int64_t item_lo, int64
     __syncthreads();
     if (item >= item_hi) break;
     const int p = find_problem(probs, n_probs, item);
-    sir_item<T, ANY_GLOBAL>(probs[p], item - probs[p].item_begin, hist, red);
+    sir_item<T, ANY_GLOBAL>(probs[p], item - probs[p].item_begin, hist);
   }
   if (threadIdx.x == 0) {
     __threadfence();
@@ -647,53 +711,19 @@ double cylinder_rows(double b, double Rc, double dy, std::vector<double> &ys,
   return dphi;
 }
 
-void split_disc_rows(int64_t L, double dx, std::vector<double> &ys, std::vector<double> &x0,
-                     std::vector<double> &count)
+double disc_row_step(double x0, double count, double dx)
 {
-  // Rows are dealt one per lane, so a disc whose rows number fewer than the
-  // lanes, or whose rows differ in length, leaves lanes idle.  Cut the rows
-  // into segments of at most S sub-elements, S chosen to minimise (passes of
-  // 256 lanes) x S over the point's L x segments; each segment starts at the
-  // x the row's accumulated walk reaches there, so every position is the
-  // reference's bit for bit.
-  double mx = 0.0;
-  for (double c : count) mx = std::max(mx, c);
-  const int64_t maxc = (int64_t) mx;
-  if (maxc <= 1 || L < 1) return;
-  int64_t best_s = maxc;
-  double best_t = 0.0;
-  // Segments shorter than 48 cost more in per-row set-up than they gain in
-  // balance (measured on MI355X: the annular benchmark's disc launch took
-  // 2.15 ms unsplit, 1.83 ms with segments down to 9 sub-elements, and the
-  // whole call was fastest with a floor of 48).
-  const int64_t smin = std::max<int64_t>({(int64_t) 48, maxc / 16});
-  for (int64_t S = maxc; S >= smin; S = std::min(S - 1, S * 31 / 32)) {
-    int64_t q = 0;
-    for (double c : count) q += ((int64_t) c + S - 1) / S;
-    const double t = std::ceil((double) (q * L) / (double) kThreads) * (double) S;
-    if (S == maxc || t < best_t) { best_t = t; best_s = S; }
+  // Within one binade of |x| the accumulated walk advances by a constant
+  // step, dx rounded to the binade's spacing: the row's mean step is dx plus
+  // those deviations over the lengths the row spends in each binade.
+  if (count < 2.0) return dx;
+  const double half = std::fabs(x0);
+  double drift = 0.0;
+  for (double lo = std::ldexp(1.0, std::ilogb(half)); lo > 4.0 * dx; lo *= 0.5) {
+    const double x = 1.5 * lo;
+    drift += 2.0 * (std::min(half, 2.0 * lo) - lo) / dx * ((x + dx) - x - dx);
   }
-  if (best_s == maxc) return;
-  std::vector<double> vy, vx, vn;
-  for (size_t r = 0; r < ys.size(); r++) {
-    double x = x0[r];
-    int64_t left = (int64_t) count[r];
-    if (left == 0) {
-      vy.push_back(ys[r]); vx.push_back(x); vn.push_back(0.0);
-      continue;
-    }
-    while (left > 0) {
-      const int64_t c = std::min(best_s, left);
-      vy.push_back(ys[r]);
-      vx.push_back(x);
-      vn.push_back((double) c);
-      for (int64_t k = 0; k < c; k++) x += dx;
-      left -= c;
-    }
-  }
-  ys.swap(vy);
-  x0.swap(vx);
-  count.swap(vn);
+  return dx + drift / (count - 1.0);
 }
 
 std::vector<double> subgrid(double w, double d)
@@ -827,16 +857,64 @@ std::vector<double> element_table(const SirProblem &p)
 
 // ------------------------------------------------------------------ plan
 
-// DREAM_HIP_SIR_WALK = rows | columns forces the sub-element walk of
-// rectangle problems (for comparisons and tests): 1 rows, 2 columns, 0 the
-// per-point choice.
+// DREAM_HIP_SIR_WALK = rows | columns | runs forces the sub-element walk
+// where the problem has it (for comparisons and tests); -1 is the per-point
+// choice.
 int walk_override()
 {
   const char *e = std::getenv("DREAM_HIP_SIR_WALK");
-  if (!e) return 0;
-  if (std::strcmp(e, "rows") == 0) return 1;
-  if (std::strcmp(e, "columns") == 0) return 2;
-  return 0;
+  if (!e) return -1;
+  if (std::strcmp(e, "rows") == 0) return WALK_ROWS;
+  if (std::strcmp(e, "columns") == 0) return WALK_COLUMNS;
+  if (std::strcmp(e, "runs") == 0) return WALK_RUNS;
+  return -1;
+}
+
+// The order in which a disc's rows are dealt to lanes: by length, so that
+// the lanes of a wave end together.
+void order_disc_rows(std::vector<double> &ys, std::vector<double> &x0, std::vector<double> &count)
+{
+  std::vector<int> order(ys.size());
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return count[(size_t) a] > count[(size_t) b];
+  });
+  auto deal = [&](std::vector<double> &v) {
+    std::vector<double> w(v.size());
+    for (size_t k = 0; k < v.size(); k++) w[k] = v[(size_t) order[k]];
+    v.swap(w);
+  };
+  deal(ys);
+  deal(x0);
+  deal(count);
+}
+
+// Whether positions that stray by `dev` mm from equal spacing `step` may be
+// walked run by run: a few bins per step at most (each point then weighs its run
+// length), and a deviation below an eighth of the certification margin.
+bool runs_hold(double dev, double step, double c1, int64_t nt)
+{
+  return c1 > 0.0 && step > 0.0 && c1 * step <= 4.0 && 8.0 * c1 * dev <= kBoundScale * ((double) nt + 2.0);
+}
+
+// Parts to cut the lines of a point into: the count (up to `most`) that
+// minimises the mean of lane rounds per item and full lane rounds x cost of
+// a part of `len` sub-elements, stepped or in runs (a bin each 0.2 dx / (cp
+// dt/1000) steps, but at most about 20 steps).
+int64_t line_parts(int64_t lines, int64_t chunks, int64_t len, int64_t most, bool runs, double sx)
+{
+  if (len < 1) return 1;
+  double best = 0.0;
+  int64_t best_n = 1;
+  for (int64_t ns = 1; ns <= std::max<int64_t>(most, 1); ns++) {
+    const int64_t S = (len + ns - 1) / ns, n = (len + S - 1) / S;
+    const double full = (double) (lines * n) / (double) chunks / kThreads;
+    const double c = (std::ceil(full) + (runs ? full : std::ceil(full))) *
+                     (runs ? 8.0 + 6.0 * (1.0 + (double) S * std::max(0.2 * sx, 0.05))
+                           : (double) S + 4.0 + 4.0 * (double) (S - 1) * 0.15);
+    if (ns == 1 || c < best) { best = c; best_n = n; }
+  }
+  return best_n;
 }
 
 SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int target_items)
@@ -854,7 +932,7 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
   for (auto &p : problems) total_no += p.No;
 
   // Host tables and per-problem shape.
-  std::vector<std::vector<double>> xs(P), ys(P), el(P), rx0(P), rn(P), zr(P);
+  std::vector<std::vector<double>> xs(P), ys(P), el(P), rx0(P), rn(P), rdx(P), zr(P);
   std::vector<SirDev> dev(P);
   std::vector<double> cost(P, 0.0);
   size_t table_doubles = 0;
@@ -868,14 +946,30 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
     require(p.No == 0 || (p.Ro && p.delay && p.h), "SIR: null Ro, delay or h");
     require(p.shape == SIR_RECT || p.shape == SIR_CIRC || p.shape == SIR_CYLIND,
             "SIR: unknown element shape");
-    int64_t nx_cost;
+    const double c1 = 1000.0 / (p.cp * p.dt), lam = p.cp * p.dt / 1000.0;
+    const int force = walk_override();
+    int64_t nx_cost, disc_parts = 1;
+    bool runs = false;
     if (p.shape == SIR_CIRC) {
       disc_rows(p.R, p.dx, p.dy, ys[i], rx0[i], rn[i]);
-      split_disc_rows((int64_t) (p.G.size() / 3), p.dx, ys[i], rx0[i], rn[i]);
+      order_disc_rows(ys[i], rx0[i], rn[i]);
       double sum = 0.0, mx = 0.0;
-      for (double c : rn[i]) { sum += c; mx = std::max(mx, c); }
+      for (size_t r = 0; r < rn[i].size(); r++) {
+        sum += rn[i][r];
+        mx = std::max(mx, rn[i][r]);
+        rdx[i].push_back(disc_row_step(rx0[i][r], rn[i][r], p.dx));
+      }
+      for (size_t r = 0; r < rn[i].size(); r++) rdx[i].push_back(1.0 / rdx[i][r]);
+      // An accumulated position is within half an ulp of R per step.
+      runs = force != WALK_ROWS && force != WALK_COLUMNS && p.R > 0.0 &&
+             runs_hold(mx * std::ldexp(1.0, std::ilogb(p.R) - 52), p.dx, c1, p.nt);
+      // Rows are dealt one part per lane; stepped parts below 48
+      // sub-elements cost more set-up than the balance gains.
+      disc_parts = line_parts(L * (int64_t) ys[i].size(), 1, (int64_t) mx,
+                              std::min<int64_t>((int64_t) mx / (runs ? 16 : 48), 16), runs,
+                              p.dx / lam);
       xs[i].assign(1, 0.0);                     // unused by the disc walk
-      nx_cost = ys[i].empty() ? 0 : (int64_t) (sum / (double) ys[i].size() + 1.0);
+      nx_cost = ys[i].empty() ? 0 : (int64_t) (sum / (double) ((int64_t) ys[i].size() * disc_parts) + 1.0);
       if (mx == 0.0) nx_cost = 0;
     } else if (p.shape == SIR_CYLIND) {
       xs[i] = subgrid(p.a, p.dx);
@@ -887,7 +981,7 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
       nx_cost = (int64_t) xs[i].size();
     }
     el[i] = element_table(p);
-    const int64_t nx = nx_cost, ny = (int64_t) ys[i].size();
+    const int64_t nx = nx_cost, ny = (int64_t) ys[i].size() * disc_parts;
     require(L * ny < (1ll << 31) && nx < (1ll << 31), "SIR: element x row count too large");
     SirDev &d = dev[i];
     std::memset(&d, 0, sizeof d);
@@ -900,8 +994,9 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
     d.ny = (int32_t) ny;
     d.shape = p.shape;
     d.dx = p.dx;
+    d.rows = (int32_t) ys[i].size();
     int stride = 1;
-    if (ny > 64) {
+    if (ny > 64 && p.shape != SIR_CIRC) {
       stride = (int) (ny / 64);
       while (gcd_int(stride, (int) ny) != 1) stride++;
     }
@@ -916,7 +1011,8 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
     d.cp = p.cp;
     d.dt = p.dt;
     d.inv_dt = 1.0 / p.dt;
-    d.c1 = 1000.0 / (p.cp * p.dt);
+    d.c1 = c1;
+    d.ic1 = lam;
     d.amp = 1000.0 / (2.0 * M_PI * p.dt);
     d.h = p.h;
     const int64_t Q = L * ny;
@@ -926,24 +1022,29 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
       chunks = std::min<int64_t>(chunks, std::max<int64_t>(Q / kThreads, 1));
     }
     d.chunks = (int32_t) std::max<int64_t>(chunks, 1);
-    if (p.shape == SIR_RECT && nx > 0 && ny > 0 && walk_override() != 1) {
-      d.walk = walk_override() == 2 ? 1 : 0;
-      // Column segments: the count that minimises lane rounds per item x
-      // rows per segment x the run-length cost of a segment (a flush per
-      // segment plus one per eighth step or so), over at most ny/8
-      // segments.
+    if (p.shape == SIR_CIRC && nx > 0 && ny > 0) {
+      d.nseg = (int32_t) disc_parts;
+      d.part_len = 1.0 / (double) disc_parts;
+      d.runs = runs;
+      d.walk = !runs ? WALK_ROWS : force;
+      d.wx = d.wy = (float) (4.0 / (3.0 * M_PI) * p.R);   // mean |x| over the disc
+      d.sx = (float) (p.dx / lam);
+      d.sy = (float) (p.dy / lam);
+    }
+    if (p.shape == SIR_RECT && nx > 0 && ny > 0 && force != WALK_ROWS) {
+      const std::vector<double> &y = ys[i];
+      d.line_p0 = y[0];
+      d.line_dv = ny > 1 ? (y[(size_t) ny - 1] - y[0]) / (double) (ny - 1) : p.dy;
+      d.line_inv_dv = 1.0 / d.line_dv;
+      double dev = 0.0;
+      for (int64_t k = 0; k < ny; k++)
+        dev = std::max(dev, std::fabs(y[(size_t) k] - (y[0] + (double) k * d.line_dv)));
+      d.runs = force != WALK_COLUMNS && runs_hold(dev, d.line_dv, c1, p.nt);
+      d.walk = force == WALK_RUNS && !d.runs ? WALK_COLUMNS : force;
       const int64_t QC = L * nx;
-      double best = 0.0;
-      int64_t best_n = 1;
-      for (int64_t ns = 1; ns <= std::max<int64_t>(ny / 8, 1); ns++) {
-        const int64_t S = (ny + ns - 1) / ns;
-        const int64_t nseg = (ny + S - 1) / S;
-        const double rounds = std::ceil((double) (QC * nseg) / (double) d.chunks / kThreads);
-        const double c = rounds * (double) S * (1.0 + 4.0 * (1.0 + (double) (S - 1) * 0.15) / (double) S);
-        if (ns == 1 || c < best) { best = c; best_n = nseg; }
-      }
-      const int64_t S = (ny + best_n - 1) / best_n;
-      require(QC * best_n < (1ll << 31) - kThreads, "SIR: element x column count too large");
+      const int64_t n = line_parts(QC, d.chunks, ny, ny / 8, d.runs, p.dy / lam);
+      const int64_t S = (ny + n - 1) / n;
+      require(QC * n < (1ll << 31) - kThreads, "SIR: element x column count too large");
       d.nseg = (int32_t) ((ny + S - 1) / S);
       d.seg_len = (int32_t) S;
       d.cstep_sg = (int32_t) (kThreads / QC);
@@ -952,18 +1053,22 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
       double sxm = 0.0, sym = 0.0;
       for (double v : xs[i]) sxm += std::fabs(v);
       for (double v : ys[i]) sym += std::fabs(v);
-      const double lam = p.cp * p.dt / 1000.0;
-      d.wx = sxm / (double) nx;
-      d.wy = sym / (double) ny;
-      d.sx = p.dx / lam;
-      d.sy = p.dy / lam;
+      d.wx = (float) (sxm / (double) nx);
+      d.wy = (float) (sym / (double) ny);
+      d.sx = (float) (p.dx / lam);
+      d.sy = (float) (p.dy / lam);
+      d.rounds_r = (float) std::ceil((double) (L * ny) / d.chunks / kThreads);
+      d.rounds_c = (float) std::ceil((double) (QC * d.nseg) / d.chunks / kThreads);
     }
     const bool fits = (size_t) (p.nt + 1) * esz <= lds_cap;     // + the spare bin
+    // A disc's rows see few bins at a time (about 20 of a wave's lanes share
+    // one): four copies of a short histogram part them.
+    d.copies = p.shape == SIR_CIRC && p.nt < 1000 ? 4 : 1;
     d.mode = !fits ? SIR_GLOBAL : (d.chunks > 1 ? SIR_LDS_ATOMIC : SIR_LDS_STORE);
-    if (fits) max_nt_lds = std::max(max_nt_lds, p.nt);
+    if (fits) max_nt_lds = std::max(max_nt_lds, (p.nt + 1) * d.copies - 1);
     cost[i] = (double) Q * (double) nx / d.chunks;
     table_doubles += xs[i].size() + ys[i].size() + el[i].size() + rx0[i].size() + rn[i].size()
-                   + zr[i].size();
+                   + rdx[i].size() + zr[i].size();
     levels_.push_back(p.err_level);
   }
 
@@ -1000,6 +1105,9 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
     tables.insert(tables.end(), rx0[i].begin(), rx0[i].end());
     d.row_n = d_tables_ + tables.size();
     tables.insert(tables.end(), rn[i].begin(), rn[i].end());
+    d.row_dx = d_tables_ + tables.size();
+    d.row_idx = d.row_dx + rdx[i].size() / 2;
+    tables.insert(tables.end(), rdx[i].begin(), rdx[i].end());
     d.zrow = d_tables_ + tables.size();
     tables.insert(tables.end(), zr[i].begin(), zr[i].end());
     d.status = d_status_ + i;

@@ -33,27 +33,39 @@ struct SirDev {
   const double *delay;  int32_t delay_multi;
   int32_t L;
   const double *xs;  const double *ys;  int32_t nx, ny, row_stride, chunks;
-  // Discs: per-row first x position and sub-element count (doubles).
-  const double *row_x0;  const double *row_n;  double dx;  int32_t shape, pad1;
+  // Discs: per-row first x position, sub-element count, mean step and its
+  // reciprocal (doubles).  ny counts the rows' nseg parts, each part_len =
+  // 1/nseg of its row: j is part j / rows of row j % rows.
+  const double *row_x0;  const double *row_n;  const double *row_dx;  const double *row_idx;
+  double dx, part_len;
+  int32_t shape, rows;
   // Cylinders: per-row z offset of the curved surface (rz = z - zrow).
   const double *zrow;
   int32_t step_e, step_j, step_row, pad0;   // row walk: q += 256 as (e, j, row) steps
   const double *el;                 // 6 x L: gx gy gz foc steer num
   int64_t nt;
   double cp, dt, inv_dt, c1, amp;   // c1 = 1000/(cp dt), amp = 1000/(2 pi dt)
+  double ic1;                       // 1/c1
   void *h;
   Status *status;
   int64_t item_begin;               // first work item of this problem
   int32_t mode;                     // SIR_* below
+  int32_t copies;                   // of the LDS histogram: a power of two
   // Column walk (rectangles): the (element, x column) pairs, each cut into
   // nseg segments of seg_len rows, as units u = sg*(L*nx) + i*L + e; u +=
-  // 256 steps (e, i, sg) by cstep_*.  0 segments: rows only; walk 1: every
-  // point walks columns (else each point picks its cheaper walk).
+  // 256 steps (e, i, sg) by cstep_*.  0 segments: rows only.
   int32_t nseg;
-  int32_t seg_len, cstep_e, cstep_i, cstep_sg, walk;
-  // The walk choice: mean |xs| and |ys|, and dx, dy in samples of path
-  // (dx / (cp dt/1000), dy / (cp dt/1000)).
-  double wx, wy, sx, sy;
+  int32_t seg_len, cstep_e, cstep_i, cstep_sg;
+  // The walk of every point (0 rows, 1 columns, 2 runs), or -1: each point
+  // picks its cheapest, runs among them if `runs` is set.
+  int32_t walk, runs;
+  // The lines of the run walk over a rectangle's columns: positions
+  // line_p0 + k line_dv.
+  double line_p0, line_dv, line_inv_dv;
+  // The walk choice: mean |xs| and |ys|, dx and dy in samples of path
+  // (dx / (cp dt/1000), dy / (cp dt/1000)), lane rounds per item of the row
+  // and the column walk.
+  float wx, wy, sx, sy, rounds_r, rounds_c;
 };
 
 enum { SIR_LDS_STORE = 0, SIR_LDS_ATOMIC = 1, SIR_GLOBAL = 2 };
@@ -66,10 +78,9 @@ enum { SIR_RECT = 0, SIR_CIRC = 1, SIR_CYLIND = 2 };
 void disc_rows(double R, double dx, double dy, std::vector<double> &ys,
                std::vector<double> &x0, std::vector<double> &count);
 
-// Cuts disc rows into segments of equal-ish length for lane balance
-// (tables as disc_rows gives them; L elements per point).
-void split_disc_rows(int64_t L, double dx, std::vector<double> &ys, std::vector<double> &x0,
-                     std::vector<double> &count);
+// Mean step of the accumulated x walk of a disc row that starts at x0 (< 0)
+// and ends near -x0, to a few 1e-14 of the disc's size.
+double disc_row_step(double x0, double count, double dx);
 
 // Sub-element rows of a cylindrically curved element of y-size b and
 // curvature radius Rc (src/dreamcylind.cc:288-350): the rows are angles phi

@@ -1,0 +1,157 @@
+// sir_runs.hpp -- one line of equally spaced sub-elements, run by run.
+//
+// Along a line the coordinate offset is v_k = v0 - k dv and the distance
+// r_k = sqrt(v_k^2 + w); on each side of the foot of the perpendicular r
+// rises outwards, so the sub-elements of one sample bin are one run of
+// consecutive steps.  Instead of evaluating every sub-element's index,
+// walk_half solves for the step at which r crosses the bin's upper edge, and
+// sums 1/r over the run in closed form: with c the run's middle, n its
+// length and x the offset from it,
+//   1/r(c + x) = 1/r_c sum_j (-x/r_c)^j P_j(v_c/r_c)     (Legendre),
+// whose odd terms cancel over the run and whose even ones need only the
+// moments of 0 .. n-1.  Runs are cut at n dv <= r/30 (r/20 for an FP32
+// output), where the terms to P6 (P4) leave at most 7e-16 |P8| (2e-10) of
+// the sum, r/30 being a compromise: at r/41 (6e-17) the annular benchmark has
+// a quarter more runs.
+//
+// A bin edge that falls so close to a sub-element that the estimate could
+// round differently from the exact index sequence ends the walk there: the
+// caller steps the rest of the half by exact indices (about one line in 10^4;
+// keeping the exact sequence out of the loop keeps its registers out).  With
+// B the certification bound in samples, u = c1 r - c2 the index before
+// rounding, T the edge and vb > 0 the offset there, sub-element k is
+// certified when
+//   |u_k - T| = c1 |v_k^2 - vb^2| / (r_k + R) >= c1 dv |k - k*| vb / (2.2 R)
+// is at least B (r_k + R <= 2.2 R as w >= (8 dv)^2), k* the crossing.
+#pragma once
+
+#include <cmath>
+
+#if defined(__HIP_DEVICE_COMPILE__)
+#define DREAM_RUNS_FN __device__ __forceinline__
+#elif defined(__HIPCC__)
+#define DREAM_RUNS_FN __host__ __device__ inline
+#else
+#define DREAM_RUNS_FN inline
+#endif
+
+namespace dream {
+
+DREAM_RUNS_FN double runs_rsq(double s)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_rsq(s);
+#else
+  return (double) (float) (1.0 / std::sqrt(s));
+#endif
+}
+
+// sqrt(s), s > 0, to 2^-46.
+DREAM_RUNS_FN double runs_sqrt(double s)
+{
+  const double y = runs_rsq(s), g = s * y;
+  return __builtin_fma(0.5 * g, __builtin_fma(-g, y, 1.0), g);
+}
+
+// One line: v_k = v0 - k dv for 0 <= k < n, w the sum of the other two
+// squares, u = c1 r - c2, ic1 = 1/c1, bound the certification margin; and
+// what runs_ready derives from them.
+struct RunLine {
+  double v0, dv, inv_dv, w, c1, ic1, c2, bound;
+  double roff;    // the upper edge of bin b is b ic1 + roff
+  double tol;     // step j is certified when |j - j*| vb >= tol
+  int foot;       // first sub-element past the foot, within [0, n]
+  int cap;        // a run's longest length
+};
+
+// Whether walk_half holds on this line (n sub-elements): positive spacing,
+// at most four bins per step, w clear of both the spacing and the bin width,
+// and bins that fit an int.  False for NaN.
+template <bool REFINE>
+DREAM_RUNS_FN bool runs_ready(RunLine &l, int n)
+{
+  const double va = __builtin_fabs(l.v0), vz = __builtin_fabs(__builtin_fma(-(double) n, l.dv, l.v0));
+  const double vm = va > vz ? va : vz;
+  const double r = runs_sqrt(__builtin_fma(vm, vm, l.w));        // the line's longest distance
+  const double f = __builtin_ceil(l.v0 * l.inv_dv);
+  l.foot = f > 0.0 ? (f < (double) n ? (int) f : n) : 0;
+  l.roff = (l.c2 + 0.5) * l.ic1;
+  l.tol = 2.2 * l.bound * l.ic1 * l.inv_dv * r;
+  const double m = l.w * runs_rsq(l.w) * l.inv_dv * (REFINE ? 1.0 / 30.0 : 1.0 / 20.0);
+  l.cap = m > 1.0 ? (int) (m < 1e6 ? m : 1e6) : 1;
+  return l.dv > 0.0 && l.c1 * l.dv <= 4.0 && l.w >= 64.0 * (l.dv * l.dv) &&
+         l.w >= 4.0 * (l.ic1 * l.ic1) && l.w < 1e200 &&
+         l.c1 * r + __builtin_fabs(l.c2) < 0x1p30 && r * l.inv_dv < 0x1p30;
+}
+
+// The two halves of sub-elements [k0, k1): half 0 starts at the first one
+// past the foot and goes up, half 1 starts before it and goes down.  Sets
+// the half's length and returns its first sub-element; step j of it is
+// sub-element first + j (first - j).
+DREAM_RUNS_FN int half_of(const RunLine &l, int half, int k0, int k1, int &len)
+{
+  const int kc = l.foot < k0 ? k0 : l.foot > k1 ? k1 : l.foot;
+  len = half ? kc - k0 : k1 - kc;
+  return half ? kc - 1 : kc;
+}
+
+// Walks one half (first and len as half_of gives them) outwards:
+// emit(bin, n, sum) for each run (n may be 0), sum being the run's sum of
+// 1/r.  Returns the number of steps walked: len, or up to where an index is
+// not certified.  It ends: an iteration that takes no step raises the bin,
+// and with it the crossing (bins fit 30 bits, so r rises every time), until
+// the crossing passes a step or is not certified (NaN included).
+template <bool REFINE, typename Emit>
+DREAM_RUNS_FN int walk_half(const RunLine &l, int half, int first, int len, Emit emit)
+{
+  if (len <= 0) return 0;
+  const double ac = __builtin_fma((double) first, l.dv, -l.v0);
+  const double a0 = half ? -ac : ac;                  // offset of step 0, >= 0
+  const double us = __builtin_fma(runs_sqrt(__builtin_fma(a0, a0, l.w)), l.c1, -l.c2);
+  const double bs = __builtin_rint(us);
+  if (!(__builtin_fabs(us - bs) <= 0.5 - l.bound)) return 0;
+  int b = (int) bs;
+  const double as = __builtin_fma(-a0, l.inv_dv, 1.0), am = a0 - 0.5 * l.dv;
+  const double half_dv = 0.5 * l.dv, half_inv = 0.5 * l.inv_dv;
+  // t and p below in units that leave the products' leading factors 1.
+  constexpr double kT = 0x1.0cfeeb28b9fabp+2;         // 74.25^(1/3)
+  const double wt = kT * l.w, p1 = l.dv * l.dv * (1.0 / 12.0);
+  int j = 0;
+  bool sure;
+  do {
+    const double r = __builtin_fma((double) b, l.ic1, l.roff), rr = __builtin_fma(r, r, -l.w);
+    const double yr = runs_rsq(rr), g = rr * yr;
+    const double js1 = __builtin_fma(g, __builtin_fma(__builtin_fma(-g, yr, 1.0), half_inv, l.inv_dv), as);
+    sure = __builtin_fabs(js1 - __builtin_rint(js1)) * g >= l.tol;   // j* + 1
+    const int je = sure ? (int) js1 : j;
+    const int lim = j + l.cap < len ? j + l.cap : len;
+    const int jt = je > j ? je : j, jn = jt < lim ? jt : lim;
+    const int n = jn - j;
+    // The run's middle, its 1/r to 2^-69 (2^-46), t = kT w/r^2, p =
+    // (dv/r)^2/12 and d = p (n^2 - 1).
+    const double vm = __builtin_fma((double) (j + jn), half_dv, am);
+    const double s = __builtin_fma(vm, vm, l.w);
+    const double y = runs_rsq(s), e = __builtin_fma(-(s * y), y, 1.0);
+    const double q = __builtin_fma(y * e, REFINE ? __builtin_fma(0.375, e, 0.5) : 0.5, y);
+    const double nd = (double) n;
+    const double z = q * q, t = wt * z, p = p1 * z;
+    const double d = __builtin_fma(nd * nd, p, -p), h = __builtin_fma(-2.0, p, d);
+    // P2k(v/r), in factors of t = kT (1 - (v/r)^2), times the run's mean
+    // 2k-th power of offset / r^2k, over d.
+    double c = __builtin_fma(-1.5 / kT, t, 1.0);
+    constexpr double k4 = 4.375 / (kT * kT);
+    c = __builtin_fma((t - kT * 0x1.c4d1c42d7271dp-1) * (t - kT * 0x1.08a59c3764410p-2),
+                      __builtin_fma(1.8 * k4, h, 1.2 * k4 * p), c);
+    if (REFINE)
+      c = __builtin_fma((kT * 0x1.e2d8e04e1dfa8p-1 - t) * (kT * 0x1.20279a611af21p-1 - t) *
+                            (kT * 0x1.0b43e6b779650p-3 - t),
+                        __builtin_fma(0.75 * h, h, p * p), c);
+    const double nq = nd * q;
+    emit(b, n, __builtin_fma(nq * d, c, nq));
+    b += sure && je <= lim ? 1 : 0;
+    j = jn;
+  } while (sure && j < len);
+  return j;
+}
+
+} // namespace dream

@@ -317,3 +317,46 @@ def test_rsqrt_seed_accuracy(gpu):
     rel = np.abs(y * np.sqrt(s) - 1.0)
     assert rel.max() <= 2.0 ** -23, np.log2(rel.max())
 
+
+
+@pytest.mark.parametrize("shape", ["rect", "circ"])
+@pytest.mark.parametrize("walk", ["runs", "auto"])
+@pytest.mark.parametrize("size,step,dt,nt,near", [
+    (0.0625, 0.0625, 0.125, 40, 6.0),     # one sub-element; positions on a grid, so ties
+    (0.19, 0.0625, 0.125, 60, 2.0),       # two or three, points on the grid
+    (3.0, 0.0625, 0.125, 500, 0.3),       # lines too near for runs beside usable ones
+    (4.03, 0.05, 0.25, 300, 8.0),         # long runs, cut at their longest
+    (1.7, 0.05, 0.015, 900, 5.0),         # more than two bins a step
+    (2.2, 0.09, 0.01, 9000, 6.0),         # a response too long for LDS; 6 bins a step (no runs)
+])
+def test_run_walk(gpu, oracle, monkeypatch, shape, walk, size, step, dt, nt, near):
+    """Runs against the oracle: output, out-of-range counts, FP32 output.
+    The bar of 1e-12 is this file's; a moved sub-element is at least 1e-4."""
+    from dream_amd.torch_ops import arr_circ, arr_rect
+    if walk != "auto":
+        monkeypatch.setenv("DREAM_HIP_SIR_WALK", walk)
+    rng = np.random.default_rng(int(1000 * size))
+    No, L, cp = 40, 3, 1000.0
+    G = np.c_[[-2.0, 0.0, 2.5], [0.0, 0.25, -0.5], np.zeros(L)]
+    Ro = np.c_[rng.uniform(-4, 4, No), rng.uniform(-3, 3, No), rng.uniform(near, near + 12, No)]
+    if step == 0.0625:
+        Ro = np.rint(Ro * 16) / 16 + [0, 0, 0.3125]
+    delay = np.rint(np.linalg.norm(Ro, axis=1) / (cp * dt / 1000) - 0.3 * nt) * dt
+    delay[::2] += 0.5 * dt
+    kw = dict(err_level="ignore")
+    Rt, dl = torch.tensor(Ro.T.copy(), device="cuda"), torch.tensor(delay, device="cuda")
+    if shape == "rect":
+        ref, _, oob = oracle.dream_arr_rect(Ro, 0.3, size, step, step, dt, nt, delay, 1.0, cp, G,
+                                            nthreads=4, **kw)
+        args = (Rt, 0.3, size, step, step, dt, nt, dl, 1.0, cp, G)
+        fn = arr_rect
+    else:
+        ref, _, oob = oracle.dream_arr_circ(Ro, size / 2, step, step, dt, nt, delay, 1.0, cp, G,
+                                            nthreads=4, **kw)
+        args = (Rt, size / 2, step, step, dt, nt, dl, 1.0, cp, G)
+        fn = arr_circ
+    H, _, n = fn(*args, **kw)
+    assert n == oob
+    assert np.max(np.abs(H.cpu().numpy().T - ref)) <= 1e-12 * max(np.abs(ref).max(), 1e-300)
+    H32, _, n32 = fn(*args, out_dtype=torch.float32, **kw)
+    assert n32 == oob and rel_l2(H32.double().cpu().numpy().T, ref) <= 2e-5
