@@ -805,21 +805,21 @@ __device__ __forceinline__ void fetch_taps(__amdgpu_buffer_rsrc_t r, unsigned ab
 
 // ------------------------------------------------------------ region adjoint
 
-// Region-major adjoint: one work-group per (region of kRegion consecutive
-// pixels in visiting order, group of A-scans, frame).  Each lane keeps its
-// kRPU pixels (coordinates and g) in registers for the whole group, so the
-// pixel data are read once per group rather than once per A-scan.  The
-// Y-gradient of every A-scan of the group is scattered into an LDS window of
-// kWin samples whose start comes from the distance range between the
-// element(s) and the region's bounding box (exact interval bound plus a
-// 2-sample margin); a contribution that falls outside its window (regions
-// with a large extent) is added to gY directly.  Windows are added into the
-// zeroed gY once at the end.  Per-A-scan sums of g*value (for the
-// apodization gradients) stay in registers and are reduced once.
+// Region-major adjoint of SAFT: one work-group per (region of kRegion
+// consecutive pixels in visiting order, group of A-scans, frame).  Each lane
+// keeps its kRPU pixels (coordinates and g) in registers for the whole
+// group, so the pixel data are read once per group rather than once per
+// A-scan.  The Y-gradient of every A-scan of the group is scattered into an
+// LDS window of kWin samples whose start comes from the distance range
+// between the element and the region's bounding box (exact interval bound
+// plus a 2-sample margin); a contribution that falls outside its window
+// (regions with a large extent) is added to gY directly.  Windows are added
+// into the zeroed gY once at the end.  Per-A-scan sums of g*value (for the
+// apodization gradient) stay in registers and are reduced once.
 constexpr int kRPU = 4;                         // pixels per lane
 constexpr int kRegion = kThreads * kRPU;        // pixels per region
 constexpr int kSaftGroup = 8;                   // SAFT A-scans per work-group
-constexpr int kGI = 2, kGJ = 4;                 // two-leg group: transmits x receives
+constexpr int kGI = 2, kGJ = 4;                 // two-leg step: transmits x receives
 constexpr int kWin = 512;                       // LDS window (samples) per A-scan
 
 template <typename T>
@@ -852,11 +852,11 @@ __device__ __forceinline__ int window_start(double umin)
   return (int) floor(umin) - 2;
 }
 
-template <typename DT, typename GT, int TYPE, int INTERP, bool APOD>
+template <typename DT, typename GT, int INTERP, bool APOD>
 __global__ void __launch_bounds__(kThreads)
-das_adj_region_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int subs)
+das_adj_region_kernel(DasArgs A, const int32_t *__restrict__ perm, int subs)
 {
-  constexpr int NA = TYPE == DAS_SAFT ? kSaftGroup : kGI * kGJ;
+  constexpr int NA = kSaftGroup;
   extern __shared__ __align__(16) unsigned char smem[];
   // NA x kWin FP64 accumulators (only when gY is wanted): gfx950's LDS FP64
   // atomic add is about 20 times faster than its FP32 one.
@@ -868,30 +868,20 @@ das_adj_region_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t region = (int64_t) blockIdx.x + A.block0;
-  const int grp = blockIdx.y;
+  const int n0 = (int) blockIdx.y * kSaftGroup;       // the group's A-scans: elements n0 ..
   const int64_t frame = (int64_t) blockIdx.z + A.frame0;
-  const int Lt = A.Lt, Lr = A.Lr;
+  const int Lt = A.Lt;
   const int K = (int) A.K;
   const bool want_gy = A.gY != nullptr;
-  // The group's A-scans: SAFT elements n0.. ; two-leg transmits i0.. x receives j0..
-  int n0 = 0, i0 = 0, j0 = 0;
-  if (TYPE == DAS_SAFT) n0 = grp * kSaftGroup;
-  else { i0 = (grp / n_gj) * kGI; j0 = (grp % n_gj) * kGJ; }
 
   const GT *Ro = (const GT *) A.Ro;
   const GT *Gt = (const GT *) A.Gt;
-  const GT *Gr = (const GT *) A.Gr;
   const GT fs = (GT) A.fs_khz, inv_cp = (GT) A.inv_cp, dl = (GT) A.delay_ms;
   const GT tmax = (GT) A.leg_max;
   const GT bnd = (GT) (0x1p-40 * (fabs(2.0 * (double) fs * (double) dl) + 1.0));
   const GT fs2 = fs + fs;
   const DT *g = (const DT *) A.g + frame * A.im_stride;
   const DT *at = (const DT *) A.apod_t;
-  const DT *ar = (const DT *) A.apod_r;
-  GT y_lo = 0, y_hi = 0, x_lo = 0, x_hi = 0;
-  if (TYPE == DAS_RCA_COLTX || TYPE == DAS_RCA_ROWTX) {
-    y_lo = Gr[Lt]; y_hi = Gr[2 * Lt - 1]; x_lo = Gt[0]; x_hi = Gt[Lr - 1];
-  }
 
   // The work-group covers `subs` consecutive regions, one after the other,
   // with one set of windows (flushed once) spanning all of them.
@@ -931,39 +921,14 @@ das_adj_region_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int
           lo[c] = fmin(lo[c], s_box[c][w]); hi[c] = fmax(hi[c], s_box[3 + c][w]);
         }
       }
-      // Distance ranges of the legs to the box, then the sample range.
-      double umin;
-      if (TYPE == DAS_SAFT) {
-        const int n = min(n0 + (int) threadIdx.x, Lt - 1);
-        GT m0, m1, m2, x0, x1, x2;
-        gap_range<GT>(Gt[n], lo[0], hi[0], m0, x0);
-        gap_range<GT>(Gt[n + Lt], lo[1], hi[1], m1, x1);
-        gap_range<GT>(Gt[n + 2 * Lt], lo[2], hi[2], m2, x2);
-        const double dmin = sqrt((double) (m0 * m0 + m1 * m1 + m2 * m2));
-        umin = 2.0 * (dmin * (double) inv_cp + (double) dl) * (double) fs;
-      } else {
-        const int i = min(i0 + (int) threadIdx.x / kGJ, Lt - 1);
-        const int j = min(j0 + (int) threadIdx.x % kGJ, Lr - 1);
-        GT m0, m1, m2, x0, x1, x2;
-        if (TYPE == DAS_TFM) {
-          gap_range<GT>(Gt[i], lo[0], hi[0], m0, x0);
-          gap_range<GT>(Gt[i + Lt], lo[1], hi[1], m1, x1);
-        } else {
-          gap_range<GT>(Gt[i], lo[0], hi[0], m0, x0);
-          stripe_range<GT>(lo[1], hi[1], y_lo, y_hi, m1, x1);
-        }
-        gap_range<GT>(Gt[i + 2 * Lt], lo[2], hi[2], m2, x2);
-        const double dt_min = sqrt((double) (m0 * m0 + m1 * m1 + m2 * m2));
-        if (TYPE == DAS_TFM) {
-          gap_range<GT>(Gr[j], lo[0], hi[0], m0, x0);
-        } else {
-          stripe_range<GT>(lo[0], hi[0], x_lo, x_hi, m0, x0);
-        }
-        gap_range<GT>(Gr[j + Lr], lo[1], hi[1], m1, x1);
-        gap_range<GT>(Gr[j + 2 * Lr], lo[2], hi[2], m2, x2);
-        const double dr_min = sqrt((double) (m0 * m0 + m1 * m1 + m2 * m2));
-        umin = ((dt_min * (double) inv_cp + (double) dl) + dr_min * (double) inv_cp) * (double) fs;
-      }
+      // Distance range of the leg to the box, then the sample range.
+      const int n = min(n0 + (int) threadIdx.x, Lt - 1);
+      GT m0, m1, m2, x0, x1, x2;
+      gap_range<GT>(Gt[n], lo[0], hi[0], m0, x0);
+      gap_range<GT>(Gt[n + Lt], lo[1], hi[1], m1, x1);
+      gap_range<GT>(Gt[n + 2 * Lt], lo[2], hi[2], m2, x2);
+      const double dmin = sqrt((double) (m0 * m0 + m1 * m1 + m2 * m2));
+      const double umin = 2.0 * (dmin * (double) inv_cp + (double) dl) * (double) fs;
       s_w0[threadIdx.x] = window_start(umin);
     }
   }
@@ -992,69 +957,22 @@ das_adj_region_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int
       gp[q] = live[q] ? g[p] : DT(0);
     }
 
-    // Two-leg: receive legs of the group for the lane's pixels.
-    GT tr[TYPE == DAS_SAFT ? 1 : kGJ][kRPU];
-    GT gx_r[kRPU], gy_c[kRPU];
-    if (TYPE != DAS_SAFT) {
-#pragma unroll
-      for (int q = 0; q < kRPU; q++) {
-        gx_r[q] = GT(0); gy_c[q] = GT(0);
-        if (TYPE != DAS_TFM) {
-          gy_c[q] = stripe_gap<GT>(yo[q], y_lo, y_hi);
-          gx_r[q] = stripe_gap<GT>(xo[q], x_lo, x_hi);
-        }
-#pragma unroll
-        for (int jj = 0; jj < kGJ; jj++) {
-          const int j = min(j0 + jj, Lr - 1);
-          if (TYPE == DAS_TFM)
-            tr[jj][q] = leg3<GT>(Gr[j] - xo[q], Gr[j + Lr] - yo[q], Gr[j + 2 * Lr] - zo[q]) * inv_cp;
-          else
-            tr[jj][q] = leg3<GT>(gx_r[q], Gr[j + Lr] - yo[q], Gr[j + 2 * Lr] - zo[q]) * inv_cp;
-        }
-      }
-    }
-
 #pragma unroll
     for (int s = 0; s < NA; s++) {
-      int a, ii = 0, jj = 0;
-      bool ok;
-      DT w;
-      if (TYPE == DAS_SAFT) {
-        const int n = n0 + s;
-        ok = n < Lt;
-        a = min(n, Lt - 1);
-        w = APOD ? at[a] : DT(1);
-      } else {
-        ii = s / kGJ; jj = s % kGJ;
-        const int i = i0 + ii, j = j0 + jj;
-        ok = i < Lt && j < Lr;
-        const int ic = min(i, Lt - 1), jc = min(j, Lr - 1);
-        a = (TYPE == DAS_RCA_ROWTX) ? jc * Lt + ic : ic * Lr + jc;
-        w = APOD ? at[ic] * ar[jc] : DT(1);
-      }
-      if (!ok) continue;                           // uniform
+      const int n = n0 + s;
+      if (n >= Lt) continue;                       // uniform
+      const int a = n;
+      const DT w = APOD ? at[a] : DT(1);
       const unsigned abase = (unsigned) a * (unsigned) K;
       const int w0 = want_gy ? s_w0[s] : 0;
       GT u[kRPU], tsum[kRPU];
 #pragma unroll
       for (int q = 0; q < kRPU; q++) {
-        if (TYPE == DAS_SAFT) {
-          GT tleg;
-          u[q] = saft_pos<GT, kSaftFast<DT, GT, INTERP>>(Gt[a] - xo[q], Gt[a + Lt] - yo[q],
-                                                        Gt[a + 2 * Lt] - zo[q], inv_cp, dl, tmax,
-                                                        fs, fs2, bnd, tleg);
-          tsum[q] = tleg + tleg;
-        } else {
-          const int i = min(i0 + ii, Lt - 1);
-          GT tt;
-          if (TYPE == DAS_TFM)
-            tt = leg3<GT>(Gt[i] - xo[q], Gt[i + Lt] - yo[q], Gt[i + 2 * Lt] - zo[q]) * inv_cp;
-          else
-            tt = leg3<GT>(Gt[i] - xo[q], gy_c[q], Gt[i + 2 * Lt] - zo[q]) * inv_cp;
-          tsum[q] = tt + tr[jj][q];
-          tt += dl;
-          u[q] = (clamp_leg<GT>(tt, tmax) + clamp_leg<GT>(tr[jj][q], tmax)) * fs;
-        }
+        GT tleg;
+        u[q] = saft_pos<GT, kSaftFast<DT, GT, INTERP>>(Gt[a] - xo[q], Gt[a + Lt] - yo[q],
+                                                      Gt[a + 2 * Lt] - zo[q], inv_cp, dl, tmax,
+                                                      fs, fs2, bnd, tleg);
+        tsum[q] = tleg + tleg;
       }
       DT y0[kRPU], y1[kRPU], f[kRPU];
       int k[kRPU];
@@ -1102,15 +1020,10 @@ das_adj_region_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int
   __syncthreads();
   if (threadIdx.x < NA) {
     const int s = threadIdx.x;
-    int a = -1;
-    if (TYPE == DAS_SAFT) { if (n0 + s < Lt) a = n0 + s; }
-    else {
-      const int i = i0 + s / kGJ, j = j0 + s % kGJ;
-      if (i < Lt && j < Lr) a = (TYPE == DAS_RCA_ROWTX) ? j * Lt + i : i * Lr + j;
-    }
+    const int a = n0 + s;
     double v = 0.0;
     for (int w = 0; w < kThreads / 64; w++) v += s_z[s][w];
-    if (a >= 0 && v != 0.0) atomicAdd(&((double *) A.z_t)[a], v);
+    if (a < Lt && v != 0.0) atomicAdd(&((double *) A.z_t)[a], v);
   }
   if (threadIdx.x == 0 && INTERP == DREAM_HIP_LINEAR) {
     double v = 0.0;
@@ -1124,12 +1037,7 @@ das_adj_region_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int
       const int s = q / kWin;
       const DT v = (DT) win[q];
       if (v == DT(0)) continue;
-      int a;
-      if (TYPE == DAS_SAFT) a = n0 + s;
-      else {
-        const int i = i0 + s / kGJ, j = j0 + s % kGJ;
-        a = (TYPE == DAS_RCA_ROWTX) ? j * Lt + i : i * Lr + j;
-      }
+      const int a = n0 + s;
       const int kk = s_w0[s] + (q - s * kWin);
       if (kk < 0 || kk >= K) continue;           // a linear tap just outside the A-scan
       unsafeAtomicAdd(&gy_frame[(int64_t) a * K + kk], v);
@@ -1354,35 +1262,263 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
   }
 }
 
-// From per-A-scan sums Z[a] (region kernel) to the apodization gradients:
-// SAFT g_t[n] = Z[n]; two-leg g_t[i] = sum_j w_j Z[i,j], g_r[j] = sum_i w_i Z[i,j].
-template <typename DT>
-__global__ void adj_finalize_channel(int type, int Lt, int Lr, const double *Z, const DT *at,
-                                     const DT *ar, const double *zcp, DT *g_t, DT *g_r, DT *g_cp)
+// ------------------------------------------------------------- pair adjoint
+
+// Adjoint with gY for two-leg modes: one work-group per (region of kRegion
+// consecutive pixels in visiting order, kGJ receivers, part of the
+// transmits, frame).  Each lane keeps its kRPU pixels, their g and their
+// receive legs in registers and goes through the part's transmits kGI at a
+// time, so that a pair costs a quarter of a transmit leg and no receive leg;
+// each step scatters into the windows of its kGI x kGJ A-scans (LDS, FP64,
+// their starts from the distance ranges to the region's bounding box as in the
+// region adjoint) and adds them into gY.  Apodization sums go to z_t and z_r
+// as in the pixel adjoint.  Bound by the latency of its gathers and LDS adds
+// at three waves per SIMD (four spill: 250 -> 276 us): its 59 instructions a
+// pair fill 43 % of the issue slots, the LDS is busy 34 % of the time and the
+// gathers' address path about as much.  A work-group per group of 2 x 4
+// A-scans computed six legs, a bounding box and nine shuffle sums per 32 pairs
+// of a lane, 110 instructions a pair: 48 x 48 over 30720 pixels, linear, FP32
+// took 352 us, now 250.
+constexpr int kPartI = 64;                      // transmits of a part, at most
+
+template <typename DT, typename GT, int TYPE, int INTERP, bool APOD>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
+das_adj_pairs_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int parts)
 {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (type == DAS_SAFT) {
-    if (q < Lt && g_t) g_t[q] = (DT) Z[q];
-  } else {
-    auto Zij = [&](int i, int j) {
-      return Z[type == DAS_RCA_ROWTX ? (int64_t) j * Lt + i : (int64_t) i * Lr + j];
-    };
-    if (q < Lt && g_t) {
-      double s = 0.0;
-      for (int j = 0; j < Lr; j++) s += (ar ? (double) ar[j] : 1.0) * Zij(q, j);
-      g_t[q] = (DT) s;
+  constexpr int NA = kGI * kGJ, kWaves = kThreads / 64;
+  extern __shared__ __align__(16) unsigned char smem[];
+  double *win = reinterpret_cast<double *>(smem);
+  __shared__ GT s_box[6][kWaves], s_lim[6];
+  __shared__ int s_w0[2][NA];
+  __shared__ double s_zt[kPartI], s_zr[kGJ], s_cp[kWaves];
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t base = ((int64_t) blockIdx.x + A.block0) * kRegion;
+  const int64_t frame = (int64_t) blockIdx.z + A.frame0;
+  const int Lt = A.Lt, Lr = A.Lr;
+  const int K = (int) A.K;
+  const unsigned KB = (unsigned) K * (unsigned) sizeof(DT);
+  const int j0 = ((int) blockIdx.y % n_gj) * kGJ, part = (int) blockIdx.y / n_gj;
+  const int n_gi = (Lt + kGI - 1) / kGI;
+  const int g0 = (int) ((int64_t) part * n_gi / parts), g1 = (int) ((int64_t) (part + 1) * n_gi / parts);
+  const GT *Ro = (const GT *) A.Ro;
+  const GT *Gt = (const GT *) A.Gt;
+  const GT *Gr = (const GT *) A.Gr;
+  const GT fs = (GT) A.fs_khz, inv_cp = (GT) A.inv_cp, dl = (GT) A.delay_ms;
+  const GT tmax = (GT) A.leg_max;
+  const DT *g = (const DT *) A.g + frame * A.im_stride;
+  const DT *at = (const DT *) A.apod_t;
+  const DT *ar = (const DT *) A.apod_r;
+  GT y_lo = 0, y_hi = 0, x_lo = 0, x_hi = 0;
+  if (TYPE != DAS_TFM) { y_lo = Gr[Lt]; y_hi = Gr[2 * Lt - 1]; x_lo = Gt[0]; x_hi = Gt[Lr - 1]; }
+
+  // Lanes take their 64-pixel block transposed, as in the region adjoint.
+  const int lane_pos = (int) ((threadIdx.x & ~63u) | ((threadIdx.x & 7u) << 3) | ((threadIdx.x >> 3) & 7u));
+  GT xo[kRPU], yo[kRPU], zo[kRPU], tr[kGJ][kRPU];
+  DT gp[kRPU];
+  bool live[kRPU];
+  {
+    GT bmin[3] = {INFINITY, INFINITY, INFINITY}, bmax[3] = {-INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+    for (int q = 0; q < kRPU; q++) {
+      const int64_t idx = base + (int64_t) q * kThreads + lane_pos;
+      live[q] = idx < A.No;
+      const int64_t p = pixel_of(perm, live[q] ? idx : 0);
+      xo[q] = Ro[p]; yo[q] = Ro[p + A.No]; zo[q] = Ro[p + 2 * A.No];
+      gp[q] = live[q] ? g[p] : DT(0);
+      if (live[q]) {
+        bmin[0] = fmin(bmin[0], xo[q]); bmax[0] = fmax(bmax[0], xo[q]);
+        bmin[1] = fmin(bmin[1], yo[q]); bmax[1] = fmax(bmax[1], yo[q]);
+        bmin[2] = fmin(bmin[2], zo[q]); bmax[2] = fmax(bmax[2], zo[q]);
+      }
     }
-    if (q < Lr && g_r) {
-      double s = 0.0;
-      for (int i = 0; i < Lt; i++) s += (at ? (double) at[i] : 1.0) * Zij(i, q);
-      g_r[q] = (DT) s;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      GT mn = bmin[c], mx = bmax[c];
+      for (int off = 32; off > 0; off >>= 1) {
+        mn = fmin(mn, __shfl_xor(mn, off, 64));
+        mx = fmax(mx, __shfl_xor(mx, off, 64));
+      }
+      if (lane == 0) { s_box[c][wave] = mn; s_box[3 + c][wave] = mx; }
     }
   }
-  if (q == 0 && g_cp) *g_cp = (DT) *zcp;
+  for (int s = threadIdx.x; s < NA * kWin; s += kThreads) win[s] = 0.0;
+  if (threadIdx.x < kPartI) s_zt[threadIdx.x] = 0.0;
+  if (threadIdx.x < kGJ) s_zr[threadIdx.x] = 0.0;
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    GT v = s_box[threadIdx.x][0];
+    for (int w = 1; w < kWaves; w++) {
+      const GT o = s_box[threadIdx.x][w];
+      v = threadIdx.x < 3 ? fmin(v, o) : fmax(v, o);
+    }
+    s_lim[threadIdx.x] = v;
+  }
+  double zcp = 0.0;
+  // Stripe gaps in y (transmit leg) and the receive legs.
+  GT gy_c[kRPU];
+#pragma unroll
+  for (int q = 0; q < kRPU; q++) {
+    gy_c[q] = TYPE == DAS_TFM ? GT(0) : stripe_gap<GT>(yo[q], y_lo, y_hi);
+    const GT gx = TYPE == DAS_TFM ? GT(0) : stripe_gap<GT>(xo[q], x_lo, x_hi);
+#pragma unroll
+    for (int jj = 0; jj < kGJ; jj++) {
+      const int j = min(j0 + jj, Lr - 1);
+      const GT dx = TYPE == DAS_TFM ? Gr[j] - xo[q] : gx;
+      const GT t = leg3_wave<GT>(dx, Gr[j + Lr] - yo[q], Gr[j + 2 * Lr] - zo[q]) * inv_cp;
+      // Clamped (a pair that this changes is out of range, its cp term 0);
+      // a leg that is not finite makes the cp gradient NaN.
+      tr[jj][q] = clamp_leg<GT>(t, tmax);
+      if (INTERP == DREAM_HIP_LINEAR) zcp += (double) t * 0.0;
+    }
+  }
+  __syncthreads();
+
+  // The first sample of A-scan s of transmit group gi: the distance ranges of
+  // the legs to the box.
+  auto window_of = [&](int gi, int s) {
+    const int i = min(gi * kGI + s / kGJ, Lt - 1), j = min(j0 + s % kGJ, Lr - 1);
+    const GT lo0 = s_lim[0], lo1 = s_lim[1], lo2 = s_lim[2], hi0 = s_lim[3], hi1 = s_lim[4], hi2 = s_lim[5];
+    GT m0, m1, m2, x;
+    gap_range<GT>(Gt[i], lo0, hi0, m0, x);
+    if (TYPE == DAS_TFM) gap_range<GT>(Gt[i + Lt], lo1, hi1, m1, x);
+    else stripe_range<GT>(lo1, hi1, y_lo, y_hi, m1, x);
+    gap_range<GT>(Gt[i + 2 * Lt], lo2, hi2, m2, x);
+    const double dt_min = sqrt((double) (m0 * m0 + m1 * m1 + m2 * m2));
+    if (TYPE == DAS_TFM) gap_range<GT>(Gr[j], lo0, hi0, m0, x);
+    else stripe_range<GT>(lo0, hi0, x_lo, x_hi, m0, x);
+    gap_range<GT>(Gr[j + Lr], lo1, hi1, m1, x);
+    gap_range<GT>(Gr[j + 2 * Lr], lo2, hi2, m2, x);
+    const double dr_min = sqrt((double) (m0 * m0 + m1 * m1 + m2 * m2));
+    return window_start(((dt_min * (double) inv_cp + (double) dl) + dr_min * (double) inv_cp) *
+                        (double) fs);
+  };
+  if (threadIdx.x < NA) s_w0[0][threadIdx.x] = window_of(g0, threadIdx.x);
+  __syncthreads();
+
+  const __amdgpu_buffer_rsrc_t ry =
+      ascan_rsrc((const DT *) A.Y + frame * A.y_stride, K, (int) sizeof(DT));
+  DT *gy_frame = (DT *) A.gY + frame * A.y_stride;
+  double zr[kGJ];
+#pragma unroll
+  for (int jj = 0; jj < kGJ; jj++) zr[jj] = 0.0;
+
+  for (int gi = g0; gi < g1; gi++) {
+    const int *w0 = s_w0[(gi - g0) & 1];
+#pragma clang loop unroll(disable)
+    for (int ii = 0; ii < kGI; ii++) {
+      const int i = gi * kGI + ii;
+      if (i >= Lt) break;                          // uniform
+      const DT wi = APOD ? at[i] : DT(1);
+      GT tt0[kRPU], tt[kRPU];
+#pragma unroll
+      for (int q = 0; q < kRPU; q++) {
+        const GT dy = TYPE == DAS_TFM ? Gt[i + Lt] - yo[q] : gy_c[q];
+        tt0[q] = leg3_wave<GT>(Gt[i] - xo[q], dy, Gt[i + 2 * Lt] - zo[q]) * inv_cp;
+        tt[q] = clamp_leg<GT>(tt0[q] + dl, tmax);
+      }
+      double zi = 0.0;
+#pragma unroll
+      for (int jj = 0; jj < kGJ; jj++) {
+        const int j = j0 + jj;
+        if (j >= Lr) continue;                     // uniform
+        DT f[kRPU], y0[kRPU], y1[kRPU];
+        int k[kRPU];
+#pragma unroll
+        for (int q = 0; q < kRPU; q++) {
+          unsigned o0, o1;
+          gather_index<DT, GT, INTERP, true>((tt[q] + tr[jj][q]) * fs, true, o0, o1, f[q], k[q]);
+          if (!live[q]) k[q] = -2;                 // neither tap exists
+        }
+        const unsigned a = (unsigned) (TYPE == DAS_RCA_ROWTX ? j * Lt + i : i * Lr + j);
+#pragma unroll
+        for (int q = 0; q < kRPU; q++) {
+          y0[q] = sload<DT>(ry, (unsigned) k[q], a * KB);
+          if (INTERP != DREAM_HIP_NEAREST) y1[q] = sload<DT>(ry, (unsigned) (k[q] + 1), a * KB);
+        }
+        const int s = ii * kGJ + jj;
+        const DT wj = APOD ? ar[j] : DT(1), w = wi * wj;
+        const int ws = w0[s];
+        DT *ga = gy_frame + (int64_t) a * K;
+        DT z = DT(0), zc = DT(0);                  // over the lane's pixels
+#pragma unroll
+        for (int q = 0; q < kRPU; q++) {
+          DT val = y0[q];
+          const DT gw = gp[q] * w;
+          const int kk = k[q];
+          const unsigned l = (unsigned) (kk - ws);
+          if (INTERP == DREAM_HIP_NEAREST) {
+            if ((unsigned) kk < (unsigned) K) {
+              if (l < (unsigned) kWin) lds_atomic_add(&win[s * kWin + l], (double) gw);
+              else unsafeAtomicAdd(&ga[kk], gw);
+            }
+          } else {
+            const DT slope = y1[q] - y0[q];
+            val += f[q] * slope;
+            zc += (gp[q] * slope) * (DT) (tt0[q] + tr[jj][q]);
+            // One of the taps in [0, K); a window's entries outside it are dropped.
+            if ((unsigned) (kk + 1) <= (unsigned) K) {
+              const DT v0 = gw * (DT(1) - f[q]), v1 = gw * f[q];
+              if (l + 1u < (unsigned) kWin) {
+                lds_atomic_add(&win[s * kWin + l], (double) v0);
+                lds_atomic_add(&win[s * kWin + l + 1], (double) v1);
+              } else {
+                if (kk >= 0 && kk < K) unsafeAtomicAdd(&ga[kk], v0);
+                if (kk + 1 < K) unsafeAtomicAdd(&ga[kk + 1], v1);
+              }
+            }
+          }
+          z += gp[q] * val;
+        }
+        zi = __builtin_fma((double) wj, (double) z, zi);
+        zr[jj] = __builtin_fma((double) wi, (double) z, zr[jj]);
+        if (INTERP == DREAM_HIP_LINEAR) zcp = __builtin_fma((double) w, (double) zc, zcp);
+      }
+      const double total = wave_total(zi);
+      if (lane == 63 && total != 0.0) lds_atomic_add(&s_zt[i - g0 * kGI], total);
+    }
+    // Windows into gY, left zero for the next transmits.
+    if (gi + 1 < g1 && threadIdx.x < NA) s_w0[(gi + 1 - g0) & 1][threadIdx.x] = window_of(gi + 1, threadIdx.x);
+    __syncthreads();
+    for (int q = threadIdx.x; q < NA * kWin; q += kThreads) {
+      const double v = win[q];
+      if (v == 0.0) continue;
+      win[q] = 0.0;
+      const int s = q / kWin, i = gi * kGI + s / kGJ, j = j0 + s % kGJ;
+      const int kk = w0[s] + (q - s * kWin);
+      if (kk < 0 || kk >= K) continue;             // a linear tap just outside the A-scan
+      const int64_t a = TYPE == DAS_RCA_ROWTX ? (int64_t) j * Lt + i : (int64_t) i * Lr + j;
+      unsafeAtomicAdd(&gy_frame[a * K + kk], (DT) v);
+    }
+    __syncthreads();
+  }
+
+#pragma unroll
+  for (int jj = 0; jj < kGJ; jj++) {
+    const double total = wave_total(zr[jj]);
+    if (lane == 63 && total != 0.0) lds_atomic_add(&s_zr[jj], total);
+  }
+  if (INTERP == DREAM_HIP_LINEAR) {
+    const double total = wave_total(zcp);
+    if (lane == 63) s_cp[wave] = total;
+  }
+  __syncthreads();
+  if (threadIdx.x < kPartI && g0 * kGI + (int) threadIdx.x < Lt && s_zt[threadIdx.x] != 0.0)
+    atomicAdd(&((double *) A.z_t)[g0 * kGI + threadIdx.x], s_zt[threadIdx.x]);
+  if (threadIdx.x < kGJ && j0 + (int) threadIdx.x < Lr && s_zr[threadIdx.x] != 0.0)
+    atomicAdd(&((double *) A.z_r)[j0 + threadIdx.x], s_zr[threadIdx.x]);
+  if (threadIdx.x == 0 && INTERP == DREAM_HIP_LINEAR) {
+    double v = 0.0;
+    for (int w = 0; w < kWaves; w++) v += s_cp[w];
+    v *= -(double) A.fs_khz / A.cp;             // du/dcp = -(travel time) fs / cp
+    if (v != 0.0) atomicAdd((double *) A.z_cp, v);
+  }
 }
 
+// From the sums to the apodization gradients: SAFT g_t[n] = Z[n] (Lr = 0),
+// two-leg z_t and z_r.
 template <typename DT>
-__global__ void adj_finalize_pixel(int Lt, int Lr, const double *zt, const double *zr,
+__global__ void adj_finalize(int Lt, int Lr, const double *zt, const double *zr,
                                    const double *zcp, DT *g_t, DT *g_r, DT *g_cp)
 {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1688,7 +1824,7 @@ template <typename DT, typename GT, int TYPE, int INTERP, bool APOD>
 void adj_launch(const DasArgs &a, const int32_t *perm, bool want_gy, hipStream_t s,
                 ChunkGate *gate)
 {
-  if (TYPE == DAS_SAFT || want_gy) {
+  if constexpr (TYPE == DAS_SAFT) {
     // Region-major: (pixel region, A-scan group, frame) work-groups.
     // A work-group takes `subs` consecutive regions (one window flush for
     // all of them).  Candidates 1, 2, 4 while the grid keeps at least four
@@ -1696,14 +1832,7 @@ void adj_launch(const DasArgs &a, const int32_t *perm, bool want_gy, hipStream_t
     // group cover a wider delay range, which coarse pixel grids can
     // overflow into direct gY atomics), the first is the default.
     const int64_t regions1 = (a.No + kRegion - 1) / kRegion;
-    int n_gj = 1;
-    int64_t groups;
-    if (TYPE == DAS_SAFT) {
-      groups = (a.Lt + kSaftGroup - 1) / kSaftGroup;
-    } else {
-      n_gj = (a.Lr + kGJ - 1) / kGJ;
-      groups = (int64_t) ((a.Lt + kGI - 1) / kGI) * n_gj;
-    }
+    const int64_t groups = (a.Lt + kSaftGroup - 1) / kSaftGroup;
     // Largest first (the default), then smaller; a fixed array, so the
     // launch takes no host memory.
     int subs_cand[3], n_subs = 0;
@@ -1711,9 +1840,8 @@ void adj_launch(const DasArgs &a, const int32_t *perm, bool want_gy, hipStream_t
       if ((regions1 + sb - 1) / sb * groups * a.n_frames >= 4 * (int64_t) cu_count())
         subs_cand[n_subs++] = sb;
     subs_cand[n_subs++] = 1;
-    const int na = TYPE == DAS_SAFT ? kSaftGroup : kGI * kGJ;
-    const size_t lds = want_gy ? (size_t) na * kWin * sizeof(double) : 0;
-    const int64_t n_z = TYPE == DAS_SAFT ? a.Lt : (int64_t) a.Lt * a.Lr;
+    const size_t lds = want_gy ? (size_t) kSaftGroup * kWin * sizeof(double) : 0;
+    const int64_t n_z = a.Lt;
     auto run = [&](int subs, bool clear_z, hipStream_t st, ChunkGate *g) {
       if (clear_z) {
         zero_async(a.z_t, (size_t) n_z * sizeof(double), st);
@@ -1728,8 +1856,8 @@ void adj_launch(const DasArgs &a, const int32_t *perm, bool want_gy, hipStream_t
                     c.block0 = b0;
                     c.frame0 = f0;
                     dim3 grid((unsigned) nb, (unsigned) groups, (unsigned) nf);
-                    hipLaunchKernelGGL((das_adj_region_kernel<DT, GT, TYPE, INTERP, APOD>), grid,
-                                       dim3(kThreads), lds, st, c, perm, n_gj, subs);
+                    hipLaunchKernelGGL((das_adj_region_kernel<DT, GT, INTERP, APOD>), grid,
+                                       dim3(kThreads), lds, st, c, perm, subs);
                     DREAM_HIP_CHECK(hipGetLastError());
                   });
     };
@@ -1751,6 +1879,27 @@ void adj_launch(const DasArgs &a, const int32_t *perm, bool want_gy, hipStream_t
       }
     }
     run(subs_cand[pick], false, s, gate);
+  } else if (want_gy) {
+    // (pixel region, receiver group, part of the transmits, frame)
+    // work-groups: the transmits are cut until there are eight per CU (two
+    // rounds of the four that fit), and into parts of at most kPartI.
+    const int64_t regions = (a.No + kRegion - 1) / kRegion;
+    const int n_gj = (a.Lr + kGJ - 1) / kGJ, n_gi = (a.Lt + kGI - 1) / kGI;
+    const int64_t wgs = std::max<int64_t>(regions * n_gj * a.n_frames, 1);
+    const int parts = (int) std::min<int64_t>(
+        n_gi, std::max<int64_t>((n_gi + kPartI / kGI - 1) / (kPartI / kGI), (8 * (int64_t) cu_count() + wgs - 1) / wgs));
+    zero_async(a.gY, (size_t) (a.n_frames * a.y_stride) * sizeof(DT), s);
+    run_chunked(regions, a.n_frames, (int64_t) kRegion * pairs_per_pixel(TYPE, a.Lt, a.Lr), gate,
+                [&](int64_t b0, int64_t nb, int64_t f0, int64_t nf) {
+                  DasArgs c = a;
+                  c.block0 = b0;
+                  c.frame0 = f0;
+                  hipLaunchKernelGGL((das_adj_pairs_kernel<DT, GT, TYPE, INTERP, APOD>),
+                                     dim3((unsigned) nb, (unsigned) (n_gj * parts), (unsigned) nf),
+                                     dim3(kThreads), (size_t) kGI * kGJ * kWin * sizeof(double), s,
+                                     c, perm, n_gj, parts);
+                  DREAM_HIP_CHECK(hipGetLastError());
+                });
   } else {
     // Wave items over (frame or frame group, 64-pixel tile, part of its
     // jobs); a chunk is a range of tiles.  Tiles are split into parts until
@@ -2329,13 +2478,13 @@ void DasHandle::adjoint_dev(const void *Y, const void *Ro, const void *Gt, const
           "das adjoint: one frame of Y must be smaller than 4 GiB");
   require(type_ == DAS_SAFT || gY || (size_t) (Lt_ + Lr_) * 8 <= 65536,
           "das adjoint: too many elements for the apodization accumulators");
-  // Accumulators: Z per A-scan (region kernel) or z_t/z_r (pixel kernel), z_cp.
-  const size_t zbytes = (size_t) (n_ascans + Lt_ + Lr_ + 1) * sizeof(double);
+  // Accumulators: z_t, z_r (two-leg), z_cp.
+  const size_t zbytes = (size_t) (Lt_ + Lr_ + 1) * sizeof(double);
   double *Z;
   if (fixed_z) {
     // Allocation-free call: the caller's fixed workspace, default launch
     // shapes, one launch per kernel (no chunk events).
-    require(zbytes <= fixed_z_bytes,
+    require((size_t) (n_ascans + Lt_ + Lr_ + 1) * sizeof(double) <= fixed_z_bytes,
             "das adjoint: n_ascans + Lt + Lr + 1 exceeds the fixed workspace (262144 doubles)");
     Z = fixed_z;
   } else {
@@ -2349,7 +2498,7 @@ void DasHandle::adjoint_dev(const void *Y, const void *Ro, const void *Gt, const
     }
     Z = (double *) d_z_;
   }
-  double *zt = Z + n_ascans, *zr = zt + Lt_, *zcp = zr + Lr_;
+  double *zr = Z + Lt_, *zcp = zr + Lr_;
   zero_async(Z, zbytes, s);
   DasArgs a;
   fill_args(a, Y, Ro, Gt, Gr, dt, 0, nullptr, cp, apod_t, apod_r, n_frames, y_stride, im_stride,
@@ -2358,12 +2507,11 @@ void DasHandle::adjoint_dev(const void *Y, const void *Ro, const void *Gt, const
   a.g = g;
   a.gY = gY;
   a.z_cp = zcp;
-  const bool channel = type_ == DAS_SAFT || gY != nullptr;
-  a.z_t = channel ? (void *) Z : (void *) zt;
+  a.z_t = Z;
   a.z_r = zr;
   // The pixel kernel reads frames in groups of four (not in the
   // allocation-free call).
-  if (No_ > 0 && !channel && !fixed_z)
+  if (No_ > 0 && type_ != DAS_SAFT && !gY && !fixed_z)
     group_frames(a, Y, y_stride, n_frames, s);
   ChunkGate gate(s);
   if (No_ > 0) {
@@ -2377,25 +2525,12 @@ void DasHandle::adjoint_dev(const void *Y, const void *Ro, const void *Gt, const
   else if (gY) zero_async(gY, (size_t) (n_frames * y_stride) * elem_size(prec_), s);
   const int n = (int) std::max<int64_t>(std::max<int64_t>(Lt_, Lr_), 1);
   const int blocks = (n + 255) / 256;
-  if (prec_ == DREAM_HIP_F64) {
-    if (channel)
-      hipLaunchKernelGGL(adj_finalize_channel<double>, dim3(blocks), dim3(256), 0, s, type_,
-                         (int) Lt_, (int) Lr_, Z, (const double *) apod_t, (const double *) apod_r,
-                         zcp, (double *) g_apod_t, (double *) g_apod_r, (double *) g_cp);
-    else
-      hipLaunchKernelGGL(adj_finalize_pixel<double>, dim3(blocks), dim3(256), 0, s, (int) Lt_,
-                         (int) Lr_, zt, zr, zcp, (double *) g_apod_t, (double *) g_apod_r,
-                         (double *) g_cp);
-  } else {
-    if (channel)
-      hipLaunchKernelGGL(adj_finalize_channel<float>, dim3(blocks), dim3(256), 0, s, type_,
-                         (int) Lt_, (int) Lr_, Z, (const float *) apod_t, (const float *) apod_r,
-                         zcp, (float *) g_apod_t, (float *) g_apod_r, (float *) g_cp);
-    else
-      hipLaunchKernelGGL(adj_finalize_pixel<float>, dim3(blocks), dim3(256), 0, s, (int) Lt_,
-                         (int) Lr_, zt, zr, zcp, (float *) g_apod_t, (float *) g_apod_r,
-                         (float *) g_cp);
-  }
+  if (prec_ == DREAM_HIP_F64)
+    hipLaunchKernelGGL(adj_finalize<double>, dim3(blocks), dim3(256), 0, s, (int) Lt_, (int) Lr_,
+                       Z, zr, zcp, (double *) g_apod_t, (double *) g_apod_r, (double *) g_cp);
+  else
+    hipLaunchKernelGGL(adj_finalize<float>, dim3(blocks), dim3(256), 0, s, (int) Lt_, (int) Lr_, Z,
+                       zr, zcp, (float *) g_apod_t, (float *) g_apod_r, (float *) g_cp);
   DREAM_HIP_CHECK(hipGetLastError());
 }
 

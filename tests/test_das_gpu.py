@@ -354,6 +354,40 @@ def test_pixel_adjoint_edges(gpu, oracle, method, No, L):
                     assert abs(float(gcp) - rcp) <= (1e-9 if prec == "f64" else 1e-3) * abs(rcp)
 
 
+@pytest.mark.parametrize("method,L,No", [("tfm", 3, 5), ("rca_coltx", 13, 1100),
+                                         ("rca_rowtx", 6, 1024), ("tfm", 70, 300)])
+def test_pair_adjoint_edges(gpu, oracle, method, L, No):
+    """The two-leg adjoint with the Y gradient at partial regions, receiver
+    groups and transmit groups and at more transmits than a part holds, on
+    scattered pixels (contributions past the windows) and a compact block,
+    one frame and three, both sampling rules, against the FP64 oracle (bars
+    of test_pixel_adjoint_edges)."""
+    from dream_amd.torch_ops import DasPlan
+    Y, Gt, Gr, Ro, rng = _setup(method, L=L, seed=15, No=No)
+    F = 3
+    Yf = np.stack([Y.T * (1 + f) for f in range(F)])
+    g = rng.standard_normal((F, No))
+    at, ar = rng.uniform(0.5, 1.5, L), rng.uniform(0.5, 1.5, L)
+    for pixels in (Ro, Ro * [0.1, 0.1, 0.3]):
+        for interp in ("nearest", "linear"):
+            ref = [oracle.das_ext_adjoint(Yf[f].T, Gt, Gr, pixels, 0.02, 0.1, 1500.0, g[f], method,
+                                          interp, at, ar, nthreads=8) for f in range(F)]
+            for prec, dt_, tol in (("f64", torch.float64, 1e-10), ("f32", torch.float32, 5e-5)):
+                plan = DasPlan(method, Y.shape[0], pixels, Gt, Gr, precision=prec)
+                for n in (1, F):
+                    t = [torch.tensor(v, dtype=dt_, device="cuda").contiguous()
+                         for v in (Yf[:n], g[:n], at, ar)]
+                    gY, gat, gar, gcp = plan.adjoint(t[0], t[1], 0.02, 0.1, 1500.0, t[2], t[3],
+                                                     interp)
+                    for f in range(n):
+                        assert rel_l2(gY[f].double().cpu().numpy().T, ref[f][0]) <= tol
+                    assert rel_l2(gat.double().cpu().numpy(), sum(r[1] for r in ref[:n])) <= tol
+                    assert rel_l2(gar.double().cpu().numpy(), sum(r[2] for r in ref[:n])) <= tol
+                    if interp == "linear":
+                        rcp = sum(r[3] for r in ref[:n])
+                        assert abs(float(gcp) - rcp) <= (1e-9 if prec == "f64" else 1e-3) * abs(rcp)
+
+
 def test_autograd_function(gpu, oracle):
     from dream_amd.torch_ops import DasPlan, das_diff
     method = "saft"
