@@ -3,6 +3,7 @@
 // Every entry point converts C++ exceptions into DREAM_HIP_E* codes and keeps
 // the message for dream_hip_last_error(); no C++ type crosses the boundary.
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstring>
@@ -82,6 +83,50 @@ hipStream_t lib_stream()
 {
   if (!g_stream) DREAM_HIP_CHECK(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking));
   return g_stream;
+}
+
+namespace {
+struct Scratch {
+  int device = -1;
+  void *p[SCRATCH_USES] = {};
+  size_t bytes[SCRATCH_USES] = {};
+  void drop(int k)
+  {
+    if (p[k]) (void) hipFree(p[k]);
+    p[k] = nullptr;
+    bytes[k] = 0;
+  }
+  void drop_all() { for (int k = 0; k < SCRATCH_USES; k++) drop(k); }
+  ~Scratch() { drop_all(); }
+};
+thread_local Scratch t_scratch;
+} // namespace
+
+void *scratch_get(ScratchUse use, size_t bytes)
+{
+  Scratch &t = t_scratch;
+  int dev = 0;
+  DREAM_HIP_CHECK(hipGetDevice(&dev));
+  if (t.device != dev) {
+    t.drop_all();
+    t.device = dev;
+  }
+  bytes = std::max<size_t>(bytes, 1);
+  if (t.bytes[use] >= bytes) return t.p[use];
+  t.drop(use);
+  const size_t want = (bytes + 65535) / 65536 * 65536;
+  if (hipMalloc(&t.p[use], want) != hipSuccess) {
+    (void) hipGetLastError();
+    t.p[use] = nullptr;
+    throw Error(DREAM_HIP_ENOMEM, "device allocation failed");
+  }
+  t.bytes[use] = want;
+  return t.p[use];
+}
+
+void scratch_done(ScratchUse use)
+{
+  if (t_scratch.bytes[use] > kScratchKeep) t_scratch.drop(use);
 }
 
 template <class F>
@@ -214,7 +259,7 @@ void run_single(const SirProblem &p, int out_dtype, hipStream_t s, int *sir_err,
                 int64_t *oob_count)
 {
   std::vector<SirProblem> probs{p};
-  SirPlan plan(probs, out_dtype);
+  SirPlan plan(probs, out_dtype, true, s);
   plan.run(s, false);
   int32_t code = 0;
   int64_t oob = 0;
@@ -294,7 +339,7 @@ int dream_hip_arr_rect_dev(const double *Ro, int64_t No, double a, double b, dou
     probs.push_back(make_problem(Ro, No, a, b, dx, dy, dt, nt, delay_type, delay, v, cp,
                                  num_elements, G, foc_met, focal, steer_met, theta, phi, apod,
                                  do_apod, apod_met, apod_par, h, err_level));
-    SirPlan plan(probs, out_dtype);
+    SirPlan plan(probs, out_dtype, true, s);
     plan.run(s, false);
     int32_t code = 0;
     int64_t oob = 0;
@@ -531,7 +576,7 @@ int dream_hip_sir_att_dev(const DreamSirProblem *problems, int32_t n, double alp
     if (alpha > 2.220446049250313e-16) {          // DBL_EPSILON
       run_sir_att(probs, alpha, out_dtype, s, sir_err, oob_count);
     } else {
-      SirPlan plan(probs, out_dtype);
+      SirPlan plan(probs, out_dtype, true, s);
       plan.run(s, false);
       plan.status(sir_err, oob_count);
     }

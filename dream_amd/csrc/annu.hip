@@ -137,13 +137,10 @@ void run_arr_annu(const AnnuProblem &a, int out_dtype, hipStream_t s, int *sir_e
   // Disc responses: one SIR problem per radius (disc 0 skipped when it has
   // no area, as the reference leaves it zero).
   const size_t slot = (size_t) a.No * (size_t) a.nt;
-  double *disc = nullptr;
-  if (hipMalloc(&disc, slot * (size_t) R * sizeof(double)) != hipSuccess)
-    throw Error(DREAM_HIP_ENOMEM, "dream_arr_annu: device allocation failed");
-  AnnuRing *d_tab = nullptr;
+  double *disc = (double *) scratch_get(SCRATCH_DISCS, slot * (size_t) R * sizeof(double) +
+                                                           sizeof(AnnuRing) * (size_t) rings);
+  AnnuRing *d_tab = (AnnuRing *) (disc + slot * (size_t) R);
   try {
-    if (hipMalloc(&d_tab, sizeof(AnnuRing) * (size_t) rings) != hipSuccess)
-      throw Error(DREAM_HIP_ENOMEM, "dream_arr_annu: device allocation failed");
     DREAM_HIP_CHECK(hipMemcpyAsync(d_tab, tab.data(), sizeof(AnnuRing) * (size_t) rings,
                                    hipMemcpyHostToDevice, s));
     const double G0[3] = {0.0, 0.0, 0.0};
@@ -170,7 +167,7 @@ void run_arr_annu(const AnnuProblem &a, int out_dtype, hipStream_t s, int *sir_e
       if (a.alpha > 2.220446049250313e-16) {
         run_sir_att(probs, a.alpha, DREAM_HIP_F64, s, codes.data(), oobs.data());
       } else {
-        SirPlan plan(probs, DREAM_HIP_F64);
+        SirPlan plan(probs, DREAM_HIP_F64, true, s);
         plan.run(s, false);
         plan.status(codes.data(), oobs.data());   // synchronises `s`
       }
@@ -198,12 +195,10 @@ void run_arr_annu(const AnnuProblem &a, int out_dtype, hipStream_t s, int *sir_e
     if (oob_count) *oob_count = oob;
   } catch (...) {
     (void) hipStreamSynchronize(s);
-    if (d_tab) (void) hipFree(d_tab);
-    (void) hipFree(disc);
+    scratch_done(SCRATCH_DISCS);
     throw;
   }
-  (void) hipFree(d_tab);
-  (void) hipFree(disc);
+  scratch_done(SCRATCH_DISCS);
 }
 
 } // namespace dream

@@ -612,11 +612,7 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
   }
   const size_t o_spec = take((size_t) spec_total * sizeof(double2));
   std::vector<char> host(copied);
-  char *base = nullptr;
-  if (hipMalloc(&base, bytes) != hipSuccess) {
-    (void) hipGetLastError();
-    throw Error(DREAM_HIP_ENOMEM, "SIR with attenuation: device allocation failed");
-  }
+  char *base = (char *) scratch_get(SCRATCH_ATT, bytes);
   try {
     Status *d_status = (Status *) (base + o_status);
     for (size_t k = 0; k < grids.size(); k++) {
@@ -674,10 +670,10 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
     }
   } catch (...) {
     (void) hipStreamSynchronize(s);
-    (void) hipFree(base);
+    scratch_done(SCRATCH_ATT);
     throw;
   }
-  (void) hipFree(base);
+  scratch_done(SCRATCH_ATT);
 }
 
 } // namespace dream

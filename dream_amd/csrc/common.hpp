@@ -89,6 +89,18 @@ private:
 // priority).
 hipStream_t lib_stream();
 
+// Device scratch that a thread keeps between calls, for calls that
+// synchronise their stream before they return: one buffer per use, grown on
+// demand, kept up to kScratchKeep bytes (larger ones are freed by
+// scratch_done), given back when the thread ends, when it moves to another
+// device, or when an allocation fails.  A thread has at most one call at a
+// time, so a use has one user.  hipFree of an 88 MB buffer took 250 us, four
+// small allocations with their copies and frees 40 us of an 87 us call.
+enum ScratchUse { SCRATCH_PLAN = 0, SCRATCH_DISCS, SCRATCH_ATT, SCRATCH_USES };
+constexpr size_t kScratchKeep = (size_t) 128 << 20;
+void *scratch_get(ScratchUse use, size_t bytes);
+void scratch_done(ScratchUse use);
+
 // ------------------------------------------------------------------ device
 
 #if defined(__HIP_DEVICE_COMPILE__) || defined(__HIPCC__)

@@ -679,8 +679,13 @@ void disc_rows(double R, double dx, double dy, std::vector<double> &ys, std::vec
     const double rxs = std::sqrt(R * R - y * y);
     const double xsmin = -rxs, xsmax = rxs;
     const double x = xsmin + dx / 2.0;
+    // The accumulated walk's count: by division, unless its rounding (half
+    // an ulp of R per step) could decide it.
     double n = 0.0;
-    for (double xs = x; xs <= xsmax; xs += dx) n += 1.0;
+    const double steps = (xsmax - x) / dx;
+    const double doubt = 0x1p-50 * (steps + 4.0) * (R / dx + 4.0);
+    if (steps >= 0.0 && std::fabs(steps - std::rint(steps)) > doubt) n = std::floor(steps) + 1.0;
+    else for (double xs = x; xs <= xsmax; xs += dx) n += 1.0;
     ys.push_back(y);
     x0.push_back(x);
     count.push_back(n);
@@ -711,19 +716,26 @@ double cylinder_rows(double b, double Rc, double dy, std::vector<double> &ys,
   return dphi;
 }
 
-double disc_row_step(double x0, double count, double dx)
+void disc_row_steps(double R, double dx, const std::vector<double> &x0,
+                    const std::vector<double> &count, std::vector<double> &step)
 {
   // Within one binade of |x| the accumulated walk advances by a constant
-  // step, dx rounded to the binade's spacing: the row's mean step is dx plus
+  // step, dx rounded to the binade's spacing: a row's mean step is dx plus
   // those deviations over the lengths the row spends in each binade.
-  if (count < 2.0) return dx;
-  const double half = std::fabs(x0);
-  double drift = 0.0;
-  for (double lo = std::ldexp(1.0, std::ilogb(half)); lo > 4.0 * dx; lo *= 0.5) {
-    const double x = 1.5 * lo;
-    drift += 2.0 * (std::min(half, 2.0 * lo) - lo) / dx * ((x + dx) - x - dx);
+  double lo[16], dev[16];
+  int n = 0;
+  for (double b = std::ldexp(1.0, std::ilogb(R)); b > 4.0 * dx && n < 16; b *= 0.5, n++) {
+    lo[n] = b;
+    dev[n] = 2.0 * ((1.5 * b + dx) - 1.5 * b - dx) / dx;
   }
-  return dx + drift / (count - 1.0);
+  step.clear();
+  for (size_t r = 0; r < x0.size(); r++) {
+    const double half = std::fabs(x0[r]);
+    double drift = 0.0;
+    for (int k = 0; k < n; k++)
+      if (half > lo[k]) drift += (std::min(half, 2.0 * lo[k]) - lo[k]) * dev[k];
+    step.push_back(count[r] < 2.0 ? dx : dx + drift / (count[r] - 1.0));
+  }
 }
 
 std::vector<double> subgrid(double w, double d)
@@ -870,23 +882,25 @@ int walk_override()
   return -1;
 }
 
-// The order in which a disc's rows are dealt to lanes: by length, so that
-// the lanes of a wave end together.
+// The order in which a disc's rows are dealt to lanes: from the longest in
+// the middle outwards, so that the lanes of a wave end together.
 void order_disc_rows(std::vector<double> &ys, std::vector<double> &x0, std::vector<double> &count)
 {
-  std::vector<int> order(ys.size());
-  std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-    return count[(size_t) a] > count[(size_t) b];
-  });
-  auto deal = [&](std::vector<double> &v) {
-    std::vector<double> w(v.size());
-    for (size_t k = 0; k < v.size(); k++) w[k] = v[(size_t) order[k]];
-    v.swap(w);
-  };
-  deal(ys);
-  deal(x0);
-  deal(count);
+  const int n = (int) ys.size();
+  std::vector<double> a, b, c;
+  a.reserve(ys.size());
+  b.reserve(ys.size());
+  c.reserve(ys.size());
+  int up = n / 2, down = n / 2 - 1;
+  while (up < n || down >= 0) {
+    const int r = down < 0 || (up < n && count[(size_t) up] >= count[(size_t) down]) ? up++ : down--;
+    a.push_back(ys[(size_t) r]);
+    b.push_back(x0[(size_t) r]);
+    c.push_back(count[(size_t) r]);
+  }
+  ys.swap(a);
+  x0.swap(b);
+  count.swap(c);
 }
 
 // Whether positions that stray by `dev` mm from equal spacing `step` may be
@@ -917,8 +931,9 @@ int64_t line_parts(int64_t lines, int64_t chunks, int64_t len, int64_t most, boo
   return best_n;
 }
 
-SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int target_items)
-  : out_dtype_(out_dtype)
+SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool one_shot,
+                 hipStream_t stream)
+  : out_dtype_(out_dtype), one_shot_(one_shot)
 {
   require(out_dtype == DREAM_HIP_F64 || out_dtype == DREAM_HIP_F32,
           "SIR output precision must be DREAM_HIP_F64 or DREAM_HIP_F32");
@@ -926,7 +941,7 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
   const size_t esz = sizeof(double);          // LDS histogram entries are FP64
   const size_t lds_cap = 64 * 1024;
   const int cus = device_cus();
-  if (target_items <= 0) target_items = 8 * cus;
+  const int target_items = 8 * cus;
 
   int64_t total_no = 0;
   for (auto &p : problems) total_no += p.No;
@@ -954,11 +969,8 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
       disc_rows(p.R, p.dx, p.dy, ys[i], rx0[i], rn[i]);
       order_disc_rows(ys[i], rx0[i], rn[i]);
       double sum = 0.0, mx = 0.0;
-      for (size_t r = 0; r < rn[i].size(); r++) {
-        sum += rn[i][r];
-        mx = std::max(mx, rn[i][r]);
-        rdx[i].push_back(disc_row_step(rx0[i][r], rn[i][r], p.dx));
-      }
+      for (double c : rn[i]) { sum += c; mx = std::max(mx, c); }
+      disc_row_steps(p.R, p.dx, rx0[i], rn[i], rdx[i]);
       for (size_t r = 0; r < rn[i].size(); r++) rdx[i].push_back(1.0 / rdx[i][r]);
       // An accumulated position is within half an ulp of R per step.
       runs = force != WALK_ROWS && force != WALK_COLUMNS && p.R > 0.0 &&
@@ -1078,11 +1090,22 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return cost[a] > cost[b]; });
 
-  DREAM_HIP_CHECK(hipMalloc(&d_tables_, std::max<size_t>(table_doubles, 1) * sizeof(double)));
-  DREAM_HIP_CHECK(hipMalloc(&d_status_, std::max<size_t>(P, 1) * sizeof(Status)));
-  DREAM_HIP_CHECK(hipMalloc(&d_probs_, std::max<size_t>(P, 1) * sizeof(SirDev)));
-  DREAM_HIP_CHECK(hipMalloc(&d_counter_, 2 * sizeof(unsigned long long)));
-  DREAM_HIP_CHECK(hipMemset(d_counter_, 0, 2 * sizeof(unsigned long long)));
+  // One buffer: descriptors | status blocks | counters | tables.
+  const size_t o_status = P * sizeof(SirDev), o_counter = o_status + P * sizeof(Status);
+  const size_t o_tables = o_counter + 2 * sizeof(unsigned long long);
+  const size_t bytes = o_tables + table_doubles * sizeof(double);
+  static_assert(sizeof(SirDev) % 8 == 0 && sizeof(Status) % 8 == 0, "plan buffer alignment");
+  char *base;
+  if (one_shot_) {
+    base = (char *) scratch_get(SCRATCH_PLAN, bytes);
+  } else {
+    DREAM_HIP_CHECK(hipMalloc(&d_base_, bytes));
+    base = (char *) d_base_;
+  }
+  d_probs_ = (SirDev *) base;
+  d_status_ = (Status *) (base + o_status);
+  d_counter_ = (unsigned long long *) (base + o_counter);
+  d_tables_ = (double *) (base + o_tables);
 
   std::vector<double> tables;
   tables.reserve(table_doubles);
@@ -1125,10 +1148,21 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
   }
   n_items_ = item;
   lds_bytes_ = max_nt_lds ? (size_t) (max_nt_lds + 1) * esz : 0;
+  // Status blocks and counters start zeroed.
+  image_.assign(bytes, 0);
+  if (P) std::memcpy(image_.data(), host_.data(), P * sizeof(SirDev));
   if (!tables.empty())
-    DREAM_HIP_CHECK(hipMemcpy(d_tables_, tables.data(), tables.size() * sizeof(double),
-                              hipMemcpyHostToDevice));
-  DREAM_HIP_CHECK(hipMemcpy(d_probs_, host_.data(), P * sizeof(SirDev), hipMemcpyHostToDevice));
+    std::memcpy(image_.data() + o_tables, tables.data(), tables.size() * sizeof(double));
+  if (one_shot_) {
+    last_stream_ = stream;
+    DREAM_HIP_CHECK(hipMemcpyAsync(base, image_.data(), bytes, hipMemcpyHostToDevice, stream));
+    pending_ = true;
+  } else {
+    const hipError_t e = hipMemcpy(base, image_.data(), bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) (void) hipFree(d_base_);
+    DREAM_HIP_CHECK(e);
+    std::vector<char>().swap(image_);
+  }
 
   // Persistent grid when the list is long and uneven; otherwise one
   // work-group per item.
@@ -1152,10 +1186,13 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int tar
 SirPlan::~SirPlan()
 {
   if (graph_) (void) hipGraphExecDestroy(graph_);
-  (void) hipFree(d_tables_);
-  (void) hipFree(d_status_);
-  (void) hipFree(d_probs_);
-  (void) hipFree(d_counter_);
+  // A call that failed may leave work on its stream, and the scratch is the
+  // next call's.
+  if (one_shot_) {
+    if (pending_) (void) hipStreamSynchronize(last_stream_);
+    scratch_done(SCRATCH_PLAN);
+  }
+  if (d_base_) (void) hipFree(d_base_);
 }
 
 void SirPlan::choose(hipStream_t s)
@@ -1185,7 +1222,9 @@ void SirPlan::launch_shape(const SirShape &sh, hipStream_t s, ChunkGate *gate)
   const size_t esz = out_dtype_ == DREAM_HIP_F64 ? 8 : 4;
   for (size_t i = 0; i < zero_len_.size(); i++)
     if (zero_len_[i]) zero.emplace_back(zero_ptr_[i], (size_t) zero_len_[i] * esz);
-  launch_fill_zero_list(zero, s);
+  // The upload left the status blocks zero for the first launch.
+  if (!fresh_ || zero.size() > 1) launch_fill_zero_list(zero, s);
+  fresh_ = false;
   if (n_items_ == 0) return;
   unsigned long long *ctr = sh.persistent ? d_counter_ : nullptr;
   bool any_global = false;
@@ -1259,6 +1298,7 @@ void SirPlan::run(hipStream_t s, bool use_graph)
     // captured); the graph is then launched on the caller's stream.
     hipStream_t cs = lib_stream();
     hipGraph_t g = nullptr;
+    fresh_ = false;                               // the graph's launch clears
     DREAM_HIP_CHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     launch(cs, nullptr);
     DREAM_HIP_CHECK(hipStreamEndCapture(cs, &g));
@@ -1272,8 +1312,13 @@ void SirPlan::status(int32_t *codes, int64_t *oob)
 {
   const size_t P = host_.size();
   std::vector<Status> st(P);
+  if (P && ran_)
+    DREAM_HIP_CHECK(hipMemcpyAsync(st.data(), d_status_, P * sizeof(Status), hipMemcpyDeviceToHost,
+                                   last_stream_));
+  else if (P)
+    DREAM_HIP_CHECK(hipMemcpy(st.data(), d_status_, P * sizeof(Status), hipMemcpyDeviceToHost));
   if (ran_) DREAM_HIP_CHECK(hipStreamSynchronize(last_stream_));
-  if (P) DREAM_HIP_CHECK(hipMemcpy(st.data(), d_status_, P * sizeof(Status), hipMemcpyDeviceToHost));
+  pending_ = false;
   for (size_t i = 0; i < P; i++) {
     const int lv = levels_[i];
     int code = E_NONE;

@@ -78,9 +78,10 @@ enum { SIR_RECT = 0, SIR_CIRC = 1, SIR_CYLIND = 2 };
 void disc_rows(double R, double dx, double dy, std::vector<double> &ys,
                std::vector<double> &x0, std::vector<double> &count);
 
-// Mean step of the accumulated x walk of a disc row that starts at x0 (< 0)
-// and ends near -x0, to a few 1e-14 of the disc's size.
-double disc_row_step(double x0, double count, double dx);
+// Mean step of each disc row's accumulated x walk (from x0 < 0 to near -x0),
+// to a few 1e-14 of the disc's size.
+void disc_row_steps(double R, double dx, const std::vector<double> &x0,
+                    const std::vector<double> &count, std::vector<double> &step);
 
 // Sub-element rows of a cylindrically curved element of y-size b and
 // curvature radius Rc (src/dreamcylind.cc:288-350): the rows are angles phi
@@ -103,7 +104,10 @@ std::vector<double> element_table(const SirProblem &p);
 // A prepared batch: device tables, work list, status blocks, launch shape.
 class SirPlan {
 public:
-  SirPlan(const std::vector<SirProblem> &problems, int out_dtype, int target_items = 0);
+  // one_shot: for one call that synchronises `stream` before it returns; the
+  // plan's buffer is the thread's kept scratch.
+  SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool one_shot = false,
+          hipStream_t stream = nullptr);
   ~SirPlan();
   void run(hipStream_t s, bool use_graph);
   // Per-problem SIRError code and OOB counts (synchronises on the last run's stream).
@@ -129,6 +133,11 @@ private:
   std::vector<int> levels_;
   std::vector<int64_t> zero_len_;  // per problem: elements to zero first (0 = none)
   std::vector<void *> zero_ptr_;
+  bool one_shot_ = false;
+  bool fresh_ = true;                       // status blocks zero, not launched yet
+  bool pending_ = false;                    // a one-shot plan's stream is not yet waited for
+  std::vector<char> image_;                 // the upload, kept while it may be read
+  void *d_base_ = nullptr;                  // the buffer, if the plan owns one
   SirDev *d_probs_ = nullptr;
   double *d_tables_ = nullptr;
   Status *d_status_ = nullptr;
