@@ -1422,13 +1422,14 @@ das_adj_pairs_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int 
       for (int jj = 0; jj < kGJ; jj++) {
         const int j = j0 + jj;
         if (j >= Lr) continue;                     // uniform
-        DT f[kRPU], y0[kRPU], y1[kRPU];
+        GT f[kRPU];
+        DT y0[kRPU], y1[kRPU];
         int k[kRPU];
 #pragma unroll
         for (int q = 0; q < kRPU; q++) {
-          unsigned o0, o1;
-          gather_index<DT, GT, INTERP, true>((tt[q] + tr[jj][q]) * fs, true, o0, o1, f[q], k[q]);
-          if (!live[q]) k[q] = -2;                 // neither tap exists
+          const GT u = (tt[q] + tr[jj][q]) * fs, fk = INTERP == DREAM_HIP_NEAREST ? u : floor(u);
+          k[q] = live[q] ? (int) fk : -2;          // -2: neither tap exists
+          f[q] = u - fk;
         }
         const unsigned a = (unsigned) (TYPE == DAS_RCA_ROWTX ? j * Lt + i : i * Lr + j);
 #pragma unroll
@@ -1437,34 +1438,35 @@ das_adj_pairs_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int 
           if (INTERP != DREAM_HIP_NEAREST) y1[q] = sload<DT>(ry, (unsigned) (k[q] + 1), a * KB);
         }
         const int s = ii * kGJ + jj;
-        const DT wj = APOD ? ar[j] : DT(1), w = wi * wj;
+        const DT wj = APOD ? ar[j] : DT(1);
+        const double wd = (double) wi * (double) wj;
         const int ws = w0[s];
         DT *ga = gy_frame + (int64_t) a * K;
         DT z = DT(0), zc = DT(0);                  // over the lane's pixels
 #pragma unroll
         for (int q = 0; q < kRPU; q++) {
           DT val = y0[q];
-          const DT gw = gp[q] * w;
+          const double gw = (double) gp[q] * wd;
           const int kk = k[q];
           const unsigned l = (unsigned) (kk - ws);
           if (INTERP == DREAM_HIP_NEAREST) {
             if ((unsigned) kk < (unsigned) K) {
-              if (l < (unsigned) kWin) lds_atomic_add(&win[s * kWin + l], (double) gw);
-              else unsafeAtomicAdd(&ga[kk], gw);
+              if (l < (unsigned) kWin) lds_atomic_add(&win[s * kWin + l], gw);
+              else unsafeAtomicAdd(&ga[kk], (DT) gw);
             }
           } else {
             const DT slope = y1[q] - y0[q];
-            val += f[q] * slope;
+            val += (DT) f[q] * slope;
             zc += (gp[q] * slope) * (DT) (tt0[q] + tr[jj][q]);
             // One of the taps in [0, K); a window's entries outside it are dropped.
             if ((unsigned) (kk + 1) <= (unsigned) K) {
-              const DT v0 = gw * (DT(1) - f[q]), v1 = gw * f[q];
+              const double v1 = gw * (double) f[q], v0 = gw - v1;
               if (l + 1u < (unsigned) kWin) {
-                lds_atomic_add(&win[s * kWin + l], (double) v0);
-                lds_atomic_add(&win[s * kWin + l + 1], (double) v1);
+                lds_atomic_add(&win[s * kWin + l], v0);
+                lds_atomic_add(&win[s * kWin + l + 1], v1);
               } else {
-                if (kk >= 0 && kk < K) unsafeAtomicAdd(&ga[kk], v0);
-                if (kk + 1 < K) unsafeAtomicAdd(&ga[kk + 1], v1);
+                if (kk >= 0 && kk < K) unsafeAtomicAdd(&ga[kk], (DT) v0);
+                if (kk + 1 < K) unsafeAtomicAdd(&ga[kk + 1], (DT) v1);
               }
             }
           }
@@ -1472,7 +1474,7 @@ das_adj_pairs_kernel(DasArgs A, const int32_t *__restrict__ perm, int n_gj, int 
         }
         zi = __builtin_fma((double) wj, (double) z, zi);
         zr[jj] = __builtin_fma((double) wi, (double) z, zr[jj]);
-        if (INTERP == DREAM_HIP_LINEAR) zcp = __builtin_fma((double) w, (double) zc, zcp);
+        if (INTERP == DREAM_HIP_LINEAR) zcp = __builtin_fma(wd, (double) zc, zcp);
       }
       const double total = wave_total(zi);
       if (lane == 63 && total != 0.0) lds_atomic_add(&s_zt[i - g0 * kGI], total);

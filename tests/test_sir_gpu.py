@@ -360,3 +360,49 @@ def test_run_walk(gpu, oracle, monkeypatch, shape, walk, size, step, dt, nt, nea
     assert np.max(np.abs(H.cpu().numpy().T - ref)) <= 1e-12 * max(np.abs(ref).max(), 1e-300)
     H32, _, n32 = fn(*args, out_dtype=torch.float32, **kw)
     assert n32 == oob and rel_l2(H32.double().cpu().numpy().T, ref) <= 2e-5
+
+
+def test_calls_of_threads_and_streams_keep_apart(gpu, oracle):
+    """One-call plans use scratch kept by the calling thread: threads on their
+    own streams, each with small and large calls in turn (the scratch grows,
+    then serves the smaller) and annular calls between them, equal the same
+    calls made alone up to the order of their sums; a call that is refused
+    leaves the next one whole."""
+    import threading
+    from dream_amd import torch_ops
+    G = np.c_[np.linspace(-2, 2, 5), np.zeros(5), np.zeros(5)]
+
+    def rect(No, nt, seed):
+        rng = np.random.default_rng(seed)
+        Ro = np.c_[rng.uniform(-4, 4, No), np.zeros(No), rng.uniform(8, 30, No)]
+        d = torch.tensor(Ro[:, 2] / 1.5 - 0.5, device="cuda")
+        return torch_ops.arr_rect(torch.tensor(Ro.T.copy(), device="cuda"), 0.4, 4.0, 0.05, 0.05,
+                                  0.02, nt, d, 1.0, 1500.0, G, err_level="ignore")[0]
+
+    def annu(seed):
+        rng = np.random.default_rng(seed)
+        Ro = np.c_[rng.uniform(-3, 3, 20), np.zeros(20), rng.uniform(8, 20, 20)]
+        return torch_ops.arr_annu(torch.tensor(Ro.T.copy(), device="cuda"), [1.0, 1.1, 2.0], 0.05,
+                                  0.05, 0.05, 500, 0.0, 1.0, 1000.0, err_level="ignore")[0]
+
+    jobs = [(rect, (2100, 300, 1)), (annu, (2,)), (rect, (3000, 900, 3)), (rect, (2500, 200, 4)), (annu, (5,))]
+    want = [f(*a).cpu() for f, a in jobs]
+    with pytest.raises(RuntimeError):
+        torch_ops.arr_rect(torch.zeros((3, 1), device="cuda", dtype=torch.float64), 0.4, 4.0, 0.05,
+                           0.05, -0.02, 10, 0.0, 1.0, 1500.0, G)
+    got = {}
+
+    def work(t):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            got[t] = [[f(*a).cpu() for f, a in jobs] for _ in range(3)]
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == 3
+    for rounds in got.values():
+        for r in rounds:
+            for a, b in zip(r, want):
+                assert torch.allclose(a, b, rtol=0.0, atol=1e-13 * float(b.abs().max()))
