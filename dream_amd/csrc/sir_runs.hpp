@@ -9,10 +9,11 @@
 // length and x the offset from it,
 //   1/r(c + x) = 1/r_c sum_j (-x/r_c)^j P_j(v_c/r_c)     (Legendre),
 // whose odd terms cancel over the run and whose even ones need only the
-// moments of 0 .. n-1.  Runs are cut at n dv <= r/30 (r/20 for an FP32
-// output), where the terms to P6 (P4) leave at most 7e-16 |P8| (2e-10) of
-// the sum, r/30 being a compromise: at r/41 (6e-17) the annular benchmark has
-// a quarter more runs.
+// moments of 0 .. n-1.  Runs are cut at n dv <= r/36 (r/20 for an FP32
+// output), where the terms to P6 (P4) leave at most 2e-16 |P8| (2e-10) of
+// the sum, below the rounding of the sums themselves; at r/30 (7e-16) some
+// drawn workloads were 5 % further from their 64-bit values, at r/41 the
+// annular one takes 6 % longer.
 //
 // A bin edge that falls so close to a sub-element that the estimate could
 // round differently from the exact index sequence ends the walk there: the
@@ -77,7 +78,7 @@ DREAM_RUNS_FN bool runs_ready(RunLine &l, int n)
   l.foot = f > 0.0 ? (f < (double) n ? (int) f : n) : 0;
   l.roff = (l.c2 + 0.5) * l.ic1;
   l.tol = 2.2 * l.bound * l.ic1 * l.inv_dv * r;
-  const double m = l.w * runs_rsq(l.w) * l.inv_dv * (REFINE ? 1.0 / 30.0 : 1.0 / 20.0);
+  const double m = l.w * runs_rsq(l.w) * l.inv_dv * (REFINE ? 1.0 / 36.0 : 1.0 / 20.0);
   l.cap = m > 1.0 ? (int) (m < 1e6 ? m : 1e6) : 1;
   return l.dv > 0.0 && l.c1 * l.dv <= 4.0 && l.w >= 64.0 * (l.dv * l.dv) &&
          l.w >= 4.0 * (l.ic1 * l.ic1) && l.w < 1e200 &&
