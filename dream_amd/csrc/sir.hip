@@ -1222,8 +1222,9 @@ void SirPlan::launch_shape(const SirShape &sh, hipStream_t s, ChunkGate *gate)
   const size_t esz = out_dtype_ == DREAM_HIP_F64 ? 8 : 4;
   for (size_t i = 0; i < zero_len_.size(); i++)
     if (zero_len_[i]) zero.emplace_back(zero_ptr_[i], (size_t) zero_len_[i] * esz);
-  // The upload left the status blocks zero for the first launch.
-  if (!fresh_ || zero.size() > 1) launch_fill_zero_list(zero, s);
+  // The upload left the status blocks zero for a one-shot plan's first launch
+  // (a kept plan's may be captured and replayed).
+  if (!one_shot_ || !fresh_ || zero.size() > 1) launch_fill_zero_list(zero, s);
   fresh_ = false;
   if (n_items_ == 0) return;
   unsigned long long *ctr = sh.persistent ? d_counter_ : nullptr;
@@ -1298,7 +1299,6 @@ void SirPlan::run(hipStream_t s, bool use_graph)
     // captured); the graph is then launched on the caller's stream.
     hipStream_t cs = lib_stream();
     hipGraph_t g = nullptr;
-    fresh_ = false;                               // the graph's launch clears
     DREAM_HIP_CHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     launch(cs, nullptr);
     DREAM_HIP_CHECK(hipStreamEndCapture(cs, &g));
@@ -1312,12 +1312,15 @@ void SirPlan::status(int32_t *codes, int64_t *oob)
 {
   const size_t P = host_.size();
   std::vector<Status> st(P);
-  if (P && ran_)
+  if (one_shot_ && P) {
     DREAM_HIP_CHECK(hipMemcpyAsync(st.data(), d_status_, P * sizeof(Status), hipMemcpyDeviceToHost,
                                    last_stream_));
-  else if (P)
-    DREAM_HIP_CHECK(hipMemcpy(st.data(), d_status_, P * sizeof(Status), hipMemcpyDeviceToHost));
-  if (ran_) DREAM_HIP_CHECK(hipStreamSynchronize(last_stream_));
+    DREAM_HIP_CHECK(hipStreamSynchronize(last_stream_));
+  } else {
+    if (ran_) DREAM_HIP_CHECK(hipStreamSynchronize(last_stream_));
+    if (P)
+      DREAM_HIP_CHECK(hipMemcpy(st.data(), d_status_, P * sizeof(Status), hipMemcpyDeviceToHost));
+  }
   pending_ = false;
   for (size_t i = 0; i < P; i++) {
     const int lv = levels_[i];

@@ -134,7 +134,7 @@ private:
   std::vector<int64_t> zero_len_;  // per problem: elements to zero first (0 = none)
   std::vector<void *> zero_ptr_;
   bool one_shot_ = false;
-  bool fresh_ = true;                       // status blocks zero, not launched yet
+  bool fresh_ = true;                       // not launched yet
   bool pending_ = false;                    // a one-shot plan's stream is not yet waited for
   std::vector<char> image_;                 // the upload, kept while it may be read
   void *d_base_ = nullptr;                  // the buffer, if the plan owns one

@@ -406,3 +406,33 @@ def test_calls_of_threads_and_streams_keep_apart(gpu, oracle):
         for r in rounds:
             for a, b in zip(r, want):
                 assert torch.allclose(a, b, rtol=0.0, atol=1e-13 * float(b.abs().max()))
+
+
+def test_batch_captured_at_its_first_run(gpu):
+    """A batch whose first run is captured by the caller clears its status on
+    every replay: outputs and counts of each equal an eager run's."""
+    from dream_amd.torch_ops import SirBatch
+    rng = np.random.default_rng(8)
+    probs = []
+    for L, No in ((3, 40), (6, 25)):
+        Ro = np.c_[rng.uniform(-3, 3, No), np.zeros(No), rng.uniform(6, 12, No)]
+        probs.append(dict(Ro=torch.tensor(Ro.T.copy(), device="cuda"), a=0.5, b=3.0, dx=0.05,
+                          dy=0.05, dt=0.02, nt=120, v=1.0, cp=1500.0, err_level="ignore",
+                          delay=torch.tensor(Ro[:, 2] / 1.5 + 0.1, device="cuda"),
+                          G=np.c_[np.linspace(-2, 2, L), np.zeros(L), np.zeros(L)]))
+    eager = SirBatch(probs, out_dtype=torch.float64)
+    want = [h.clone() for h in eager.run(use_graph=False)]
+    codes, oob = eager.status()
+    assert sum(oob) > 0
+    batch = SirBatch(probs, out_dtype=torch.float64)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = batch.run(use_graph=False)
+    for _ in range(3):
+        for h in out:
+            h.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for h, w in zip(out, want):
+            assert torch.allclose(h, w, rtol=0.0, atol=1e-13 * float(w.abs().max()))
+        assert list(batch.status()[1]) == list(oob)
