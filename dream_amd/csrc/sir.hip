@@ -369,7 +369,7 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
         const int k1 = part + 1 == P.nseg ? cnt : (int) (len * (double) (part + 1));
         if (walk == WALK_RUNS && k < k1) {
           RunLine line{xe - x0, ((gdouble *) P.row_dx)[line_row], ((gdouble *) P.row_idx)[line_row],
-                       ryz, P.c1, P.ic1, c2, 0.5 - lim};
+                       ryz, P.c1, P.ic1, c2, 0.5 - lim, P.line_dev};
           if (runs_ready<REFINE_H>(line, cnt)) {
             walk_line(line, k, k1, el[5 * L + e] * P.amp, [&](int i) {
               double x = x0, h;
@@ -456,7 +456,8 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
       int j0 = sg * P.seg_len;
       const int j1 = min(j0 + P.seg_len, ny);
       if (walk == WALK_RUNS) {
-        RunLine line{ye - P.line_p0, P.line_dv, P.line_inv_dv, rxz, P.c1, P.ic1, c2, 0.5 - lim};
+        RunLine line{ye - P.line_p0, P.line_dv, P.line_inv_dv, rxz, P.c1, P.ic1, c2, 0.5 - lim,
+                     P.line_dev};
         if (runs_ready<REFINE_H>(line, ny)) {
           walk_line(line, j0, j1, el[5 * L + e] * P.amp, [&](int k) {
             const double ry = ye - ys[k];
@@ -716,28 +717,6 @@ double cylinder_rows(double b, double Rc, double dy, std::vector<double> &ys,
   return dphi;
 }
 
-void disc_row_steps(double R, double dx, const std::vector<double> &x0,
-                    const std::vector<double> &count, std::vector<double> &step)
-{
-  // Within one binade of |x| the accumulated walk advances by a constant
-  // step, dx rounded to the binade's spacing: a row's mean step is dx plus
-  // those deviations over the lengths the row spends in each binade.
-  double lo[16], dev[16];
-  int n = 0;
-  for (double b = std::ldexp(1.0, std::ilogb(R)); b > 4.0 * dx && n < 16; b *= 0.5, n++) {
-    lo[n] = b;
-    dev[n] = 2.0 * ((1.5 * b + dx) - 1.5 * b - dx) / dx;
-  }
-  step.clear();
-  for (size_t r = 0; r < x0.size(); r++) {
-    const double half = std::fabs(x0[r]);
-    double drift = 0.0;
-    for (int k = 0; k < n; k++)
-      if (half > lo[k]) drift += (std::min(half, 2.0 * lo[k]) - lo[k]) * dev[k];
-    step.push_back(count[r] < 2.0 ? dx : dx + drift / (count[r] - 1.0));
-  }
-}
-
 std::vector<double> subgrid(double w, double d)
 {
   std::vector<double> v;
@@ -965,12 +944,13 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
     const int force = walk_override();
     int64_t nx_cost, disc_parts = 1;
     bool runs = false;
+    double dev_mm = 0.0;
     if (p.shape == SIR_CIRC) {
       disc_rows(p.R, p.dx, p.dy, ys[i], rx0[i], rn[i]);
       order_disc_rows(ys[i], rx0[i], rn[i]);
       double sum = 0.0, mx = 0.0;
       for (double c : rn[i]) { sum += c; mx = std::max(mx, c); }
-      disc_row_steps(p.R, p.dx, rx0[i], rn[i], rdx[i]);
+      dev_mm = disc_row_steps(p.R, p.dx, rx0[i], rn[i], rdx[i]);
       for (size_t r = 0; r < rn[i].size(); r++) rdx[i].push_back(1.0 / rdx[i][r]);
       // An accumulated position is within half an ulp of R per step.
       runs = force != WALK_ROWS && force != WALK_COLUMNS && p.R > 0.0 &&
@@ -1038,20 +1018,17 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
       d.nseg = (int32_t) disc_parts;
       d.part_len = 1.0 / (double) disc_parts;
       d.runs = runs;
+      d.line_dev = dev_mm;
       d.walk = !runs ? WALK_ROWS : force;
       d.wx = d.wy = (float) (4.0 / (3.0 * M_PI) * p.R);   // mean |x| over the disc
       d.sx = (float) (p.dx / lam);
       d.sy = (float) (p.dy / lam);
     }
     if (p.shape == SIR_RECT && nx > 0 && ny > 0 && force != WALK_ROWS) {
-      const std::vector<double> &y = ys[i];
-      d.line_p0 = y[0];
-      d.line_dv = ny > 1 ? (y[(size_t) ny - 1] - y[0]) / (double) (ny - 1) : p.dy;
+      d.line_p0 = ys[i][0];
+      line_fit(ys[i], p.dy, d.line_dv, d.line_dev);
       d.line_inv_dv = 1.0 / d.line_dv;
-      double dev = 0.0;
-      for (int64_t k = 0; k < ny; k++)
-        dev = std::max(dev, std::fabs(y[(size_t) k] - (y[0] + (double) k * d.line_dv)));
-      d.runs = force != WALK_COLUMNS && runs_hold(dev, d.line_dv, c1, p.nt);
+      d.runs = force != WALK_COLUMNS && runs_hold(d.line_dev, d.line_dv, c1, p.nt);
       d.walk = force == WALK_RUNS && !d.runs ? WALK_COLUMNS : force;
       const int64_t QC = L * nx;
       const int64_t n = line_parts(QC, d.chunks, ny, ny / 8, d.runs, p.dy / lam);

@@ -60,8 +60,9 @@ struct SirDev {
   // picks its cheapest, runs among them if `runs` is set.
   int32_t walk, runs;
   // The lines of the run walk over a rectangle's columns: positions
-  // line_p0 + k line_dv.
-  double line_p0, line_dv, line_inv_dv;
+  // line_p0 + k line_dv, and their largest deviation from it (a disc's rows':
+  // from their mean steps).
+  double line_p0, line_dv, line_inv_dv, line_dev;
   // The walk choice: mean |xs| and |ys|, dx and dy in samples of path
   // (dx / (cp dt/1000), dy / (cp dt/1000)), lane rounds per item of the row
   // and the column walk.
@@ -77,11 +78,6 @@ enum { SIR_RECT = 0, SIR_CIRC = 1, SIR_CYLIND = 2 };
 // the count of each row.
 void disc_rows(double R, double dx, double dy, std::vector<double> &ys,
                std::vector<double> &x0, std::vector<double> &count);
-
-// Mean step of each disc row's accumulated x walk (from x0 < 0 to near -x0),
-// to a few 1e-14 of the disc's size.
-void disc_row_steps(double R, double dx, const std::vector<double> &x0,
-                    const std::vector<double> &count, std::vector<double> &step);
 
 // Sub-element rows of a cylindrically curved element of y-size b and
 // curvature radius Rc (src/dreamcylind.cc:288-350): the rows are angles phi

@@ -26,7 +26,9 @@
 // is at least B (r_k + R <= 2.2 R as w >= (8 dv)^2), k* the crossing.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
+#include <vector>
 
 #if defined(__HIP_DEVICE_COMPILE__)
 #define DREAM_RUNS_FN __device__ __forceinline__
@@ -59,6 +61,7 @@ DREAM_RUNS_FN double runs_sqrt(double s)
 // what runs_ready derives from them.
 struct RunLine {
   double v0, dv, inv_dv, w, c1, ic1, c2, bound;
+  double dev = 0.0;   // the positions' largest deviation from v0 - k dv
   double roff;    // the upper edge of bin b is b ic1 + roff
   double tol;     // step j is certified when |j - j*| vb >= tol
   int foot;       // first sub-element past the foot, within [0, n]
@@ -66,8 +69,8 @@ struct RunLine {
 };
 
 // Whether walk_half holds on this line (n sub-elements): positive spacing,
-// at most four bins per step, w clear of both the spacing and the bin width,
-// and bins that fit an int.  False for NaN.
+// at most four bins per step, w clear of the spacing, the bin width and (FP64
+// output) the deviation, and bins that fit an int.  False for NaN.
 template <bool REFINE>
 DREAM_RUNS_FN bool runs_ready(RunLine &l, int n)
 {
@@ -80,7 +83,8 @@ DREAM_RUNS_FN bool runs_ready(RunLine &l, int n)
   l.tol = 2.2 * l.bound * l.ic1 * l.inv_dv * r;
   const double m = l.w * runs_rsq(l.w) * l.inv_dv * (REFINE ? 1.0 / 36.0 : 1.0 / 20.0);
   l.cap = m > 1.0 ? (int) (m < 1e6 ? m : 1e6) : 1;
-  return l.dv > 0.0 && l.c1 * l.dv <= 4.0 && l.w >= 64.0 * (l.dv * l.dv) &&
+  const double near = REFINE ? 0x1p46 * l.dev : 0.0;
+  return l.dv > 0.0 && l.c1 * l.dv <= 4.0 && l.w >= 64.0 * (l.dv * l.dv) && l.w >= near * near &&
          l.w >= 4.0 * (l.ic1 * l.ic1) && l.w < 1e200 &&
          l.c1 * r + __builtin_fabs(l.c2) < 0x1p30 && r * l.inv_dv < 0x1p30;
 }
@@ -153,6 +157,55 @@ DREAM_RUNS_FN int walk_half(const RunLine &l, int half, int first, int len, Emit
     j = jn;
   } while (sure && j < len);
   return j;
+}
+
+// ------------------------------------------------------------------ host
+
+// The fit of positions y (rising by about d): y[0] + k dv, and the largest
+// deviation from it.
+inline void line_fit(const std::vector<double> &y, double d, double &dv, double &dev)
+{
+  const size_t n = y.size();
+  dv = n > 1 ? (y[n - 1] - y[0]) / (double) (n - 1) : d;
+  dev = 0.0;
+  for (size_t k = 0; k < n; k++) dev = std::max(dev, std::fabs(y[k] - (y[0] + (double) k * dv)));
+}
+
+// Mean step of each disc row's accumulated x walk (from x0 < 0 to near -x0),
+// to a few 1e-14 of the disc's size; returns the rows' largest deviation from
+// their mean steps.
+inline double disc_row_steps(double R, double dx, const std::vector<double> &x0,
+                             const std::vector<double> &count, std::vector<double> &step)
+{
+  // Within one binade of |x| the accumulated walk advances by a constant
+  // step, dx rounded to the binade's spacing: a row's mean step is dx plus
+  // those deviations over the lengths the row spends in each binade.
+  double lo[16], dev[16];
+  int n = 0;
+  for (double b = std::ldexp(1.0, std::ilogb(R)); b > 4.0 * dx && n < 16; b *= 0.5, n++) {
+    lo[n] = b;
+    dev[n] = 2.0 * ((1.5 * b + dx) - 1.5 * b - dx) / dx;
+  }
+  step.clear();
+  double worst = 0.0;
+  for (size_t r = 0; r < x0.size(); r++) {
+    const double half = std::fabs(x0[r]);
+    double drift = 0.0;
+    for (int k = 0; k < n; k++)
+      if (half > lo[k]) drift += (std::min(half, 2.0 * lo[k]) - lo[k]) * dev[k];
+    step.push_back(count[r] < 2.0 ? dx : dx + drift / (count[r] - 1.0));
+    // The walk strays from the mean step most where it leaves a binade, on
+    // either side of the middle alike.
+    double at = 0.0;
+    for (int k = 0; k < n; k++)
+      if (half > lo[k]) {
+        at += 0.5 * (std::min(half, 2.0 * lo[k]) - lo[k]) * dev[k];
+        worst = std::max(worst, std::fabs(at - 0.5 * drift * (half - lo[k]) / half));
+      }
+  }
+  // The roundings of the steps that cross binades, of the ends and of the
+  // mean step itself.
+  return R > 0.0 ? worst + std::ldexp(1.0, std::ilogb(R) - 50) : 0.0;
 }
 
 } // namespace dream

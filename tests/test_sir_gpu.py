@@ -436,3 +436,31 @@ def test_batch_captured_at_its_first_run(gpu):
         for h, w in zip(out, want):
             assert torch.allclose(h, w, rtol=0.0, atol=1e-13 * float(w.abs().max()))
         assert list(batch.status()[1]) == list(oob)
+
+
+@pytest.mark.parametrize("shape,size,step", [("rect", 200.0, 0.01), ("circ", 50.0, 0.02)])
+def test_long_lines_sum_as_steps(gpu, monkeypatch, shape, size, step):
+    """Apertures whose accumulated positions stray from equal spacing by more
+    than FP64 amplitudes bear: the run walk's responses equal the stepped
+    walk's to both walks' 2^-47 per sub-element and their sums' rounding,
+    half an ulp for each of a bin's sub-elements (runs on these lines without
+    a bound on the deviation: 3e-13)."""
+    from dream_amd.torch_ops import arr_circ, arr_rect
+    z = np.array([20.0, 23.0, 31.0])
+    Ro = torch.tensor(np.c_[[0.0, 30.0, -45.0], [10.0, 60.0, 45.0], z].T.copy(), device="cuda")
+    if shape == "rect":
+        args, fn = (Ro, 2 * step, size, step, step), arr_rect
+    else:
+        args, fn = (Ro, size, step, 2.0), arr_circ
+    rest = (0.02, 7000, torch.tensor(z / 1.5, device="cuda"), 1.0, 1500.0, np.zeros((1, 3)))
+    out = {}
+    for walk in ("rows", "runs"):
+        monkeypatch.setenv("DREAM_HIP_SIR_WALK", walk)
+        H, _, oob = fn(*args, *rest, err_level="ignore")
+        out[walk] = (H.cpu().numpy(), oob)
+    (a, na), (b, nb) = out["rows"], out["runs"]
+    assert na == nb
+    # A bin of m sub-elements at up to 170 mm holds at least m amp/170.
+    amp = 1000.0 / (2 * np.pi * 0.02) * step * (step if shape == "rect" else 2.0)
+    m = a * 170.0 / amp + 1.0
+    assert np.all(np.abs(a - b) <= a * (2.0 ** -46 + m * 2.0 ** -53))
