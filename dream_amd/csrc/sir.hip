@@ -310,21 +310,12 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
     if (lane == __ffsll((long long) act) - 1) oob_s += cnt_w;
     return ((out_mask >> lane) & 1ull) != 0;
   };
-  // Sub-elements [k0, k1) of a usable line, run by run; step(k) adds one
-  // that no run certifies.  Runs outside [0, nt) add to the spare bin.
-  auto walk_line = [&](const RunLine &line, int k0, int k1, double amp, auto step) {
-#pragma clang loop unroll(disable)
-    for (int half = 0; half < 2; half++) {
-      int len;
-      const int first = half_of(line, half, k0, k1, len);
-      int m = walk_half<REFINE_H>(line, half, first, len, [&](int b, int n, double v) {
-        const bool in = (unsigned) b < (unsigned) nt;
-        if (use_lds) lds_add(hist + min((unsigned) b, (unsigned) nt), amp * v);
-        else if (in) global_add(out + b, (T) (amp * v));
-        oob += in ? 0 : n;
-      });
-      for (; m < len; m++) step(half ? first - m : first + m);
-    }
+  // A run of a usable line; outside [0, nt) it adds to the spare bin.
+  auto add_run = [&](double amp, int b, int n, double v) {
+    const bool in = (unsigned) b < (unsigned) nt;
+    if (use_lds) lds_add(hist + min((unsigned) b, (unsigned) nt), amp * v);
+    else if (in) global_add(out + b, (T) (amp * v));
+    oob += in ? 0 : n;
   };
   if (!columns) {
     const int Q = L * ny;
@@ -367,30 +358,29 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
         const double len = (double) cnt * P.part_len;
         int k = (int) (len * (double) part);
         const int k1 = part + 1 == P.nseg ? cnt : (int) (len * (double) (part + 1));
+        // Sub-elements [lo, hi) by the accumulated walk.
+        auto steps = [&](int lo, int hi) {
+          double x = x0;
+          for (int m = 0; m < lo; m++) x += P.dx;
+          for (; lo < hi; lo++) {
+            double h;
+            const double ru = sir_index<REFINE_H>(xe - x, ryy, rzz, ryz, c1h, c2, lim, P.cp, d,
+                                                  P.dt, h);
+            accumulate(sat_i32(ru), h);
+            x += P.dx;
+          }
+        };
         if (walk == WALK_RUNS && k < k1) {
           RunLine line{xe - x0, ((gdouble *) P.row_dx)[line_row], ((gdouble *) P.row_idx)[line_row],
                        ryz, P.c1, P.ic1, c2, 0.5 - lim, P.line_dev};
           if (runs_ready<REFINE_H>(line, cnt)) {
-            walk_line(line, k, k1, el[5 * L + e] * P.amp, [&](int i) {
-              double x = x0, h;
-              for (int m = 0; m < i; m++) x += P.dx;
-              const double ru = sir_index<REFINE_H>(xe - x, ryy, rzz, ryz, c1h, c2, lim, P.cp, d,
-                                                    P.dt, h);
-              accumulate(sat_i32(ru), h);
-            });
+            const double amp = el[5 * L + e] * P.amp;
+            walk_line<REFINE_H>(line, k, k1, [&](int b, int n, double v) { add_run(amp, b, n, v); },
+                                steps);
             k = k1;
           }
         }
-        double x = x0;
-        if (k < k1)
-          for (int m = 0; m < k; m++) x += P.dx;
-        for (; k < k1; k++) {
-          double h;
-          const double ru = sir_index<REFINE_H>(xe - x, ryy, rzz, ryz, c1h, c2, lim, P.cp, d,
-                                                P.dt, h);
-          accumulate(sat_i32(ru), h);
-          x += P.dx;
-        }
+        if (k < k1) steps(k, k1);
       } else {
         int i = 0;
         for (; i + kBlock <= nx; i += kBlock) {
@@ -459,13 +449,17 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
         RunLine line{ye - P.line_p0, P.line_dv, P.line_inv_dv, rxz, P.c1, P.ic1, c2, 0.5 - lim,
                      P.line_dev};
         if (runs_ready<REFINE_H>(line, ny)) {
-          walk_line(line, j0, j1, el[5 * L + e] * P.amp, [&](int k) {
-            const double ry = ye - ys[k];
-            double r, h;
-            if (!sir_fast<REFINE_H>(ry, rxz, c1h, c2, lim, r, h))
-              sir_exact<REFINE_H>(rx, ry * ry, rzz, P.cp, d, P.dt, r, h);
-            accumulate(sat_i32(r), h);
-          });
+          const double amp = el[5 * L + e] * P.amp;
+          walk_line<REFINE_H>(line, j0, j1, [&](int b, int n, double v) { add_run(amp, b, n, v); },
+                              [&](int lo, int hi) {
+                                for (; lo < hi; lo++) {
+                                  const double ry = ye - ys[lo];
+                                  double r, h;
+                                  if (!sir_fast<REFINE_H>(ry, rxz, c1h, c2, lim, r, h))
+                                    sir_exact<REFINE_H>(rx, ry * ry, rzz, P.cp, d, P.dt, r, h);
+                                  accumulate(sat_i32(r), h);
+                                }
+                              });
           j0 = j1;
         }
       }

@@ -16,8 +16,8 @@
 // annular one takes 6 % longer.
 //
 // A bin edge that falls so close to a sub-element that the estimate could
-// round differently from the exact index sequence ends the walk there: the
-// caller steps the rest of the half by exact indices (about one line in 10^4;
+// round differently from the exact index sequence ends the walk there:
+// walk_line has the rest of the half stepped by exact indices (about one line in 10^4;
 // keeping the exact sequence out of the loop keeps its registers out).  With
 // B the certification bound in samples, u = c1 r - c2 the index before
 // rounding, T the edge and vb > 0 the offset there, sub-element k is
@@ -157,6 +157,22 @@ DREAM_RUNS_FN int walk_half(const RunLine &l, int half, int first, int len, Emit
     j = jn;
   } while (sure && j < len);
   return j;
+}
+
+// Sub-elements [k0, k1) of a usable line: emit as walk_half's, and step(lo,
+// hi) for the stretch of a half that no run certifies, at most two of them,
+// each to be walked upwards (a disc's position is accumulated from its row's
+// start, so that one by one and downwards they would cost their square).
+template <bool REFINE, typename Emit, typename Step>
+DREAM_RUNS_FN void walk_line(const RunLine &l, int k0, int k1, Emit emit, Step step)
+{
+#pragma clang loop unroll(disable)
+  for (int half = 0; half < 2; half++) {
+    int len;
+    const int first = half_of(l, half, k0, k1, len);
+    const int m = walk_half<REFINE>(l, half, first, len, emit);
+    if (m < len) step(half ? first - len + 1 : first + m, half ? first - m + 1 : first + len);
+  }
 }
 
 // ------------------------------------------------------------------ host

@@ -7,6 +7,10 @@
 //   run_sums_check disc RADIUS STEP NEAR: a disc's rows.
 //     Points NEAR mm and more away.  Print lines walked, lines left to step,
 //     worst error (REFINE), largest deviation from the fit and its bound.
+//   run_sums_check rest SEED LINES: disc rows with a sub-element on a rounding
+//     boundary.  Prints lines, sub-elements left to step, the most position
+//     updates that these take (in lengths of the row), and sub-elements not
+//     walked exactly once.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -141,11 +145,55 @@ static int aperture(bool disc, double size, double step, double near)
   return 0;
 }
 
+static int rest(int lines)
+{
+  double most = 0.0;
+  long wrong = 0, used = 0, left = 0;
+  for (int q = 0; q < lines; q++) {
+    const int n = 200 + (int) uni(0.0, 4000.0), tie = (int) uni(0.0, n);
+    RunLine l;
+    l.dv = 0.02;
+    l.inv_dv = 50.0;
+    l.v0 = uni(-0.2, 1.2) * n * l.dv;
+    const double z = uni(4.0, 40.0), vt = l.v0 - tie * l.dv, dt = uni(0.02, 0.1);
+    const double t = std::sqrt(z * z + vt * vt) * 1000.0 / 1500.0;
+    l.w = z * z;
+    grid_of(l, 1500.0, dt, t - (std::floor(t / dt) + 0.5) * dt, 2000.0);
+    if (!dream::runs_ready<true>(l, n)) continue;
+    used++;
+    // In parts, as the kernel walks them.
+    const int parts = 1 + q % 5;
+    for (int p = 0; p < parts; p++) {
+      const int k0 = n * p / parts, k1 = n * (p + 1) / parts;
+      long updates = 0, walked = 0;
+      std::vector<int> seen((size_t) n, 0);
+      dream::walk_line<true>(l, k0, k1, [&](int, int c, double) { walked += c; },
+                             [&](int lo, int hi) {
+        updates += hi;                       // from the row's start, then along
+        left += hi - lo;
+        for (; lo < hi; lo++) seen[(size_t) lo]++;
+      });
+      for (int k = 0; k < n; k++) {
+        walked += seen[(size_t) k];
+        wrong += seen[(size_t) k] > (k >= k0 && k < k1 ? 1 : 0);
+      }
+      wrong += std::labs(walked - (k1 - k0));
+      most = std::fmax(most, (double) updates / (double) n);
+    }
+  }
+  std::printf("%ld %ld %.3f %ld\n", used, left, most, wrong);
+  return 0;
+}
+
 int main(int argc, char **argv)
 {
   if (argc > 3 && std::strcmp(argv[1], "equal") == 0) {
     gen.seed((unsigned) std::atoi(argv[2]));
     return equal(std::atoi(argv[3]));
+  }
+  if (argc > 3 && std::strcmp(argv[1], "rest") == 0) {
+    gen.seed((unsigned) std::atoi(argv[2]));
+    return rest(std::atoi(argv[3]));
   }
   if (argc < 5) return 2;
   gen.seed(1);

@@ -59,3 +59,13 @@ def test_accumulated_positions(check, shape, size, step, near, walked):
     assert fit >= walked
     assert seen <= bound
     assert worst <= 2.0 ** -47 + 4e-15
+
+
+def test_rest_of_a_half_is_one_stretch(check):
+    """The sub-elements that no run certifies are walked once each, in
+    stretches: positions accumulated from a disc row's start take at most two
+    passes over the row, not one pass for each sub-element."""
+    used, left, most, wrong = check("rest", 1, 4000)
+    assert used > 3000 and left > 1000
+    assert wrong == 0
+    assert most <= 2.0
