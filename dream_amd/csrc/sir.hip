@@ -53,6 +53,7 @@
 #include <numeric>
 #include <type_traits>
 
+#include "plan_layout.hpp"
 #include "sir.hpp"
 #include "sir_runs.hpp"
 #include "tune.hpp"
@@ -1061,10 +1062,9 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return cost[a] > cost[b]; });
 
-  // One buffer: descriptors | status blocks | counters | tables.
-  const size_t o_status = P * sizeof(SirDev), o_counter = o_status + P * sizeof(Status);
-  const size_t o_tables = o_counter + 2 * sizeof(unsigned long long);
-  const size_t bytes = o_tables + table_doubles * sizeof(double);
+  const PlanLayout at = plan_layout(P * sizeof(SirDev), P * sizeof(Status),
+                                    2 * sizeof(unsigned long long), table_doubles * sizeof(double));
+  const size_t bytes = at.bytes;
   static_assert(sizeof(SirDev) % 8 == 0 && sizeof(Status) % 8 == 0, "plan buffer alignment");
   char *base;
   if (one_shot_) {
@@ -1074,9 +1074,9 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
     base = (char *) d_base_;
   }
   d_probs_ = (SirDev *) base;
-  d_status_ = (Status *) (base + o_status);
-  d_counter_ = (unsigned long long *) (base + o_counter);
-  d_tables_ = (double *) (base + o_tables);
+  d_status_ = (Status *) (base + at.status);
+  d_counter_ = (unsigned long long *) (base + at.counter);
+  d_tables_ = (double *) (base + at.tables);
 
   std::vector<double> tables;
   tables.reserve(table_doubles);
@@ -1123,7 +1123,7 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
   image_.assign(bytes, 0);
   if (P) std::memcpy(image_.data(), host_.data(), P * sizeof(SirDev));
   if (!tables.empty())
-    std::memcpy(image_.data() + o_tables, tables.data(), tables.size() * sizeof(double));
+    std::memcpy(image_.data() + at.tables, tables.data(), tables.size() * sizeof(double));
   if (one_shot_) {
     last_stream_ = stream;
     DREAM_HIP_CHECK(hipMemcpyAsync(base, image_.data(), bytes, hipMemcpyHostToDevice, stream));
