@@ -171,44 +171,90 @@ __device__ __forceinline__ int find_problem(const SirDev *P, int n, int64_t item
 // run into the histogram when the bin changes, which along x happens at a
 // rate of about min(1, |rx|/r dx/l) per step (l = cp dt/1000, one sample of
 // path) and along y at min(1, |ry|/r dy/l); with up to 256 elements' mean
-// offsets for rx and ry, the cheapest walk is taken: a stepped flush counts
-// as 4 contributions, a run as 6 (75 instructions against 19.5 for a
-// contribution, and its flush), a line's set-up for runs as 8, and each walk
-// pays for its partly filled lane rounds.  Every wave of the point computes
-// the same sums in the same order, so all its items agree.
+// offsets for rx and ry, the cheaper stepped walk counts a flush as 4
+// contributions, and each walk pays for its partly filled lane rounds.
+//
+// A run's price: iterations a step (runs_per_step) for the wave's worst line,
+// as its lanes wait for it.  Near points are stepped (4096 points 1 mm from 64
+// elements of 0.4 x 10 mm, steps of 0.05 mm: 0.88 ms in runs, 0.36 in columns;
+// at 20 mm 0.17 against 0.36).  Measured over 84 forced calls (1 to 128
+// elements, 20 to 300 sub-elements a line, points at 0.05 to 20 mm, samples of
+// 0.03 to 0.3 mm of path): an iteration takes 2.0 to 2.7 stepped sub-elements,
+// a line's set-up and ends some 14, a stepped line's 6.  Every wave of the
+// point computes the same sums in the same order, so all its items agree.
 enum { WALK_ROWS = 0, WALK_COLUMNS = 1, WALK_RUNS = 2 };
+constexpr float kRunSteps = 2.7f, kLineSteps = 14.0f, kUnitSteps = 6.0f;
+
+// Largest value and sum over the wave, along DPP rows of 16 lanes and then
+// across them, from lane 63.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_f(float old, float v)
+{
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL,
+                                                    ROWS, 0xf, false));
+}
+__device__ __forceinline__ float last_lane(float v)
+{
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+__device__ __forceinline__ float wave_max_f(float v)
+{
+  v = __builtin_fmaxf(v, dpp_f<0x111, 0xf>(v, v));      // row_shr 1, 2, 4, 8
+  v = __builtin_fmaxf(v, dpp_f<0x112, 0xf>(v, v));
+  v = __builtin_fmaxf(v, dpp_f<0x114, 0xf>(v, v));
+  v = __builtin_fmaxf(v, dpp_f<0x118, 0xf>(v, v));
+  v = __builtin_fmaxf(v, dpp_f<0x142, 0xa>(v, v));      // row_bcast 15, 31
+  v = __builtin_fmaxf(v, dpp_f<0x143, 0xc>(v, v));
+  return last_lane(v);
+}
+__device__ __forceinline__ float wave_sum_f(float v)
+{
+  v += dpp_f<0x111, 0xf>(0.0f, v);
+  v += dpp_f<0x112, 0xf>(0.0f, v);
+  v += dpp_f<0x114, 0xf>(0.0f, v);
+  v += dpp_f<0x118, 0xf>(0.0f, v);
+  v += dpp_f<0x142, 0xa>(0.0f, v);
+  v += dpp_f<0x143, 0xc>(0.0f, v);
+  return last_lane(v);
+}
 
 __device__ __forceinline__ int pick_walk(const SirDev &P, double xo, double yo, double zo)
 {
   gdouble *el = (gdouble *) P.el;
-  const int L = P.L, every = (L + 255) / 256;
-  float fx = 0.0f, fy = 0.0f, n = 0.0f;
-  for (int e = (int) (threadIdx.x & 63) * every; e < L; e += 64 * every) {
-    const float mx = __builtin_fmaxf(__builtin_fabsf((float) (xo - el[e])), P.wx);
-    const float my = __builtin_fmaxf(__builtin_fabsf((float) (yo - el[L + e])), P.wy);
-    const float mz = (float) (zo - el[2 * L + e]);
+  const int L = P.L, every = P.pick_every;
+  const bool disc = P.shape == SIR_CIRC;
+  float fx = 0.0f, fy = 0.0f, its = 0.0f;
+  for (int g = 0; g < L; g += 64 * every) {
+    const int e = g + (int) (threadIdx.x & 63) * every, ec = min(e, L - 1);
+    const float cx = __builtin_fabsf((float) (xo - el[ec])), cy = __builtin_fabsf((float) (yo - el[L + ec]));
+    const float mx = __builtin_fmaxf(cx, P.wx), my = __builtin_fmaxf(cy, P.wy);
+    const float mz = (float) (zo - el[2 * L + ec]);
     const float q = __builtin_amdgcn_rsqf(mx * mx + my * my + mz * mz);
-    fx += __builtin_fminf(1.0f, mx * q * P.sx);       // NaN (all zero) counts as 1
-    fy += __builtin_fminf(1.0f, my * q * P.sy);
-    n += 1.0f;
+    if (e < L) {
+      fx += __builtin_fminf(1.0f, mx * q * P.sx);       // NaN (all zero) counts as 1
+      fy += __builtin_fminf(1.0f, my * q * P.sy);
+    }
+    // The element's nearest line, at its mean offset along it.
+    const float across = __builtin_fmaxf((disc ? cy : cx) - P.half, 0.0f), along = disc ? mx : my;
+    const float w = across * across + mz * mz;
+    float rate = runs_per_step(along, w, disc ? P.sx : P.sy, P.line_cap);
+    if (!(w >= P.line_wmin)) rate = __builtin_fmaxf(rate, 1.0f);   // stepped after all
+    its += wave_max_f(rate);
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    fx += __shfl_xor(fx, off, 64);
-    fy += __shfl_xor(fy, off, 64);
-    n += __shfl_xor(n, off, 64);
-  }
-  fx /= n;
-  fy /= n;
+  fx = wave_sum_f(fx) * P.pick_inv_n;
+  fy = wave_sum_f(fy) * P.pick_inv_n;
+  its *= P.pick_inv_g;
   const float nx = (float) P.nx, S = (float) P.seg_len;
   int walk;
-  if (P.shape == SIR_CIRC) {
-    walk = 8.0f + 6.0f * (1.0f + nx * fx) < nx * (1.0f + 4.0f * fx) ? WALK_RUNS : WALK_ROWS;
+  if (disc) {
+    walk = kLineSteps + kRunSteps * nx * its < nx + kUnitSteps ? WALK_RUNS : WALK_ROWS;
   } else {
     const float cost_r = P.rounds_r * (nx + 4.0f + 4.0f * (nx - 1.0f) * fx);
     const float cost_c = P.rounds_c * (S + 4.0f + 4.0f * (S - 1.0f) * fy);
-    const float cost_u = P.rounds_c * (8.0f + 6.0f * (1.0f + (S - 1.0f) * fy));
-    walk = cost_c < cost_r ? WALK_COLUMNS : WALK_ROWS;
-    if (P.runs && cost_u < __builtin_fminf(cost_c, cost_r)) walk = WALK_RUNS;
+    const bool columns = cost_c < cost_r;
+    walk = columns ? WALK_COLUMNS : WALK_ROWS;
+    const float stepped = columns ? P.rounds_c * (S + kUnitSteps) : P.rounds_r * (nx + kUnitSteps);
+    if (P.runs && P.rounds_c * (kLineSteps + kRunSteps * S * its) < stepped) walk = WALK_RUNS;
   }
   return __builtin_amdgcn_readfirstlane(walk);
 }
@@ -446,10 +492,14 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
       unsigned long long out_mask = 0;
       int j0 = sg * P.seg_len;
       const int j1 = min(j0 + P.seg_len, ny);
+      bool by_runs = false;
       if (walk == WALK_RUNS) {
         RunLine line{ye - P.line_p0, P.line_dv, P.line_inv_dv, rxz, P.c1, P.ic1, c2, 0.5 - lim,
                      P.line_dev};
-        if (runs_ready<REFINE_H>(line, ny)) {
+        // All lines of the wave or none: with one unfit (a point near the
+        // aperture) the wave steps its columns together, in blocks.
+        by_runs = __all(runs_ready<REFINE_H>(line, ny));
+        if (by_runs) {
           const double amp = el[5 * L + e] * P.amp;
           walk_line<REFINE_H>(line, j0, j1, [&](int b, int n, double v) { add_run(amp, b, n, v); },
                               [&](int lo, int hi) {
@@ -468,7 +518,7 @@ __device__ __forceinline__ void sir_item(const SirDev &P, int64_t local, double 
       // blocks of kBlock rows are a uniform count: the shorter length's when
       // any of its lanes holds a last segment.
       const int last_len = ny - (P.nseg - 1) * P.seg_len;
-      const int nb = walk == WALK_RUNS ? 0
+      const int nb = by_runs ? 0
                    : (__ballot(j1 - j0 < P.seg_len) ? last_len : P.seg_len) / kBlock;
       int j = j0;
       for (int blk = 0; blk < nb; blk++, j += kBlock) {
@@ -885,6 +935,19 @@ bool runs_hold(double dev, double step, double c1, int64_t nt)
   return c1 > 0.0 && step > 0.0 && c1 * step <= 4.0 && 8.0 * c1 * dev <= kBoundScale * ((double) nt + 2.0);
 }
 
+// What pick_walk asks: its elements, and of lines of spacing dv the distance
+// beyond which they are fit (runs_ready) and the longest run at a distance.
+void line_limits(SirDev &d, double dv, bool fp64)
+{
+  d.pick_every = (d.L + 255) / 256;
+  const int n = (d.L + d.pick_every - 1) / d.pick_every;
+  d.pick_inv_n = 1.0f / (float) n;
+  d.pick_inv_g = 1.0f / (float) ((n + 63) / 64);
+  const double near = fp64 ? 0x1p46 * d.line_dev : 0.0;
+  d.line_wmin = (float) std::max({64.0 * dv * dv, 4.0 * d.ic1 * d.ic1, near * near});
+  d.line_cap = (float) (1.0 / ((fp64 ? 36.0 : 20.0) * dv));
+}
+
 // Parts to cut the lines of a point into: the count (up to `most`) that
 // minimises the mean of lane rounds per item and full lane rounds x cost of
 // a part of `len` sub-elements, stepped or in runs (a bin each 0.2 dx / (cp
@@ -913,6 +976,7 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
           "SIR output precision must be DREAM_HIP_F64 or DREAM_HIP_F32");
   const size_t P = problems.size();
   const size_t esz = sizeof(double);          // LDS histogram entries are FP64
+  const bool fp64 = out_dtype == DREAM_HIP_F64;
   const size_t lds_cap = 64 * 1024;
   const int cus = device_cus();
   const int target_items = 8 * cus;
@@ -1014,6 +1078,8 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
       d.part_len = 1.0 / (double) disc_parts;
       d.runs = runs;
       d.line_dev = dev_mm;
+      d.half = (float) p.R;
+      line_limits(d, p.dx, fp64);
       d.walk = !runs ? WALK_ROWS : force;
       d.wx = d.wy = (float) (4.0 / (3.0 * M_PI) * p.R);   // mean |x| over the disc
       d.sx = (float) (p.dx / lam);
@@ -1023,6 +1089,8 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
       d.line_p0 = ys[i][0];
       line_fit(ys[i], p.dy, d.line_dv, d.line_dev);
       d.line_inv_dv = 1.0 / d.line_dv;
+      d.half = (float) std::max(xs[i].back(), -xs[i].front());
+      line_limits(d, d.line_dv, fp64);
       d.runs = force != WALK_COLUMNS && runs_hold(d.line_dev, d.line_dv, c1, p.nt);
       d.walk = force == WALK_RUNS && !d.runs ? WALK_COLUMNS : force;
       const int64_t QC = L * nx;

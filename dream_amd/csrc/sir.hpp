@@ -65,8 +65,13 @@ struct SirDev {
   double line_p0, line_dv, line_inv_dv, line_dev;
   // The walk choice: mean |xs| and |ys|, dx and dy in samples of path
   // (dx / (cp dt/1000), dy / (cp dt/1000)), lane rounds per item of the row
-  // and the column walk.
-  float wx, wy, sx, sy, rounds_r, rounds_c;
+  // and the column walk; for runs the elements' half extent across the lines,
+  // the least squared distance of fit lines and the longest run per mm of distance.
+  float wx, wy, sx, sy, rounds_r, rounds_c, half, line_wmin, line_cap;
+  // The elements it looks at (every pick_every-th), and one over their number
+  // and their groups of 64.
+  int32_t pick_every;
+  float pick_inv_n, pick_inv_g;
 };
 
 enum { SIR_LDS_STORE = 0, SIR_LDS_ATOMIC = 1, SIR_GLOBAL = 2 };

@@ -89,6 +89,23 @@ DREAM_RUNS_FN bool runs_ready(RunLine &l, int n)
          l.c1 * r + __builtin_fabs(l.c2) < 0x1p30 && r * l.inv_dv < 0x1p30;
 }
 
+// About how many iterations walk_half takes a step, for a line whose squared
+// distance from the point is w and whose sub-elements lie `along` from the
+// foot on average, s bins a step at the most, cap_per_mm w^0.5 the longest run: a
+// run ends with its bin or at its longest (one sub-element at the least).
+// The larger of the two rates and half the smaller.
+DREAM_RUNS_FN float runs_per_step(float along, float w, float s, float cap_per_mm)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float q = __builtin_amdgcn_rsqf(w), qa = __builtin_amdgcn_rsqf(w + along * along);
+#else
+  const float q = 1.0f / std::sqrt(w), qa = 1.0f / std::sqrt(w + along * along);
+#endif
+  const float bins = along * qa * s;
+  const float cuts = 1.0f / __builtin_fmaxf(1.0f, __builtin_floorf(w * q * cap_per_mm));
+  return __builtin_fmaxf(bins, cuts) + 0.5f * __builtin_fminf(bins, cuts);
+}
+
 // The two halves of sub-elements [k0, k1): half 0 starts at the first one
 // past the foot and goes up, half 1 starts before it and goes down.  Sets
 // the half's length and returns its first sub-element; step j of it is

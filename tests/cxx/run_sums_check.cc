@@ -11,6 +11,8 @@
 //     boundary.  Prints lines, sub-elements left to step, the most position
 //     updates that these take (in lengths of the row), and sub-elements not
 //     walked exactly once.
+//   run_sums_check price SEED LINES: prints lines and the least and largest
+//     ratio of a line's iterations to runs_per_step's.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -185,11 +187,45 @@ static int rest(int lines)
   return 0;
 }
 
+static int price(int lines)
+{
+  double least = 1e9, most = 0.0;
+  long used = 0;
+  for (int q = 0; q < lines; q++) {
+    const int n = 100 + (int) uni(0.0, 400.0);
+    RunLine l;
+    l.dv = 0.05;
+    l.inv_dv = 20.0;
+    l.v0 = uni(-0.5, 1.5) * n * l.dv;
+    const double z = 0.5 * std::exp(uni(0.0, 4.5));
+    l.w = z * z;
+    grid_of(l, 1500.0, 0.01 * std::exp(uni(0.0, 3.0)), z / 1.5, 2000.0);
+    if (!dream::runs_ready<true>(l, n)) continue;
+    long its = 0;
+    bool all = true;                       // no doubtful edge
+    double along = 0.0;
+    for (int k = 0; k < n; k++) along += std::fabs(l.v0 - k * l.dv) / n;
+    dream::walk_line<true>(l, 0, n, [&](int, int, double) { its++; }, [&](int, int) { all = false; });
+    if (!all) continue;
+    used++;
+    const double r = (double) its / (n * dream::runs_per_step((float) along, (float) l.w, (float) (l.c1 * l.dv),
+                                                              (float) (1.0 / (36.0 * l.dv))));
+    least = std::fmin(least, r);
+    most = std::fmax(most, r);
+  }
+  std::printf("%ld %.3f %.3f\n", used, least, most);
+  return 0;
+}
+
 int main(int argc, char **argv)
 {
   if (argc > 3 && std::strcmp(argv[1], "equal") == 0) {
     gen.seed((unsigned) std::atoi(argv[2]));
     return equal(std::atoi(argv[3]));
+  }
+  if (argc > 3 && std::strcmp(argv[1], "price") == 0) {
+    gen.seed((unsigned) std::atoi(argv[2]));
+    return price(std::atoi(argv[3]));
   }
   if (argc > 3 && std::strcmp(argv[1], "rest") == 0) {
     gen.seed((unsigned) std::atoi(argv[2]));

@@ -69,3 +69,15 @@ def test_rest_of_a_half_is_one_stretch(check):
     assert used > 3000 and left > 1000
     assert wrong == 0
     assert most <= 2.0
+
+
+def test_price_of_runs(check):
+    """The walk choice's estimate of a line's iterations against the walk's, for
+    points at 0.5 to 45 mm (with the runs' longest length left out of it a near
+    line was priced at a tenth of its iterations and below).  The estimate adds
+    half the smaller of two rates where the true count lies between their
+    larger and their sum, and takes the mean offset for all sub-elements: 1/1.6
+    to 1.5."""
+    used, least, most = check("price", 1, 20000)
+    assert used > 18000
+    assert 1 / 1.6 <= least and most <= 1.5
