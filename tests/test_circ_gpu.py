@@ -84,3 +84,20 @@ def test_mixed_rect_and_disc_batch(gpu, oracle):
     for H, ref in zip(batch.run(use_graph=True), refs):
         torch.cuda.synchronize()
         assert rel_l2(H.cpu().numpy().T, ref) <= 2e-5
+
+
+@pytest.mark.parametrize("nt", [999, 1000, 1999, 2000])
+def test_copies_of_the_histogram(gpu, oracle, nt):
+    """Response lengths on either side of those at which the number of LDS
+    histogram copies changes: equal to the oracle to this file's bar."""
+    from dream_amd.torch_ops import arr_circ
+    rng = np.random.default_rng(nt)
+    G = np.c_[[-1.2, 0.0, 1.3], [0.1, 0.0, -0.2], np.zeros(3)]
+    Ro = np.c_[rng.uniform(-4, 4, 30), rng.uniform(-3, 3, 30), rng.uniform(3, 20, 30)]
+    dt = 20.0 / nt
+    ref, _, oob = oracle.dream_arr_circ(Ro, 0.5, 0.03, 0.03, dt, nt, np.array([0.5]), 1.0, 1500.0, G,
+                                        nthreads=4, err_level="ignore")
+    H, _, n = arr_circ(torch.tensor(Ro.T.copy(), device="cuda"), 0.5, 0.03, 0.03, dt, nt, 0.5, 1.0,
+                       1500.0, G, err_level="ignore")
+    assert n == oob
+    assert np.max(np.abs(H.cpu().numpy().T - ref)) <= 1e-12 * np.abs(ref).max()
