@@ -1099,6 +1099,14 @@ __device__ __forceinline__ float weigh(frames4 g, frames4 v)
 // waiting: 64 x 64 elements, 2^19 voxels, 8 frames, nearest-lower took 6.25 ms,
 // now 3.0 (the forward 2.33); one FP32 frame of 48 x 48 over 30720 pixels,
 // linear, 330 us, now 95.
+//
+// FP32 sums: a group's kG products for a transmit, a job's rows for a
+// receiver; everything past them, and the speed's sum from the first product on,
+// is FP64.  With the row's 16 receivers and the wave's total in FP32 the four
+// products of a frame group cost the transmit gradient 13 to 29 % more error
+// than one frame at a time had (1.20 -> 1.36e-7 RMS, 32 x 32; now 0.91e-7),
+// for 3 % of the time.  The order in which work-groups add their FP64 sums is
+// not fixed: a gradient's last few 1e-16 differ from call to call.
 // Waves per SIMD of the pixel adjoint, near what its registers allow: FP32
 // nearest-lower groups of four frames fit four waves (3.0 ms; three 3.6, five
 // spill and take 7.3), linear sampling is fastest with all it asks for
@@ -1201,11 +1209,11 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
           if (__all(!valid || !(lo < (GT) K) || !(hi > GT(-1)))) continue;
           const DT wi = APOD ? at[i] : DT(1);
           constexpr int kG = (INTERP == DREAM_HIP_NEAREST ? kRC : kRC / 2) / (FR == 4 ? 2 : 1);
-          DT zi = DT(0), zc = DT(0);
+          double zi = 0.0, zc = 0.0;
 #pragma unroll
           for (int g0 = 0; g0 < kRC; g0 += kG) {
             unsigned o0[kG], o1[kG];
-            DT f[kG];
+            DT f[kG], zg = DT(0);
             VT y0[kG], y1[kG];
 #pragma unroll
             for (int jj = 0; jj < kG; jj++) {
@@ -1228,23 +1236,24 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
               if (INTERP == DREAM_HIP_LINEAR) {
                 const DT slope = weigh(gp, y1[jj] - y0[jj]);
                 val += f[jj] * slope;
-                zc += wj * slope * (DT) (tt0 + tr[g0 + jj]);
+                zc = __builtin_fma((double) (wj * slope), (double) (tt0 + tr[g0 + jj]), zc);
               }
-              zi = fma_d(wj, val, zi);
+              zg = fma_d(wj, val, zg);
               zj[g0 + jj] = fma_d(wi, val, zj[g0 + jj]);
             }
+            zi += (double) zg;
           }
-          const DT total = wave_total(zi);
-          if (lane == 63 && total != DT(0)) lds_atomic_add(&zt[i], (double) total);
-          if (INTERP == DREAM_HIP_LINEAR) zcp += (double) (wi * zc);
+          const double total = wave_total(zi);
+          if (lane == 63 && total != 0.0) lds_atomic_add(&zt[i], total);
+          if (INTERP == DREAM_HIP_LINEAR) zcp = __builtin_fma((double) wi, zc, zcp);
         }
       };
       if (all_valid && j0 + kRC <= Lr) rows(std::true_type{});
       else rows(std::false_type{});
 #pragma unroll
       for (int jj = 0; jj < kRC; jj++) {
-        const DT total = wave_total(zj[jj]);
-        if (lane == 63 && j0 + jj < Lr && total != DT(0)) lds_atomic_add(&zr[j0 + jj], (double) total);
+        const double total = wave_total((double) zj[jj]);
+        if (lane == 63 && j0 + jj < Lr && total != 0.0) lds_atomic_add(&zr[j0 + jj], total);
       }
     }
   }
