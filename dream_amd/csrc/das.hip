@@ -1074,10 +1074,11 @@ __device__ __forceinline__ T wave_total(T v)
 __device__ __forceinline__ float fma_d(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_d(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// <g, v> of a lane: one frame's product, or (FR = 4) a record's four.
-__device__ __forceinline__ float weigh(float g, float v) { return g * v; }
-__device__ __forceinline__ double weigh(double g, double v) { return g * v; }
-__device__ __forceinline__ float weigh(frames4 g, frames4 v)
+// What a lane sums over its pairs: one frame's sample, whose sums g weighs
+// at their end, or (FR = 4) the product of a record's four with their g.
+__device__ __forceinline__ float lane_value(float, float v) { return v; }
+__device__ __forceinline__ double lane_value(double, double v) { return v; }
+__device__ __forceinline__ float lane_value(frames4 g, frames4 v)
 {
   return __builtin_fmaf(g[3], v[3], __builtin_fmaf(g[2], v[2], __builtin_fmaf(g[1], v[1], g[0] * v[0])));
 }
@@ -1100,13 +1101,14 @@ __device__ __forceinline__ float weigh(frames4 g, frames4 v)
 // now 3.0 (the forward 2.33); one FP32 frame of 48 x 48 over 30720 pixels,
 // linear, 330 us, now 95.
 //
-// FP32 sums: a group's kG products for a transmit, a job's rows for a
-// receiver; everything past them, and the speed's sum from the first product on,
-// is FP64.  With the row's 16 receivers and the wave's total in FP32 the four
-// products of a frame group cost the transmit gradient 13 to 29 % more error
-// than one frame at a time had (1.20 -> 1.36e-7 RMS, 32 x 32; now 0.91e-7),
-// for 3 % of the time.  The order in which work-groups add their FP64 sums is
-// not fixed: a gradient's last few 1e-16 differ from call to call.
+// FP32 sums run over a row's 16 receivers, 16 rows of a receiver and the wave;
+// g weighs one frame's at their end.  A frame group's products carry the rounding
+// of four frames already: with linear sampling its sums are FP64 from a gather
+// group of a row on (in FP32 the transmit gradient had 13 to 29 % more error
+// than one frame at a time, 1.20 -> 1.36e-7 RMS, 32 x 32; now 0.91e-7, for 5 %
+// of the time).  The speed's sum is FP64 from the first product on.  The
+// order in which work-groups add their FP64 sums is not fixed: a gradient's
+// last few 1e-16 differ from call to call.
 // Waves per SIMD of the pixel adjoint, near what its registers allow: FP32
 // nearest-lower groups of four frames fit four waves (3.0 ms; three 3.6, five
 // spill and take 7.3), linear sampling is fastest with all it asks for
@@ -1122,6 +1124,8 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
 {
   static_assert(FR == 1 || std::is_same<DT, float>::value, "frame groups: FP32");
   using VT = lane_t<DT, FR>;
+  // A row's and the wave's totals (see the comment above).
+  using ST = typename std::conditional<INTERP == DREAM_HIP_LINEAR && FR == 4, double, DT>::type;
   extern __shared__ __align__(16) unsigned char smem[];
   double *zt = reinterpret_cast<double *>(smem);
   double *zr = zt + A.Lt;
@@ -1159,6 +1163,7 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
     const GT xo = Ro[p], yo = Ro[p + A.No], zo = Ro[p + 2 * A.No];
     const DT *gv = (const DT *) A.g;
     VT gp;
+    DT g1 = DT(1);                    // the sums' weight: one frame's g
     const VT *Yf;
     if constexpr (FR == 4) {
 #pragma unroll
@@ -1166,7 +1171,7 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
         gp[q] = valid && 4 * row + q < A.n_frames ? gv[(4 * row + q) * A.im_stride + p] : 0.0f;
       Yf = (const VT *) A.Yg + row * A.yg_stride;
     } else {
-      gp = valid ? gv[row * A.im_stride + p] : DT(0);
+      gp = g1 = valid ? gv[row * A.im_stride + p] : DT(0);
       Yf = (const VT *) A.Y + row * A.y_stride;
     }
     const __amdgpu_buffer_rsrc_t ry = ascan_rsrc(Yf, K, (int) sizeof(VT));
@@ -1188,16 +1193,17 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
           tr[jj] = leg3_wave<GT>(Gr[j] - xo, Gr[j + Lr] - yo, Gr[j + 2 * Lr] - zo) * inv_cp;
         else
           tr[jj] = leg3_wave<GT>(gx_r, Gr[j + Lr] - yo, Gr[j + 2 * Lr] - zo) * inv_cp;
-        zj[jj] = DT(0);
         // The linear rule's cp gradient weighs with the unclamped travel time.
         const GT t = clamp_leg<GT>(tr[jj], tmax);
         if (INTERP == DREAM_HIP_NEAREST) tr[jj] = t;
         trmin = jj ? fmin(trmin, t) : t;
         trmax = jj ? fmax(trmax, t) : t;
       }
+      // FP32 receivers' sums run over 16 rows at the most.
+      int ib = i0, ie;
       auto rows = [&](auto all_live) {
         constexpr bool ALL_LIVE = decltype(all_live)::value;
-        for (int i = i0; i < i1; i++) {
+        for (int i = ib; i < ie; i++) {
           GT tt;
           if (TYPE == DAS_TFM)
             tt = leg3_wave<GT>(Gt[i] - xo, Gt[i + Lt] - yo, Gt[i + 2 * Lt] - zo) * inv_cp;
@@ -1209,7 +1215,8 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
           if (__all(!valid || !(lo < (GT) K) || !(hi > GT(-1)))) continue;
           const DT wi = APOD ? at[i] : DT(1);
           constexpr int kG = (INTERP == DREAM_HIP_NEAREST ? kRC : kRC / 2) / (FR == 4 ? 2 : 1);
-          double zi = 0.0, zc = 0.0;
+          ST zi = ST(0);
+          double zc = 0.0;
 #pragma unroll
           for (int g0 = 0; g0 < kRC; g0 += kG) {
             unsigned o0[kG], o1[kG];
@@ -1229,31 +1236,40 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
               y0[jj] = sload<VT>(ry, o0[jj], soff);
               if (INTERP != DREAM_HIP_NEAREST) y1[jj] = sload<VT>(ry, o1[jj], soff);
             }
+            // All of the group's gathers before the first use: where the
+            // scheduler saw registers scarce it let the uses wait in between.
+            if constexpr (INTERP == DREAM_HIP_NEAREST && (sizeof(DT) == 8 || !ALL_LIVE))
+              __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int jj = 0; jj < kG; jj++) {
               const DT wj = APOD ? ar[min(j0 + g0 + jj, Lr - 1)] : DT(1);
-              DT val = weigh(gp, y0[jj]);
+              DT val = lane_value(gp, y0[jj]);
               if (INTERP == DREAM_HIP_LINEAR) {
-                const DT slope = weigh(gp, y1[jj] - y0[jj]);
+                const DT slope = lane_value(gp, y1[jj] - y0[jj]);
                 val += f[jj] * slope;
                 zc = __builtin_fma((double) (wj * slope), (double) (tt0 + tr[g0 + jj]), zc);
               }
               zg = fma_d(wj, val, zg);
               zj[g0 + jj] = fma_d(wi, val, zj[g0 + jj]);
             }
-            zi += (double) zg;
+            zi += (ST) zg;
           }
-          const double total = wave_total(zi);
-          if (lane == 63 && total != 0.0) lds_atomic_add(&zt[i], total);
-          if (INTERP == DREAM_HIP_LINEAR) zcp = __builtin_fma((double) wi, zc, zcp);
+          const ST total = wave_total((ST) g1 * zi);
+          if (lane == 63 && total != ST(0)) lds_atomic_add(&zt[i], (double) total);
+          if (INTERP == DREAM_HIP_LINEAR) zcp = __builtin_fma((double) wi * (double) g1, zc, zcp);
         }
       };
-      if (all_valid && j0 + kRC <= Lr) rows(std::true_type{});
-      else rows(std::false_type{});
+      for (; ib < i1; ib = ie) {
+        ie = sizeof(DT) == 4 ? min(ib + kTB, i1) : i1;
 #pragma unroll
-      for (int jj = 0; jj < kRC; jj++) {
-        const double total = wave_total((double) zj[jj]);
-        if (lane == 63 && j0 + jj < Lr && total != 0.0) lds_atomic_add(&zr[j0 + jj], total);
+        for (int jj = 0; jj < kRC; jj++) zj[jj] = DT(0);
+        if (all_valid && j0 + kRC <= Lr) rows(std::true_type{});
+        else rows(std::false_type{});
+#pragma unroll
+        for (int jj = 0; jj < kRC; jj++) {
+          const ST total = wave_total((ST) (g1 * zj[jj]));
+          if (lane == 63 && j0 + jj < Lr && total != ST(0)) lds_atomic_add(&zr[j0 + jj], (double) total);
+        }
       }
     }
   }
@@ -1921,11 +1937,15 @@ void adj_launch(const DasArgs &a, const int32_t *perm, bool want_gy, hipStream_t
     const int64_t tiles = ((a.No + 63) / 64) * rows;
     constexpr int64_t kItems = 4;
     const int64_t slots = (int64_t) cu_count() * 4 * (kThreads / 64);
-    // Blocks of 16 transmits amortise a job's 16 receive legs best; images
-    // that leave the device idle take shorter blocks, down to 4.
-    int tb = kTB;
+    // One frame at a time: a job's 16 receive legs are shared by a block of 64
+    // transmits while that leaves two jobs per wave slot, by 16 otherwise, by down
+    // to 4 where the device would be idle.  Frame groups take 16 at the most: at
+    // 128 x 128 elements, 2^14 pixels, 8 frames, 64 made them 0.65 -> 0.75 ms.
+    // 64 x 64 elements, 2^18 voxels, nearest-lower, blocks of 16 -> 64: FP64, 8
+    // frames 5.98 -> 5.07 ms, one FP32 frame 0.58 -> 0.49.
+    int tb = groups ? kTB : 4 * kTB;
     auto jobs_of = [&](int n) { return (int64_t) ((a.Lr + kRC - 1) / kRC) * ((a.Lt + n - 1) / n); };
-    while (tb > 4 && tiles * jobs_of(tb) < slots) tb /= 2;
+    while (tb > 4 && tiles * jobs_of(tb) < (tb > kTB ? 2 : 1) * slots) tb /= 2;
     const int64_t jobs = jobs_of(tb);
     const int split = (int) std::max<int64_t>(1, std::min(jobs, (kItems * slots + tiles - 1) / std::max<int64_t>(tiles, 1)));
     const size_t lds = (size_t) (a.Lt + a.Lr) * sizeof(double);

@@ -671,3 +671,36 @@ def test_frame_group_gradient_rounding(gpu, method, Lt, Lr, No):
             t[0], t[1], 0.02, 0.1, 1500.0, t[2], t[3], "linear", want_gy=False)
         sq.append(rel_l2(got[1].double().cpu().numpy(), ref[1].cpu().numpy()) ** 2)
     assert np.sqrt(np.mean(sq)) <= 1.25e-7
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("Lt,Lr,No", [
+    (63, 20, 30000),        # a block of 64 transmits that is not full, ragged receivers
+    (65, 16, 40000),        # one transmit past a block of 64
+    (40, 33, 70000),        # blocks of 32, one receiver past two chunks
+    (17, 48, 9000),         # one transmit past a block of 16
+])
+def test_pixel_adjoint_transmit_blocks(gpu, oracle, prec, Lt, Lr, No):
+    """Sizes at the edges of the pixel adjoint's transmit blocks and receiver
+    chunks, one frame, nearest-lower: apodization gradients against the FP64
+    oracle to this file's bars (FP32: 5e-6, thirty times its rounding)."""
+    from dream_amd.torch_ops import DasPlan
+    rng = np.random.default_rng(Lt)
+    K = 700
+    xt, xr = np.linspace(-5, 5, Lt), np.linspace(-4, 6, Lr)
+    Gt, Gr = np.c_[xt, np.zeros(Lt), np.zeros(Lt)], np.c_[xr, np.zeros(Lr), np.zeros(Lr)]
+    Ro = np.c_[rng.uniform(-6, 6, No), np.zeros(No), rng.uniform(1, 9, No)]
+    dt_ = torch.float64 if prec == "f64" else torch.float32
+    Y = rng.standard_normal((K, Lt * Lr)).astype(np.float32).astype(np.float64)
+    g = rng.standard_normal(No).astype(np.float32).astype(np.float64)
+    at = rng.uniform(0.5, 1.5, Lt).astype(np.float32).astype(np.float64)
+    ar = rng.uniform(0.5, 1.5, Lr).astype(np.float32).astype(np.float64)
+    _, gat, gar, _ = oracle.das_ext_adjoint(Y, Gt, Gr, Ro, 0.02, 0.1, 1500.0, g, "tfm", "nearest",
+                                            at, ar, nthreads=8)
+    plan = DasPlan("tfm", K, Ro, Gt, Gr, precision=prec)
+    t = [torch.tensor(a, dtype=dt_, device="cuda") for a in (Y.T.copy(), g, at, ar)]
+    _, rat, rar, _ = plan.adjoint(t[0], t[1], 0.02, 0.1, 1500.0, t[2], t[3], "nearest",
+                                  want_gy=False, want_cp=False)
+    bar = 1e-10 if prec == "f64" else 5e-6
+    assert rel_l2(rat.double().cpu().numpy(), gat) <= bar
+    assert rel_l2(rar.double().cpu().numpy(), gar) <= bar
