@@ -1109,12 +1109,14 @@ __device__ __forceinline__ float lane_value(frames4 g, frames4 v)
 // of the time).  The speed's sum is FP64 from the first product on.  The
 // order in which work-groups add their FP64 sums is not fixed: a gradient's
 // last few 1e-16 differ from call to call.
-// Waves per SIMD of the pixel adjoint, near what its registers allow: FP32
-// nearest-lower groups of four frames fit four waves (3.0 ms; three 3.6, five
-// spill and take 7.3), linear sampling is fastest with all it asks for
-// (eight frames of 2^18 voxels 2.9 ms, held to two waves 3.2).
+// Waves per SIMD of the pixel adjoint, near what its registers allow:
+// nearest-lower sampling fits four (FP32 groups of four frames 3.0 ms; three
+// 3.6, five spill and take 7.3), FP32 linear sampling is fastest with all it
+// asks for (eight frames of 2^18 voxels 2.9 ms, held to two waves 3.2), FP64
+// linear then drops to one wave in some modes (48 x 48 elements, 131072
+// voxels, 8 frames 3.7 ms, two waves 2.3).
 template <typename DT, int INTERP>
-constexpr int kAdjWaves = INTERP == DREAM_HIP_LINEAR ? 1 : (sizeof(DT) == 4 ? 4 : 3);
+constexpr int kAdjWaves = INTERP == DREAM_HIP_LINEAR ? (sizeof(DT) == 4 ? 1 : 2) : 4;
 
 template <typename DT, typename GT, int TYPE, int INTERP, bool APOD, int FR = 1>
 __global__ void __launch_bounds__(kThreads)
@@ -1164,14 +1166,16 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
     const DT *gv = (const DT *) A.g;
     VT gp;
     DT g1 = DT(1);                    // the sums' weight: one frame's g
+    DT g_sum;
     const VT *Yf;
     if constexpr (FR == 4) {
 #pragma unroll
       for (int q = 0; q < 4; q++)
         gp[q] = valid && 4 * row + q < A.n_frames ? gv[(4 * row + q) * A.im_stride + p] : 0.0f;
+      g_sum = (gp[0] + gp[1]) + (gp[2] + gp[3]);
       Yf = (const VT *) A.Yg + row * A.yg_stride;
     } else {
-      gp = g1 = valid ? gv[row * A.im_stride + p] : DT(0);
+      gp = g1 = g_sum = valid ? gv[row * A.im_stride + p] : DT(0);
       Yf = (const VT *) A.Y + row * A.y_stride;
     }
     const __amdgpu_buffer_rsrc_t ry = ascan_rsrc(Yf, K, (int) sizeof(VT));
@@ -1186,19 +1190,27 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
       GT tr[kRC];
       DT zj[kRC];
       GT trmin, trmax;
+      // Zero samples times a non-finite weight, g or travel time are NaN: rows
+      // with one are not skipped (a sum is not finite if one of its terms is
+      // not).
+      DT odd_w = g_sum;
+      GT odd_t = GT(0);
 #pragma unroll
       for (int jj = 0; jj < kRC; jj++) {
         const int j = min(j0 + jj, Lr - 1);
+        if (APOD) odd_w += ar[j];
         if (TYPE == DAS_TFM)
           tr[jj] = leg3_wave<GT>(Gr[j] - xo, Gr[j + Lr] - yo, Gr[j + 2 * Lr] - zo) * inv_cp;
         else
           tr[jj] = leg3_wave<GT>(gx_r, Gr[j + Lr] - yo, Gr[j + 2 * Lr] - zo) * inv_cp;
         // The linear rule's cp gradient weighs with the unclamped travel time.
+        if (INTERP == DREAM_HIP_LINEAR) odd_t += tr[jj];
         const GT t = clamp_leg<GT>(tr[jj], tmax);
         if (INTERP == DREAM_HIP_NEAREST) tr[jj] = t;
         trmin = jj ? fmin(trmin, t) : t;
         trmax = jj ? fmax(trmax, t) : t;
       }
+      const bool plain = __all(__builtin_isfinite(odd_w) && __builtin_isfinite(odd_t));
       // FP32 receivers' sums run over 16 rows at the most.
       int ib = i0, ie;
       auto rows = [&](auto all_live) {
@@ -1212,8 +1224,10 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
           const GT tt0 = tt;
           tt = clamp_leg<GT>(tt + dl, tmax);
           const GT lo = (tt + trmin) * fs, hi = (tt + trmax) * fs;
-          if (__all(!valid || !(lo < (GT) K) || !(hi > GT(-1)))) continue;
           const DT wi = APOD ? at[i] : DT(1);
+          const bool fine = __builtin_isfinite(wi) &&
+                            (INTERP == DREAM_HIP_NEAREST || __builtin_isfinite(tt0));
+          if (plain && __all(!valid || (fine && (!(lo < (GT) K) || !(hi > GT(-1)))))) continue;
           constexpr int kG = (INTERP == DREAM_HIP_NEAREST ? kRC : kRC / 2) / (FR == 4 ? 2 : 1);
           ST zi = ST(0);
           double zc = 0.0;

@@ -704,3 +704,54 @@ def test_pixel_adjoint_transmit_blocks(gpu, oracle, prec, Lt, Lr, No):
     bar = 1e-10 if prec == "f64" else 5e-6
     assert rel_l2(rat.double().cpu().numpy(), gat) <= bar
     assert rel_l2(rar.double().cpu().numpy(), gar) <= bar
+
+
+@pytest.mark.parametrize("frames", [1, 5])
+@pytest.mark.parametrize("method", ["tfm", "rca_coltx"])
+@pytest.mark.parametrize("odd", ["pixel nan", "pixel inf", "element inf", "g", "apod_t", "apod_r"])
+def test_adjoint_non_finite_input(gpu, method, odd, frames):
+    """One non-finite value where no pair reaches the data: the gradients it
+    weighs are NaN (a zero sample times it), with or without the data gradient
+    and whichever pixels share its wave; the others stay finite."""
+    from dream_amd.torch_ops import DasPlan
+    Lt, Lr, K, No = 20, 18, 64, 300
+    rng = np.random.default_rng(4)
+    xt, xr = np.linspace(-2, 2, Lt), np.linspace(-2, 2, Lr)
+    Gt = np.c_[xt, np.zeros(Lt), np.zeros(Lt)]
+    Gr = np.c_[xr, np.zeros(Lr), np.zeros(Lr)] if method == "tfm" else \
+        np.c_[np.zeros(Lr), xr, np.zeros(Lr)]
+    Ro = np.c_[rng.uniform(-2, 2, No), rng.uniform(-2, 2, No), rng.uniform(500, 600, No)]
+    Y, g = rng.standard_normal((frames, Lt * Lr, K)), rng.standard_normal((frames, No))
+    at, ar = rng.uniform(0.5, 1.5, Lt), rng.uniform(0.5, 1.5, Lr)
+    if odd.startswith("pixel"):
+        Ro[77, 2] = float(odd.split()[1])
+    elif odd == "element inf":
+        Gt[3, 2] = np.inf
+    elif odd == "g":
+        g[-1, 77] = np.nan
+    elif odd == "apod_t":
+        at[3] = np.inf
+    else:
+        ar[3] = np.inf
+    for prec in ("f64", "f32"):
+        dt_ = torch.float64 if prec == "f64" else torch.float32
+        t = [torch.tensor(a, dtype=dt_, device="cuda") for a in (Y, g, at, ar)]
+        plan = DasPlan(method, K, Ro, Gt, Gr, precision=prec)
+        for interp in ("nearest", "linear"):
+            for want_gy in (True, False):
+                _, gat, gar, gcp = plan.adjoint(t[0], t[1], 0.02, 0.1, 1500.0, t[2], t[3], interp,
+                                                want_gy=want_gy, want_cp=interp == "linear")
+                nan = [bool(torch.isnan(v).all()) if odd in ("g", "apod_t", "apod_r") else
+                       bool(torch.isnan(v).any()) for v in (gat, gar)]
+                fin = [bool(torch.isfinite(v).all()) for v in (gat, gar)]
+                key = (prec, interp, want_gy)
+                if odd == "g":
+                    assert nan == [True, True], key
+                elif odd == "apod_t":
+                    assert nan[1] and fin[0], key
+                elif odd == "apod_r":
+                    assert nan[0] and fin[1], key
+                else:
+                    assert fin == [True, True], key
+                if interp == "linear":
+                    assert bool(torch.isnan(gcp)), key
