@@ -1114,7 +1114,7 @@ __device__ __forceinline__ float lane_value(frames4 g, frames4 v)
 // 3.6, five spill and take 7.3), FP32 linear sampling is fastest with all it
 // asks for (eight frames of 2^18 voxels 2.9 ms, held to two waves 3.2), FP64
 // linear then drops to one wave in some modes (48 x 48 elements, 131072
-// voxels, 8 frames 3.7 ms, two waves 2.3).
+// voxels, 8 frames 3.7 ms, two waves 2.5).
 template <typename DT, int INTERP>
 constexpr int kAdjWaves = INTERP == DREAM_HIP_LINEAR ? (sizeof(DT) == 4 ? 1 : 2) : 4;
 
