@@ -49,6 +49,8 @@
 #include <cmath>
 #include <cstring>
 #include <numeric>
+#include <string>
+#include <unordered_map>
 
 namespace dream {
 
@@ -507,6 +509,7 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
   std::vector<double> tables;
   std::vector<AttDev> dev_p(P);
   std::vector<AttGrid> grids;
+  std::unordered_map<std::string, size_t> known;        // grids by their bytes
   std::vector<int64_t> cells;                   // per grid: (point, element) pairs it serves
   std::vector<size_t> off_sub(P), off_el(P), grid_of(P);
   std::vector<int64_t> spec_off(P);
@@ -554,8 +557,7 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
     g.alpha = alpha;
     g.step = p.cp * g.dt_s;
     d.gmax = 0.515 * alpha / g.dt_s;
-    size_t gi = 0;
-    while (gi < grids.size() && std::memcmp(&grids[gi], &g, sizeof g) != 0) gi++;
+    const size_t gi = known.try_emplace(std::string((const char *) &g, sizeof g), grids.size()).first->second;
     if (gi == grids.size()) {
       grids.push_back(g);
       cells.push_back(0);
@@ -569,8 +571,8 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
     // Whole elements per chunk where the array has enough of them: a chunk
     // that ends inside an element transforms that element's cells twice.
     if (chunks <= L) chunks = L / (L / chunks);
-    // The chunks' spectra are kept apart: at most 256 MiB of them.
-    chunks = std::max<int64_t>(1, std::min<int64_t>(chunks, (256ll << 20) / 16 / K / std::max<int64_t>(p.No, 1)));
+    // The chunks' spectra are kept apart: at most 256 MiB of them in the call.
+    chunks = std::max<int64_t>(1, std::min<int64_t>(chunks, (256ll << 20) / 16 / (int64_t) P / K / std::max<int64_t>(p.No, 1)));
     d.chunks = (int32_t) chunks;
     d.bin_blocks = (int32_t) ((K + kBinBlock - 1) / kBinBlock);
     d.item_begin = items;
@@ -600,12 +602,16 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
   const size_t o_status = take(P * sizeof(Status));
   std::vector<size_t> o_gam, o_tw, o_table;
   std::vector<bool> has_table;
-  int64_t grid_work = 1;
+  int64_t grid_work = 1, table_total = 0;
   for (size_t k = 0; k < grids.size(); k++) {
     const int64_t nt = grids[k].nt, K = nt / 2 + 1;
     // The table pays when the (point, element) pairs that read it, about 16
     // samples each, are more than its nt rows, and is not used with sub-cells.
-    const bool t = q == 1 && nt * K * (int64_t) sizeof(double2) <= kTableBytes && cells[k] * 16 >= nt;
+    // All tables of a call take 8 times kTableBytes at the most.
+    const int64_t table = nt * K * (int64_t) sizeof(double2);
+    const bool t = q == 1 && table <= kTableBytes && cells[k] * 16 >= nt &&
+                   table_total + table <= 8 * kTableBytes;
+    if (t) table_total += table;
     has_table.push_back(t);
     o_gam.push_back(take((size_t) K * sizeof(double2)));
     o_tw.push_back(take((size_t) nt * sizeof(double2)));
@@ -643,11 +649,15 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
     DREAM_HIP_CHECK(hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, s));
     const AttGrid *d_grids = (const AttGrid *) (base + o_grids);
     const AttDev *d_probs = (const AttDev *) (base + o_probs);
-    hipLaunchKernelGGL(att_grid_kernel,
-                       dim3((unsigned) std::min<int64_t>((grid_work + kThreads - 1) / kThreads, 4096),
-                            (unsigned) grids.size()),
-                       dim3(kThreads), 0, s, d_grids, d_status, (int) P);
-    DREAM_HIP_CHECK(hipGetLastError());
+    // In launches of up to 32768 grids (the y extent's limit is 65535).
+    for (size_t k = 0; k < grids.size(); k += 32768) {
+      const size_t n = std::min<size_t>(grids.size() - k, 32768);
+      hipLaunchKernelGGL(att_grid_kernel,
+                         dim3((unsigned) std::min<int64_t>((grid_work + kThreads - 1) / kThreads, 4096),
+                              (unsigned) n),
+                         dim3(kThreads), 0, s, d_grids + k, d_status, k == 0 ? (int) P : 0);
+      DREAM_HIP_CHECK(hipGetLastError());
+    }
     if (items > 0) {
       if (terms == 8)
         hipLaunchKernelGGL(att_spectrum_kernel<8>, dim3((unsigned) items), dim3(kThreads), lds, s,

@@ -148,3 +148,50 @@ def test_attenuated_moments(gpu, oracle, alpha, delay, nt):
     ref, _, _ = oracle.dreamrect(Ro, *geom, step, step, dt, nt, d, 1.0, CP, err_level="ignore",
                                  nthreads=4, alpha=alpha)
     assert _close(H, ref)
+
+
+def _att_batch(n, nt, dts, points):
+    """n one-element problems with their own intervals in one call."""
+    import ctypes
+
+    import torch
+    from dream_amd import _lib
+    Ro = torch.tensor(np.c_[np.linspace(-1, 1, points), np.zeros(points),
+                            np.linspace(3, 5, points)].T.copy(), device="cuda")
+    d = torch.zeros(1, dtype=torch.float64, device="cuda")
+    H = torch.empty((n, points, nt), dtype=torch.float64, device="cuda")
+    G, one = np.zeros((1, 3)), np.ones(1)
+    q = (_lib.DreamSirProblem * n)()
+    for i in range(n):
+        p = q[i]
+        p.Ro, p.No, p.a, p.b, p.dx, p.dy = Ro.data_ptr(), points, 0.2, 0.2, 0.1, 0.1
+        p.dt, p.nt, p.delay_type, p.delay, p.v, p.cp = dts[i], nt, 0, d.data_ptr(), 1.0, CP
+        p.num_elements, p.G, p.focal, p.apod = 1, G.ctypes.data, one.ctypes.data, one.ctypes.data
+        p.foc_met, p.steer_met = _lib.FOC_MET["off"], _lib.STEER_MET["off"]
+        p.err_level = _lib.ERR_LEVEL["ignore"]
+        p.h = H.data_ptr() + i * points * nt * 8
+
+    def run(lo, hi):
+        _lib.check(_lib.lib().dream_hip_sir_att_dev(
+            ctypes.cast(ctypes.byref(q, lo * ctypes.sizeof(_lib.DreamSirProblem)),
+                        ctypes.POINTER(_lib.DreamSirProblem)),
+            hi - lo, 5.0, _lib.F64, None, None, torch.cuda.current_stream().cuda_stream))
+        return H[lo:hi].cpu().numpy()
+    return run
+
+
+@pytest.mark.parametrize("n,nt,points,pick", [
+    (66000, 4, 1, [0, 32767, 32768, 65535, 65536, 65999]),    # more than one launch's grids
+    (12, 2000, 130, [0, 7, 8, 11]),                           # more than the tables' 256 MiB
+])
+def test_many_intervals_in_one_call(gpu, n, nt, points, pick):
+    """Problems that share no frequency grid: as many as a caller has, each
+    equal to its own call, whether its factors came from a table or not (the two
+    evaluate the same exponentials, apart by a few ulp of phases of 2 pi nt)."""
+    dts = np.linspace(0.8, 1.2, n) * 4.0 / CP * 1000.0 / nt * 2.0
+    run = _att_batch(n, nt, dts, points)
+    every = run(0, n)
+    for i in pick:
+        alone = run(i, i + 1)[0]
+        assert np.abs(alone).max() > 0
+        assert np.max(np.abs(every[i] - alone)) <= 1e-11 * np.abs(alone).max()
