@@ -229,8 +229,9 @@ att_spectrum_kernel(const AttDev *__restrict__ probs, int n_probs)
     square_range(xe, A.lo[0], A.hi[0], mn, mx);
     square_range(ye, A.lo[1], A.hi[1], mn, mx);
     square_range(ze, A.lo[2], A.hi[2], mn, mx);
-    const double ulo = __builtin_sqrt(mn) * A.c1 - c2 - 2.0;
-    const double uhi = __builtin_sqrt(mx) * A.c1 - c2 + 2.0;
+    // (A negative speed turns the range round.)
+    const double ua = __builtin_sqrt(mn) * A.c1 - c2, ub = __builtin_sqrt(mx) * A.c1 - c2;
+    const double ulo = __builtin_fmin(ua, ub) - 2.0, uhi = __builtin_fmax(ua, ub) + 2.0;
     const int64_t lo = ulo > 0.0 ? (int64_t) __builtin_fmin(ulo, ntd) : 0;
     const int64_t hi = uhi < ntd - 1.0 ? (int64_t) __builtin_fmax(uhi, -1.0) : A.nt - 1;
     const bool use_table = table && q == 1 && __builtin_fabs(d * (A.cp * 1e-6)) * A.gmax <= 300.0;
@@ -609,7 +610,7 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
     // samples each, are more than its nt rows, and is not used with sub-cells.
     // All tables of a call take 8 times kTableBytes at the most.
     const int64_t table = nt * K * (int64_t) sizeof(double2);
-    const bool t = q == 1 && table <= kTableBytes && cells[k] * 16 >= nt &&
+    const bool t = q == 1 && grids[k].step > 0.0 && table <= kTableBytes && cells[k] * 16 >= nt &&
                    table_total + table <= 8 * kTableBytes;
     if (t) table_total += table;
     has_table.push_back(t);
