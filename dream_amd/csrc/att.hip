@@ -650,7 +650,7 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
     DREAM_HIP_CHECK(hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, s));
     const AttGrid *d_grids = (const AttGrid *) (base + o_grids);
     const AttDev *d_probs = (const AttDev *) (base + o_probs);
-    // In launches of up to 32768 grids (the y extent's limit is 65535).
+    // In launches of up to 32768 grids (HIP states 65535 as the y extent's limit).
     for (size_t k = 0; k < grids.size(); k += 32768) {
       const size_t n = std::min<size_t>(grids.size() - k, 32768);
       hipLaunchKernelGGL(att_grid_kernel,

@@ -199,12 +199,13 @@ def test_many_intervals_in_one_call(gpu, n, nt, points, pick):
 
 @pytest.mark.parametrize("alpha", [1.0, 5.0])
 def test_negative_speed_as_the_oracle(gpu, oracle, alpha):
-    """A negative speed turns delays and samples round; no value is refused."""
+    """A negative speed turns delays and samples round; no value is refused.
+    The element's distances span some fifty samples."""
     from dream_amd.dreamrect import dreamrect
-    Ro = np.array([[0.0, 0.0, 10.0], [0.4, 0.2, 12.0]])
-    d = -Ro[:, 2] * 1000.0 / CP - 4.0
-    H = dreamrect(Ro, [1.0, 2.0], [0.1, 0.1, 0.05, 160], d, [1.0, -CP, alpha], "ignore")
-    ref, _, _ = oracle.dreamrect(Ro, 1.0, 2.0, 0.1, 0.1, 0.05, 160, d, 1.0, -CP,
+    Ro = np.array([[0.0, 0.0, 5.0], [0.4, 0.2, 6.0]])
+    d = -Ro[:, 2] * 1000.0 / CP - 1.6
+    H = dreamrect(Ro, [1.0, 6.0], [0.1, 0.1, 0.01, 200], d, [1.0, -CP, alpha], "ignore")
+    ref, _, _ = oracle.dreamrect(Ro, 1.0, 6.0, 0.1, 0.1, 0.01, 200, d, 1.0, -CP,
                                  err_level="ignore", nthreads=2, alpha=alpha)
     assert np.abs(ref).max() > 0
     assert _close(H, ref)
