@@ -12,6 +12,7 @@
 
 #include "conv.hpp"
 #include "das.hpp"
+#include "scratch.hpp"
 #include "sir.hpp"
 #include "tune.hpp"
 
@@ -86,48 +87,58 @@ hipStream_t lib_stream()
 }
 
 namespace {
-struct Scratch {
-  int device = -1;
-  void *p[SCRATCH_USES] = {};
-  size_t bytes[SCRATCH_USES] = {};
-  void drop(int k)
+struct DeviceMemory {
+  static int current()
   {
-    if (p[k]) (void) hipFree(p[k]);
-    p[k] = nullptr;
-    bytes[k] = 0;
+    int dev = 0;
+    DREAM_HIP_CHECK(hipGetDevice(&dev));
+    return dev;
   }
-  void drop_all() { for (int k = 0; k < SCRATCH_USES; k++) drop(k); }
-  ~Scratch() { drop_all(); }
+  static bool alloc(void **p, size_t bytes)
+  {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void) hipGetLastError();
+    return false;
+  }
+  static void release(void *p) { (void) hipFree(p); }
 };
-thread_local Scratch t_scratch;
+using Pool = ScratchPool<DeviceMemory, SCRATCH_USES>;
+// Never destroyed: threads may end after the library's static objects.
+Pool &pool()
+{
+  static Pool *p = new Pool;
+  return *p;
+}
+struct ThreadScratch : Pool::Thread {
+  ThreadScratch() { pool().join(*this); }
+  ~ThreadScratch() { pool().leave(*this); }
+};
+thread_local ThreadScratch t_scratch;
 } // namespace
 
-void *scratch_get(ScratchUse use, size_t bytes)
+void *ScratchHold::get(size_t bytes)
 {
-  Scratch &t = t_scratch;
-  int dev = 0;
-  DREAM_HIP_CHECK(hipGetDevice(&dev));
-  if (t.device != dev) {
-    t.drop_all();
-    t.device = dev;
-  }
-  bytes = std::max<size_t>(bytes, 1);
-  if (t.bytes[use] >= bytes) return t.p[use];
-  t.drop(use);
-  const size_t want = (bytes + 65535) / 65536 * 65536;
-  if (hipMalloc(&t.p[use], want) != hipSuccess) {
-    (void) hipGetLastError();
-    t.p[use] = nullptr;
-    throw Error(DREAM_HIP_ENOMEM, "device allocation failed");
-  }
-  t.bytes[use] = want;
-  return t.p[use];
+  void *p = pool().get(t_scratch, use_, bytes);
+  if (!p) throw Error(DREAM_HIP_ENOMEM, "device allocation failed");
+  held_ = true;
+  return p;
 }
 
-void scratch_done(ScratchUse use)
+ScratchHold::~ScratchHold()
 {
-  if (t_scratch.bytes[use] > kScratchKeep) t_scratch.drop(use);
+  if (!held_) return;
+  // A call that failed may leave work on its stream, and the scratch is the
+  // next call's.
+  if (wait_) (void) hipStreamSynchronize(stream_);
+  pool().done(t_scratch, use_, kScratchKeep);
 }
+
+hipError_t device_malloc(void **p, size_t bytes)
+{
+  return pool().alloc(p, bytes) ? hipSuccess : hipErrorOutOfMemory;
+}
+
+bool device_make_room() { return pool().make_room(); }
 
 template <class F>
 int guarded(F f)
@@ -154,12 +165,12 @@ struct DevBuf {
   DevBuf(const void *src, size_t bytes, hipStream_t s)
   {
     if (!bytes) return;
-    if (hipMalloc(&p, bytes) != hipSuccess) throw Error(DREAM_HIP_ENOMEM, "device allocation failed");
+    if (device_malloc(&p, bytes) != hipSuccess) throw Error(DREAM_HIP_ENOMEM, "device allocation failed");
     DREAM_HIP_CHECK(hipMemcpyAsync(p, src, bytes, hipMemcpyHostToDevice, s));
   }
   explicit DevBuf(size_t bytes)
   {
-    if (bytes && hipMalloc(&p, bytes) != hipSuccess)
+    if (bytes && device_malloc(&p, bytes) != hipSuccess)
       throw Error(DREAM_HIP_ENOMEM, "device allocation failed");
   }
   ~DevBuf() { if (p) (void) hipFree(p); }

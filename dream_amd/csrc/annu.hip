@@ -137,68 +137,64 @@ void run_arr_annu(const AnnuProblem &a, int out_dtype, hipStream_t s, int *sir_e
   // Disc responses: one SIR problem per radius (disc 0 skipped when it has
   // no area, as the reference leaves it zero).
   const size_t slot = (size_t) a.No * (size_t) a.nt;
-  double *disc = (double *) scratch_get(SCRATCH_DISCS, slot * (size_t) R * sizeof(double) +
-                                                           sizeof(AnnuRing) * (size_t) rings);
+  ScratchHold scratch(SCRATCH_DISCS);
+  double *disc = (double *) scratch.get(slot * (size_t) R * sizeof(double) +
+                                        sizeof(AnnuRing) * (size_t) rings);
   AnnuRing *d_tab = (AnnuRing *) (disc + slot * (size_t) R);
-  try {
-    DREAM_HIP_CHECK(hipMemcpyAsync(d_tab, tab.data(), sizeof(AnnuRing) * (size_t) rings,
-                                   hipMemcpyHostToDevice, s));
-    const double G0[3] = {0.0, 0.0, 0.0};
-    std::vector<SirProblem> probs;
-    for (int64_t k = 0; k < R; k++) {
-      if (k == 0 && skip0) continue;
-      SirProblem p;
-      p.Ro = a.Ro;  p.No = a.No;
-      p.shape = SIR_CIRC;  p.R = a.Gr[k];
-      p.dx = a.dx;  p.dy = a.dy;  p.dt = a.dt;  p.nt = a.nt;
-      p.delay_type = a.delay_type;  p.delay = a.delay;
-      p.v = a.v;  p.cp = a.cp;
-      p.G.assign(G0, G0 + 3);
-      p.foc_met = 0;  p.focal.assign(1, 0.0);
-      p.err_level = a.err_level;
-      p.h = disc + (size_t) k * slot;
-      probs.push_back(p);
-    }
-    int code = E_NONE;
-    int64_t oob = 0;
-    if (!probs.empty()) {
-      std::vector<int32_t> codes(probs.size());
-      std::vector<int64_t> oobs(probs.size());
-      if (a.alpha > 2.220446049250313e-16) {
-        run_sir_att(probs, a.alpha, DREAM_HIP_F64, s, codes.data(), oobs.data());
-      } else {
-        SirPlan plan(probs, DREAM_HIP_F64, true, s);
-        plan.run(s, false);
-        plan.status(codes.data(), oobs.data());   // synchronises `s`
-      }
-      // A point's status is its last disc's; a stop ends the call at once.
-      for (size_t q = 0; q < probs.size(); q++) {
-        oob += oobs[q];
-        if (codes[q] == E_OOB) code = E_OOB;
-      }
-      if (code != E_OOB) code = codes.back();   // the last disc is radius R - 1
-    }
-    if (code != E_OOB) {
-      const int64_t total = a.No * a.nt;
-      const int64_t blocks = (total + kCombineThreads - 1) / kCombineThreads;
-      require(blocks <= 0x7fffffffLL, "dream_arr_annu: problem too large");
-      if (out_dtype == DREAM_HIP_F64)
-        annu_combine_kernel<double><<<(unsigned) blocks, kCombineThreads, 0, s>>>(
-            disc, a.nt, a.No, (int) rings, d_tab, (double *) a.h);
-      else
-        annu_combine_kernel<float><<<(unsigned) blocks, kCombineThreads, 0, s>>>(
-            disc, a.nt, a.No, (int) rings, d_tab, (float *) a.h);
-      DREAM_HIP_CHECK(hipGetLastError());
-    }
-    DREAM_HIP_CHECK(hipStreamSynchronize(s));
-    if (sir_err) *sir_err = code;
-    if (oob_count) *oob_count = oob;
-  } catch (...) {
-    (void) hipStreamSynchronize(s);
-    scratch_done(SCRATCH_DISCS);
-    throw;
+  scratch.pending(s);
+  DREAM_HIP_CHECK(hipMemcpyAsync(d_tab, tab.data(), sizeof(AnnuRing) * (size_t) rings,
+                                 hipMemcpyHostToDevice, s));
+  const double G0[3] = {0.0, 0.0, 0.0};
+  std::vector<SirProblem> probs;
+  for (int64_t k = 0; k < R; k++) {
+    if (k == 0 && skip0) continue;
+    SirProblem p;
+    p.Ro = a.Ro;  p.No = a.No;
+    p.shape = SIR_CIRC;  p.R = a.Gr[k];
+    p.dx = a.dx;  p.dy = a.dy;  p.dt = a.dt;  p.nt = a.nt;
+    p.delay_type = a.delay_type;  p.delay = a.delay;
+    p.v = a.v;  p.cp = a.cp;
+    p.G.assign(G0, G0 + 3);
+    p.foc_met = 0;  p.focal.assign(1, 0.0);
+    p.err_level = a.err_level;
+    p.h = disc + (size_t) k * slot;
+    probs.push_back(p);
   }
-  scratch_done(SCRATCH_DISCS);
+  int code = E_NONE;
+  int64_t oob = 0;
+  if (!probs.empty()) {
+    std::vector<int32_t> codes(probs.size());
+    std::vector<int64_t> oobs(probs.size());
+    if (a.alpha > 2.220446049250313e-16) {
+      run_sir_att(probs, a.alpha, DREAM_HIP_F64, s, codes.data(), oobs.data());
+    } else {
+      SirPlan plan(probs, DREAM_HIP_F64, true, s);
+      plan.run(s, false);
+      plan.status(codes.data(), oobs.data());   // synchronises `s`
+    }
+    // A point's status is its last disc's; a stop ends the call at once.
+    for (size_t q = 0; q < probs.size(); q++) {
+      oob += oobs[q];
+      if (codes[q] == E_OOB) code = E_OOB;
+    }
+    if (code != E_OOB) code = codes.back();   // the last disc is radius R - 1
+  }
+  if (code != E_OOB) {
+    const int64_t total = a.No * a.nt;
+    const int64_t blocks = (total + kCombineThreads - 1) / kCombineThreads;
+    require(blocks <= 0x7fffffffLL, "dream_arr_annu: problem too large");
+    if (out_dtype == DREAM_HIP_F64)
+      annu_combine_kernel<double><<<(unsigned) blocks, kCombineThreads, 0, s>>>(
+          disc, a.nt, a.No, (int) rings, d_tab, (double *) a.h);
+    else
+      annu_combine_kernel<float><<<(unsigned) blocks, kCombineThreads, 0, s>>>(
+          disc, a.nt, a.No, (int) rings, d_tab, (float *) a.h);
+    DREAM_HIP_CHECK(hipGetLastError());
+  }
+  DREAM_HIP_CHECK(hipStreamSynchronize(s));
+  scratch.settled();
+  if (sir_err) *sir_err = code;
+  if (oob_count) *oob_count = oob;
 }
 
 } // namespace dream

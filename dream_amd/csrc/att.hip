@@ -624,76 +624,72 @@ void run_sir_att(const std::vector<SirProblem> &problems, double alpha_db, int o
   const size_t table_bytes = tables.size() * sizeof(double);
   const bool apart = table_bytes > 65536;
   std::vector<char> host(apart ? o_tables : copied);
-  char *base = (char *) scratch_get(SCRATCH_ATT, bytes);
-  try {
-    Status *d_status = (Status *) (base + o_status);
-    for (size_t k = 0; k < grids.size(); k++) {
-      grids[k].gam = (double2 *) (base + o_gam[k]);
-      grids[k].tw = (double2 *) (base + o_tw[k]);
-      if (has_table[k]) grids[k].table = (double2 *) (base + o_table[k]);
-    }
-    for (size_t i = 0; i < P; i++) {
-      AttDev &d = dev_p[i];
-      d.sub = (const double *) (base + o_tables) + off_sub[i];
-      d.el = (const double *) (base + o_tables) + off_el[i];
-      d.grid = grids[grid_of[i]];
-      d.spec = (double2 *) (base + o_spec) + spec_off[i];
-      d.status = d_status + i;
-    }
-    std::memcpy(host.data() + o_grids, grids.data(), grids.size() * sizeof(AttGrid));
-    std::memcpy(host.data() + o_probs, dev_p.data(), P * sizeof(AttDev));
-    if (apart)
-      DREAM_HIP_CHECK(hipMemcpyAsync(base + o_tables, tables.data(), table_bytes,
-                                     hipMemcpyHostToDevice, s));
-    else if (table_bytes)
-      std::memcpy(host.data() + o_tables, tables.data(), table_bytes);
-    DREAM_HIP_CHECK(hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, s));
-    const AttGrid *d_grids = (const AttGrid *) (base + o_grids);
-    const AttDev *d_probs = (const AttDev *) (base + o_probs);
-    // In launches of up to 32768 grids (HIP states 65535 as the y extent's limit).
-    for (size_t k = 0; k < grids.size(); k += 32768) {
-      const size_t n = std::min<size_t>(grids.size() - k, 32768);
-      hipLaunchKernelGGL(att_grid_kernel,
-                         dim3((unsigned) std::min<int64_t>((grid_work + kThreads - 1) / kThreads, 4096),
-                              (unsigned) n),
-                         dim3(kThreads), 0, s, d_grids + k, d_status, k == 0 ? (int) P : 0);
-      DREAM_HIP_CHECK(hipGetLastError());
-    }
-    if (items > 0) {
-      if (terms == 8)
-        hipLaunchKernelGGL(att_spectrum_kernel<8>, dim3((unsigned) items), dim3(kThreads), lds, s,
-                           d_probs, (int) P);
-      else
-        hipLaunchKernelGGL(att_spectrum_kernel<12>, dim3((unsigned) items), dim3(kThreads), lds, s,
-                           d_probs, (int) P);
-      DREAM_HIP_CHECK(hipGetLastError());
-    }
-    if (outs > 0) {
-      hipLaunchKernelGGL(att_c2r_kernel, dim3((unsigned) outs), dim3(kThreads), 0, s, d_probs,
-                         (int) P);
-      DREAM_HIP_CHECK(hipGetLastError());
-    }
-    std::vector<Status> st(P);
-    DREAM_HIP_CHECK(hipMemcpyAsync(st.data(), d_status, P * sizeof(Status),
-                                   hipMemcpyDeviceToHost, s));
-    DREAM_HIP_CHECK(hipStreamSynchronize(s));
-    for (size_t i = 0; i < P; i++) {
-      const int lv = problems[i].err_level;
-      int code = E_NONE;
-      if (lv == L_STOP || lv == L_PSTOP) {
-        if (st[i].any_oob) code = E_OOB;
-      } else if (st[i].last_elem_oob) {
-        code = level_code(lv);
-      }
-      if (codes) codes[i] = code;
-      if (oobs) oobs[i] = (int64_t) st[i].oob;
-    }
-  } catch (...) {
-    (void) hipStreamSynchronize(s);
-    scratch_done(SCRATCH_ATT);
-    throw;
+  std::vector<Status> st(P);
+  ScratchHold scratch(SCRATCH_ATT);
+  char *base = (char *) scratch.get(bytes);
+  scratch.pending(s);
+  Status *d_status = (Status *) (base + o_status);
+  for (size_t k = 0; k < grids.size(); k++) {
+    grids[k].gam = (double2 *) (base + o_gam[k]);
+    grids[k].tw = (double2 *) (base + o_tw[k]);
+    if (has_table[k]) grids[k].table = (double2 *) (base + o_table[k]);
   }
-  scratch_done(SCRATCH_ATT);
+  for (size_t i = 0; i < P; i++) {
+    AttDev &d = dev_p[i];
+    d.sub = (const double *) (base + o_tables) + off_sub[i];
+    d.el = (const double *) (base + o_tables) + off_el[i];
+    d.grid = grids[grid_of[i]];
+    d.spec = (double2 *) (base + o_spec) + spec_off[i];
+    d.status = d_status + i;
+  }
+  std::memcpy(host.data() + o_grids, grids.data(), grids.size() * sizeof(AttGrid));
+  std::memcpy(host.data() + o_probs, dev_p.data(), P * sizeof(AttDev));
+  if (apart)
+    DREAM_HIP_CHECK(hipMemcpyAsync(base + o_tables, tables.data(), table_bytes,
+                                   hipMemcpyHostToDevice, s));
+  else if (table_bytes)
+    std::memcpy(host.data() + o_tables, tables.data(), table_bytes);
+  DREAM_HIP_CHECK(hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, s));
+  const AttGrid *d_grids = (const AttGrid *) (base + o_grids);
+  const AttDev *d_probs = (const AttDev *) (base + o_probs);
+  // In launches of up to 32768 grids (HIP states 65535 as the y extent's limit).
+  for (size_t k = 0; k < grids.size(); k += 32768) {
+    const size_t n = std::min<size_t>(grids.size() - k, 32768);
+    hipLaunchKernelGGL(att_grid_kernel,
+                       dim3((unsigned) std::min<int64_t>((grid_work + kThreads - 1) / kThreads, 4096),
+                            (unsigned) n),
+                       dim3(kThreads), 0, s, d_grids + k, d_status, k == 0 ? (int) P : 0);
+    DREAM_HIP_CHECK(hipGetLastError());
+  }
+  if (items > 0) {
+    if (terms == 8)
+      hipLaunchKernelGGL(att_spectrum_kernel<8>, dim3((unsigned) items), dim3(kThreads), lds, s,
+                         d_probs, (int) P);
+    else
+      hipLaunchKernelGGL(att_spectrum_kernel<12>, dim3((unsigned) items), dim3(kThreads), lds, s,
+                         d_probs, (int) P);
+    DREAM_HIP_CHECK(hipGetLastError());
+  }
+  if (outs > 0) {
+    hipLaunchKernelGGL(att_c2r_kernel, dim3((unsigned) outs), dim3(kThreads), 0, s, d_probs,
+                       (int) P);
+    DREAM_HIP_CHECK(hipGetLastError());
+  }
+  DREAM_HIP_CHECK(hipMemcpyAsync(st.data(), d_status, P * sizeof(Status),
+                                 hipMemcpyDeviceToHost, s));
+  DREAM_HIP_CHECK(hipStreamSynchronize(s));
+  scratch.settled();
+  for (size_t i = 0; i < P; i++) {
+    const int lv = problems[i].err_level;
+    int code = E_NONE;
+    if (lv == L_STOP || lv == L_PSTOP) {
+      if (st[i].any_oob) code = E_OOB;
+    } else if (st[i].last_elem_oob) {
+      code = level_code(lv);
+    }
+    if (codes) codes[i] = code;
+    if (oobs) oobs[i] = (int64_t) st[i].oob;
+  }
 }
 
 } // namespace dream

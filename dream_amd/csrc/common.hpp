@@ -89,17 +89,37 @@ private:
 // priority).
 hipStream_t lib_stream();
 
-// Device scratch that a thread keeps between calls, for calls that
-// synchronise their stream before they return: one buffer per use, grown on
-// demand, kept up to kScratchKeep bytes (larger ones are freed by
-// scratch_done), given back when the thread ends, when it moves to another
-// device, or when an allocation fails.  A thread has at most one call at a
-// time, so a use has one user.  hipFree of an 88 MB buffer took 250 us, four
-// small allocations with their copies and frees 40 us of an 87 us call.
+// Device scratch that a thread keeps between calls (scratch.hpp), for calls
+// that synchronise their stream before they return: one buffer per use, grown
+// on demand, kept up to kScratchKeep bytes.  hipFree of an 88 MB buffer took 250
+// us, four small allocations with their copies and frees 40 us of an 87 us call.
 enum ScratchUse { SCRATCH_PLAN = 0, SCRATCH_DISCS, SCRATCH_ATT, SCRATCH_USES };
 constexpr size_t kScratchKeep = (size_t) 128 << 20;
-void *scratch_get(ScratchUse use, size_t bytes);
-void scratch_done(ScratchUse use);
+
+// A call's hold on its thread's scratch: from get to the end of its life,
+// when the stream it names is waited for first.
+class ScratchHold {
+public:
+  explicit ScratchHold(ScratchUse use) : use_(use) {}
+  ~ScratchHold();
+  ScratchHold(const ScratchHold &) = delete;
+  ScratchHold &operator=(const ScratchHold &) = delete;
+  void *get(size_t bytes);                 // throws DREAM_HIP_ENOMEM
+  void pending(hipStream_t s) { wait_ = true; stream_ = s; }
+  void settled() { wait_ = false; }        // the stream has been waited for
+
+private:
+  ScratchUse use_;
+  bool held_ = false, wait_ = false;
+  hipStream_t stream_ = nullptr;
+};
+
+// hipMalloc that has idle scratch given back before it fails.
+hipError_t device_malloc(void **p, size_t bytes);
+template <typename T>
+hipError_t device_malloc(T **p, size_t bytes) { return device_malloc((void **) p, bytes); }
+// After another allocation failed: whether scratch was given back.
+bool device_make_room();
 
 // ------------------------------------------------------------------ device
 

@@ -561,7 +561,7 @@ const Cx<T> *twiddles()
         }
     }
     void *d = nullptr;
-    DREAM_HIP_CHECK(hipMalloc(&d, h.size() * sizeof(Cx<T>)));
+    DREAM_HIP_CHECK(device_malloc(&d, h.size() * sizeof(Cx<T>)));
     DREAM_HIP_CHECK(hipMemcpy(d, h.data(), h.size() * sizeof(Cx<T>), hipMemcpyHostToDevice));
     p = d;
   }
@@ -613,7 +613,13 @@ void launch_conv_fft(T *Y, const T *A, int64_t MA, int64_t N, int64_t L, int64_t
   }
   // The layers' filter spectra, stream-ordered scratch.
   Cx<T> *F = nullptr;
-  DREAM_HIP_CHECK(hipMallocAsync((void **) &F, (size_t) L * X::N * sizeof(Cx<T>), s));
+  const size_t bytes = (size_t) L * X::N * sizeof(Cx<T>);
+  hipError_t got = hipMallocAsync((void **) &F, bytes, s);
+  if (got == hipErrorOutOfMemory && device_make_room()) {
+    (void) hipGetLastError();
+    got = hipMallocAsync((void **) &F, bytes, s);
+  }
+  DREAM_HIP_CHECK(got);
   hipLaunchKernelGGL((fft_filter_kernel<T, LG>), dim3((unsigned) L), block, X::kLds, s, B, MB,
                      b_layer, tw, F);
   hipLaunchKernelGGL((conv_fft_kernel<T, LG, FFT_LAYERS>), dim3((unsigned) pairs), block, X::kLds,

@@ -2198,7 +2198,7 @@ DasHandle::DasHandle(int type, int64_t K, int64_t No, int64_t Lt, int64_t Lr, in
     require(rca_extents_in_bounds(Lt, Lr),
           "das: RCA stripe extents are read at rows[Lt .. 2 Lt - 1] and columns[Lr - 1] "
           "(extra_src/das.cc:464-467); need 2 Lt <= 3 Lr and Lr <= 3 Lt");
-  DREAM_HIP_CHECK(hipMalloc(&d_status_, sizeof(Status)));
+  DREAM_HIP_CHECK(device_malloc(&d_status_, sizeof(Status)));
   DREAM_HIP_CHECK(hipMemset(d_status_, 0, sizeof(Status)));
   DREAM_HIP_CHECK(hipHostMalloc(&h_status_, sizeof(Status)));
 }
@@ -2260,7 +2260,7 @@ void DasHandle::ensure_scratch(size_t bytes)
   (void) hipFree(d_scratch_);
   d_scratch_ = nullptr;
   d_scratch_bytes_ = 0;
-  if (hipMalloc(&d_scratch_, bytes) != hipSuccess)
+  if (device_malloc(&d_scratch_, bytes) != hipSuccess)
     throw Error(DREAM_HIP_ENOMEM, "das: device allocation failed (partial sums)");
   d_scratch_bytes_ = bytes;
 }
@@ -2279,7 +2279,7 @@ void DasHandle::set_pixel_order(const int32_t *perm, int64_t n)
             "das: the pixel order must be a permutation of 0..No-1");
     seen[(size_t) perm[q]] = 1;
   }
-  if (!d_perm_) DREAM_HIP_CHECK(hipMalloc(&d_perm_, (size_t) std::max<int64_t>(No_, 1) * 4));
+  if (!d_perm_) DREAM_HIP_CHECK(device_malloc(&d_perm_, (size_t) std::max<int64_t>(No_, 1) * 4));
   if (n) DREAM_HIP_CHECK(hipMemcpy(d_perm_, perm, (size_t) n * 4, hipMemcpyHostToDevice));
 }
 
@@ -2340,7 +2340,7 @@ void DasHandle::group_frames(DasArgs &a, const void *Y, int64_t y_stride, int64_
     (void) hipFree(d_grp_);
     d_grp_ = nullptr;
     d_grp_bytes_ = 0;
-    if (hipMalloc(&d_grp_, bytes) == hipSuccess) d_grp_bytes_ = bytes;
+    if (device_malloc(&d_grp_, bytes) == hipSuccess) d_grp_bytes_ = bytes;
     else (void) hipGetLastError();
   }
   if (!d_grp_) return;
@@ -2396,7 +2396,7 @@ int DasHandle::run_dev(const void *Y, const void *Ro, const void *Gt, const void
       (void) hipFree(d_sym_);
       d_sym_ = nullptr;
       d_sym_bytes_ = 0;
-      if (hipMalloc(&d_sym_, bytes) != hipSuccess)
+      if (device_malloc(&d_sym_, bytes) != hipSuccess)
         throw Error(DREAM_HIP_ENOMEM, "das: device allocation failed (symmetrized A-scans)");
       d_sym_bytes_ = bytes;
     }
@@ -2456,7 +2456,7 @@ int DasHandle::run_host(const void *Y, const void *Ro, const void *Gt, const voi
     (void) hipFree(d_buf_);
     d_buf_ = nullptr;
     d_buf_bytes_ = 0;
-    if (hipMalloc(&d_buf_, total) != hipSuccess)
+    if (device_malloc(&d_buf_, total) != hipSuccess)
       throw Error(DREAM_HIP_ENOMEM, "das: device allocation failed");
     d_buf_bytes_ = total;
   }
@@ -2537,7 +2537,7 @@ void DasHandle::adjoint_dev(const void *Y, const void *Ro, const void *Gt, const
       (void) hipFree(d_z_);
       d_z_ = nullptr;
       d_z_bytes_ = 0;
-      if (hipMalloc(&d_z_, zbytes) != hipSuccess)
+      if (device_malloc(&d_z_, zbytes) != hipSuccess)
         throw Error(DREAM_HIP_ENOMEM, "das adjoint: device allocation failed");
       d_z_bytes_ = zbytes;
     }
@@ -2659,7 +2659,7 @@ DasUni::DasUni(int type, int64_t K, const double gt[3], const double gr[3], cons
   if (f) uni_tables<float>(type, gt, gr, Lt_, Lr_, tabs);
   else uni_tables<double>(type, gt, gr, Lt_, Lr_, tabs);
   const size_t ro_bytes = (size_t) No_ * 3 * gs_;
-  DREAM_HIP_CHECK(hipMalloc(&d_geom_, ro_bytes + tabs.size() + 16));
+  DREAM_HIP_CHECK(device_malloc(&d_geom_, ro_bytes + tabs.size() + 16));
   char *base = (char *) d_geom_;
   DREAM_HIP_CHECK(hipMemcpy(base + ro_bytes, tabs.data(), tabs.size(), hipMemcpyHostToDevice));
   const int blocks = (int) ((No_ + 255) / 256);
@@ -2756,7 +2756,7 @@ void DasUni::run_host(const void *Y, double dt, double delay, double cp, void *I
     (void) hipFree(d_buf_);
     d_buf_ = nullptr;
     d_buf_bytes_ = 0;
-    if (hipMalloc(&d_buf_, total) != hipSuccess)
+    if (device_malloc(&d_buf_, total) != hipSuccess)
       throw Error(DREAM_HIP_ENOMEM, "das_uni: device allocation failed");
     d_buf_bytes_ = total;
   }
@@ -2840,10 +2840,10 @@ DasBatch::DasBatch(const DreamDasProblem *probs, int32_t n, int type, int precis
   n_probs_ = (int32_t) sorted.size();
   n_items_ = item;
   const size_t nb = std::max<size_t>(sorted.size(), 1);
-  DREAM_HIP_CHECK(hipMalloc(&d_args_, nb * sizeof(DasArgs)));
-  DREAM_HIP_CHECK(hipMalloc(&d_begin_, nb * sizeof(int64_t)));
-  DREAM_HIP_CHECK(hipMalloc(&d_delay_, nb * sizeof(double)));
-  DREAM_HIP_CHECK(hipMalloc(&d_counter_, 2 * sizeof(unsigned long long)));
+  DREAM_HIP_CHECK(device_malloc(&d_args_, nb * sizeof(DasArgs)));
+  DREAM_HIP_CHECK(device_malloc(&d_begin_, nb * sizeof(int64_t)));
+  DREAM_HIP_CHECK(device_malloc(&d_delay_, nb * sizeof(double)));
+  DREAM_HIP_CHECK(device_malloc(&d_counter_, 2 * sizeof(unsigned long long)));
   DREAM_HIP_CHECK(hipMemset(d_counter_, 0, 2 * sizeof(unsigned long long)));
   // Scalar delays in the geometry type (float for the reference-float path).
   if (gs == 8) {

@@ -1139,9 +1139,9 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
   static_assert(sizeof(SirDev) % 8 == 0 && sizeof(Status) % 8 == 0, "plan buffer alignment");
   char *base;
   if (one_shot_) {
-    base = (char *) scratch_get(SCRATCH_PLAN, bytes);
+    base = (char *) scratch_.get(bytes);
   } else {
-    DREAM_HIP_CHECK(hipMalloc(&d_base_, bytes));
+    DREAM_HIP_CHECK(device_malloc(&d_base_, bytes));
     base = (char *) d_base_;
   }
   d_probs_ = (SirDev *) base;
@@ -1198,7 +1198,7 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
   if (one_shot_) {
     last_stream_ = stream;
     DREAM_HIP_CHECK(hipMemcpyAsync(base, image_.data(), bytes, hipMemcpyHostToDevice, stream));
-    pending_ = true;
+    scratch_.pending(stream);
   } else {
     const hipError_t e = hipMemcpy(base, image_.data(), bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) (void) hipFree(d_base_);
@@ -1228,12 +1228,6 @@ SirPlan::SirPlan(const std::vector<SirProblem> &problems, int out_dtype, bool on
 SirPlan::~SirPlan()
 {
   if (graph_) (void) hipGraphExecDestroy(graph_);
-  // A call that failed may leave work on its stream, and the scratch is the
-  // next call's.
-  if (one_shot_) {
-    if (pending_) (void) hipStreamSynchronize(last_stream_);
-    scratch_done(SCRATCH_PLAN);
-  }
   if (d_base_) (void) hipFree(d_base_);
 }
 
@@ -1363,7 +1357,7 @@ void SirPlan::status(int32_t *codes, int64_t *oob)
     if (P)
       DREAM_HIP_CHECK(hipMemcpy(st.data(), d_status_, P * sizeof(Status), hipMemcpyDeviceToHost));
   }
-  pending_ = false;
+  scratch_.settled();
   for (size_t i = 0; i < P; i++) {
     const int lv = levels_[i];
     int code = E_NONE;
@@ -1381,7 +1375,7 @@ void rsq_seed(const double *s, int64_t n, double *y)
 {
   if (n <= 0) return;
   double *d = nullptr;
-  DREAM_HIP_CHECK(hipMalloc(&d, 2 * (size_t) n * sizeof(double)));
+  DREAM_HIP_CHECK(device_malloc(&d, 2 * (size_t) n * sizeof(double)));
   DREAM_HIP_CHECK(hipMemcpy(d, s, (size_t) n * sizeof(double), hipMemcpyHostToDevice));
   const int blocks = (int) ((n + 255) / 256);
   hipLaunchKernelGGL(rsq_seed_kernel, dim3(blocks), dim3(256), 0, lib_stream(), d, n, d + n);
@@ -1402,8 +1396,8 @@ void rect_indices(double xo, double yo, double zo, double a, double b, double dx
   if (m <= 0) return;
   double *d_xy = nullptr;
   int64_t *d_it = nullptr;
-  DREAM_HIP_CHECK(hipMalloc(&d_xy, (xs.size() + ys.size()) * sizeof(double)));
-  DREAM_HIP_CHECK(hipMalloc(&d_it, (size_t) m * sizeof(int64_t)));
+  DREAM_HIP_CHECK(device_malloc(&d_xy, (xs.size() + ys.size()) * sizeof(double)));
+  DREAM_HIP_CHECK(device_malloc(&d_it, (size_t) m * sizeof(int64_t)));
   DREAM_HIP_CHECK(hipMemcpy(d_xy, xs.data(), xs.size() * sizeof(double), hipMemcpyHostToDevice));
   DREAM_HIP_CHECK(hipMemcpy(d_xy + xs.size(), ys.data(), ys.size() * sizeof(double),
                             hipMemcpyHostToDevice));

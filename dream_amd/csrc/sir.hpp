@@ -136,9 +136,9 @@ private:
   std::vector<void *> zero_ptr_;
   bool one_shot_ = false;
   bool fresh_ = true;                       // not launched yet
-  bool pending_ = false;                    // a one-shot plan's stream is not yet waited for
   std::vector<char> image_;                 // the upload, kept while it may be read
-  void *d_base_ = nullptr;                  // the buffer, if the plan owns one
+  ScratchHold scratch_{SCRATCH_PLAN};       // the buffer of a one-shot plan
+  void *d_base_ = nullptr;                  // of a kept one
   SirDev *d_probs_ = nullptr;
   double *d_tables_ = nullptr;
   Status *d_status_ = nullptr;
