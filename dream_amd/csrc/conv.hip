@@ -6,9 +6,10 @@
 // linear convolutions computed by the reference through zero-padded FFTs of
 // length M_A + M_B - 1; the result is the same sum
 //     y[k] = sum_l sum_i b_l[i] a_l[k - i],   k = 0 .. M_A + M_B - 2,
-// which is evaluated here directly in the data type (no FFT round trip).
+// taken directly in the data type for short filters, through transforms for
+// long ones (the FFT path below).
 //
-// Mapping.  One work-group per (output column, tile of kTile outputs).  The
+// Mapping of the direct sum.  One work-group per (output column, tile of kTile outputs).  The
 // filter b is consumed in chunks of kChunk taps; for each chunk the taps and
 // the window of a they meet are staged in LDS, and each thread accumulates
 // kR outputs spaced kThreads apart, so consecutive lanes read consecutive
@@ -500,18 +501,38 @@ int max_lds_bytes()
   return bytes;
 }
 
-// Transform lengths built: 2^10 .. 2^14 FP32, .. 2^13 FP64; shorter outputs
-// are padded to 2^10.
+// Transform lengths: 2^10 .. 2^14 FP32, .. 2^13 FP64, half the longest with
+// layers, a quarter with filters per column; shorter outputs are padded to
+// 2^10, longer ones summed directly.  (These limits -- one, two or three arrays
+// of points in 160 KiB -- are the radix-2 kernels' of before; the sums and second
+// spectra are in registers now, so longer transforms would fit, but a call's
+// rounding would change with its route.)  The rule and the launches share
+// them, so what is chosen is built.
 constexpr int kMinLog = 10;
 template <typename T>
 constexpr int kMaxLog = sizeof(T) == 4 ? 14 : 13;
+template <typename T>
+constexpr bool fft_length(int lg, int kind)
+{
+  return lg >= kMinLog && lg <= kMaxLog<T> && ((size_t) (kind + 1) << lg) * sizeof(Cx<T>) <= 160 * 1024;
+}
+// LDS a transform's work-group asks for: an array of points, two with filters
+// per column, each padded by one point in 16.
+template <typename T>
+size_t fft_lds(int lg, int kind)
+{
+  const size_t points = (size_t) 1 << lg;
+  return (kind == FFT_COLUMNS ? 2 : 1) * (points + points / 16) * sizeof(Cx<T>);
+}
 
 // DREAM_HIP_CONV = direct | fft forces a path (for comparisons and tests);
-// otherwise the FFT path is taken when it fits in LDS and the direct sum
-// would cost several times more arithmetic.  Returns log2 of the transform's
-// length, 0 for the direct sum.  The choice is by arithmetic, not by the
-// paths' measured times: a transform's rounding errors are relative to the
-// column's largest sample, the direct sum's to each output's own terms.
+// otherwise the FFT path is taken when its length is built and the direct sum
+// would cost more than four times its arithmetic.  Returns log2 of the
+// transform's length, 0 for the direct sum.  The ratio was set for radix-2
+// passes through LDS and kept: the transforms are about four times faster now,
+// but a transform's rounding errors are relative to the column's largest
+// sample, the direct sum's to each output's own terms, so moving the line
+// would change the results of calls on it.
 template <typename T>
 int fft_log_if_chosen(int64_t MA, int64_t MB, int64_t L, bool per_col)
 {
@@ -523,11 +544,8 @@ int fft_log_if_chosen(int64_t MA, int64_t MB, int64_t L, bool per_col)
   int bits = 1;
   while ((1ll << bits) < MY) bits++;
   const int64_t NF = 1ll << bits;
-  // Longest transform: one, two (layers) or three (filters per column)
-  // complex arrays of it fit in a work-group's LDS.
-  const int bufs = per_col ? 3 : (L > 1 ? 2 : 1);
-  if (bits > kMaxLog<T> || (size_t) bufs * NF * sizeof(Cx<T>) > (size_t) max_lds_bytes()) return 0;
-  const int lg = std::max(bits, kMinLog);
+  const int lg = std::max(bits, kMinLog), kind = per_col ? FFT_COLUMNS : (L > 1 ? FFT_LAYERS : FFT_ONE);
+  if (!fft_length<T>(lg, kind) || fft_lds<T>(lg, kind) > (size_t) max_lds_bytes()) return 0;
   if (force_fft) return lg;
   // Per column: direct 2 MA MB L flops; FFT (two columns per transform)
   // about 5 NF log2 NF per transform, (L + 1) transforms per pair (2 L + 1
@@ -590,15 +608,14 @@ void launch_conv_fft(T *Y, const T *A, int64_t MA, int64_t N, int64_t L, int64_t
   const int64_t pairs = (N + 1) / 2;
   const dim3 block(X::NT);
   if (b_col != 0) {
-    // Longer transforms with per-column filters are not chosen (two arrays of
-    // points beside each other, see fft_log_if_chosen).
-    if constexpr (2 * X::kLds <= 160 * 1024) {
+    if constexpr (fft_length<T>(LG, FFT_COLUMNS)) {
       hipLaunchKernelGGL((conv_fft_kernel<T, LG, FFT_COLUMNS>), dim3((unsigned) pairs), block,
                          2 * X::kLds, s, Y, A, MA, N, L, a_col, a_layer, B, MB, b_col, b_layer,
                          mode, tw, (const Cx<T> *) nullptr);
       DREAM_HIP_CHECK(hipGetLastError());
+      return;
     }
-    return;
+    throw Error(DREAM_HIP_ERUNTIME, "conv: no transform of this length for filters per column");
   }
   if (L == 1) {
     // As many work-groups as the device holds at once, with an equal number
@@ -611,23 +628,27 @@ void launch_conv_fft(T *Y, const T *A, int64_t MA, int64_t N, int64_t L, int64_t
     DREAM_HIP_CHECK(hipGetLastError());
     return;
   }
-  // The layers' filter spectra, stream-ordered scratch.
-  Cx<T> *F = nullptr;
-  const size_t bytes = (size_t) L * X::N * sizeof(Cx<T>);
-  hipError_t got = hipMallocAsync((void **) &F, bytes, s);
-  if (got == hipErrorOutOfMemory && device_make_room()) {
-    (void) hipGetLastError();
-    got = hipMallocAsync((void **) &F, bytes, s);
+  if constexpr (fft_length<T>(LG, FFT_LAYERS)) {
+    // The layers' filter spectra, stream-ordered scratch.
+    Cx<T> *F = nullptr;
+    const size_t bytes = (size_t) L * X::N * sizeof(Cx<T>);
+    hipError_t got = hipMallocAsync((void **) &F, bytes, s);
+    if (got == hipErrorOutOfMemory && device_make_room()) {
+      (void) hipGetLastError();
+      got = hipMallocAsync((void **) &F, bytes, s);
+    }
+    DREAM_HIP_CHECK(got);
+    hipLaunchKernelGGL((fft_filter_kernel<T, LG>), dim3((unsigned) L), block, X::kLds, s, B, MB,
+                       b_layer, tw, F);
+    hipLaunchKernelGGL((conv_fft_kernel<T, LG, FFT_LAYERS>), dim3((unsigned) pairs), block, X::kLds,
+                       s, Y, A, MA, N, L, a_col, a_layer, B, MB, b_col, b_layer, mode, tw,
+                       (const Cx<T> *) F);
+    const hipError_t e = hipGetLastError();
+    (void) hipFreeAsync(F, s);
+    DREAM_HIP_CHECK(e);
+    return;
   }
-  DREAM_HIP_CHECK(got);
-  hipLaunchKernelGGL((fft_filter_kernel<T, LG>), dim3((unsigned) L), block, X::kLds, s, B, MB,
-                     b_layer, tw, F);
-  hipLaunchKernelGGL((conv_fft_kernel<T, LG, FFT_LAYERS>), dim3((unsigned) pairs), block, X::kLds,
-                     s, Y, A, MA, N, L, a_col, a_layer, B, MB, b_col, b_layer, mode, tw,
-                     (const Cx<T> *) F);
-  const hipError_t e = hipGetLastError();
-  (void) hipFreeAsync(F, s);
-  DREAM_HIP_CHECK(e);
+  throw Error(DREAM_HIP_ERUNTIME, "conv: no transform of this length for layers");
 }
 
 } // namespace

@@ -178,3 +178,27 @@ def test_every_transform_length(gpu, conv_path, dtype, logs, tol, kind):
                              torch.tensor(B, dtype=dtype, device="cuda"))
                 err = np.max(np.abs(Y.double().cpu().numpy() - ref)) / np.abs(ref).max()
                 assert err <= tol, (lg, MY, N, kind, err)
+
+
+@pytest.mark.parametrize("dtype,longest,tol", [
+    (torch.float64, {"vec": 13, "layer": 12, "col": 11}, 1e-13),
+    (torch.float32, {"vec": 14, "layer": 13, "col": 12}, 2e-6)])
+@pytest.mark.parametrize("kind", ["vec", "layer", "col"])
+def test_past_the_longest_transform(gpu, conv_path, dtype, longest, tol, kind):
+    """One sample past the longest transform of each kind, the FFT path asked
+    for: every output is written, by the direct sum, to the bars of the lengths
+    that are built."""
+    from dream_amd.torch_ops import conv_sum
+    rng = np.random.default_rng(94)
+    conv_path("fft")
+    MY, MB, N = (1 << longest[kind]) + 1, 70, 3
+    MA, L = MY - MB + 1, 3 if kind == "layer" else 1
+    A = rng.standard_normal((L, N, MA))
+    B = rng.standard_normal({"vec": (MB,), "layer": (L, MB), "col": (N, MB)}[kind])
+    Bf = {"vec": lambda l, n: B, "layer": lambda l, n: B[l], "col": lambda l, n: B[n]}[kind]
+    ref = np.array([sum(np.convolve(A[l, n], Bf(l, n)) for l in range(L)) for n in range(N)])
+    out = torch.full((N, MY), float("nan"), dtype=dtype, device="cuda")
+    Y = conv_sum(torch.tensor(A if L > 1 else A[0], dtype=dtype, device="cuda"),
+                 torch.tensor(B, dtype=dtype, device="cuda"), out=out)
+    err = np.max(np.abs(Y.double().cpu().numpy() - ref)) / np.abs(ref).max()
+    assert err <= tol, (kind, err)
