@@ -37,9 +37,9 @@
 // the direct sum: 64 points x 16 elements x 3600 sub-elements at nt = 400
 // took 3950 us for 7.4e8 of them; the moments take 43 us (147 with an LDS
 // atomic per contribution instead of the lanes' runs), the grid tables 6 and
-// the transform 12, and the call went from 4080 to 178 us.  What bounds it
-// now is the call's set-up on the host; on the device the geometry and the
-// moments' LDS atomics.
+// the transform 12, and the call went from 4060 to 124 us.  What bounds it
+// now is the call on the host (its set-up, one upload, one read-back); on the
+// device the geometry and the moments' LDS atomics, with 1.5 waves per SIMD.
 // A work-group holds at most kBinBlock bins; longer responses split each
 // point's bins over several work-groups (any nt).
 

@@ -113,11 +113,12 @@ conv_sum_kernel(T *__restrict__ Y, const T *__restrict__ A, int64_t MA, int64_t 
 // between passes.  Forward transforms are decimation in frequency (natural
 // order in, digit-reversed out), the product is formed in that order, the
 // inverse is decimation in time: no reordering passes.  What bounds it: the
-// butterflies' FP64/FP32 instructions, about 90 per point and transform at N =
-// 4096, then the exchanges (4 per column pair, 2 N complex each).  Radix-2
-// passes in LDS took 12 reads and writes of the array per transform instead of
-// 2 and were bound by them: a call of 4096 x 2000 by 300 taps FP32 went from
-// 158 to 35 us, 1024 x 2000 by 2000 taps FP64 from 77 to 20 us.
+// butterflies' FP64/FP32 instructions, about 45 per point and transform at N =
+// 4096 (FP32: the VALU busy 55 %), then the exchanges (4 per column pair, 2 N
+// complex each).  Radix-2 passes in LDS took 12 reads and writes of the array
+// per transform instead of 2 and were bound by them: a call of 4096 x 2000 by
+// 300 taps FP32 went from 158 to 36 us, 1024 x 2000 by 2000 taps FP64 from 77
+// to 20 us.
 //
 // LDS positions are padded by one point in 16, which spreads the strided
 // accesses of every pass over the banks (without, the last pass's stride of

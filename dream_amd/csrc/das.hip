@@ -1094,10 +1094,10 @@ __device__ __forceinline__ float lane_value(frames4 g, frames4 v)
 // block of `tb` transmits x 16 receivers, so that a small image is split over
 // many waves.  As in the forward a group of kG gathers
 // is issued before any is used, a row out of range for the whole wave is
-// skipped, and the bound is the address path of the gathers (25 L1 lookups
-// per 64-lane gather of a 16-byte record).  A wave that ran all transmits of
-// a chunk and reduced every row by shuffles spent 81 % of its cycles
-// waiting: 64 x 64 elements, 2^19 voxels, 8 frames, nearest-lower took 6.25 ms,
+// skipped, and the bound is the address path of the gathers (24 L1 lookups
+// per 64-lane gather of a 16-byte record, 0.97 a CU cycle).  A wave that ran
+// all transmits of a chunk and reduced every row by shuffles spent 81 % of its
+// cycles waiting: 64 x 64 elements, 2^19 voxels, 8 frames, nearest-lower took 6.25 ms,
 // now 3.0 (the forward 2.33); one FP32 frame of 48 x 48 over 30720 pixels,
 // linear, 330 us, now 95.
 //
@@ -1312,12 +1312,12 @@ das_adj_pixel_kernel(DasArgs A, const int32_t *__restrict__ perm, int64_t tile_e
 // their starts from the distance ranges to the region's bounding box as in the
 // region adjoint) and adds them into gY.  Apodization sums go to z_t and z_r
 // as in the pixel adjoint.  Bound by the latency of its gathers and LDS adds
-// at three waves per SIMD (four spill: 250 -> 276 us): its 59 instructions a
-// pair fill 43 % of the issue slots, the LDS is busy 34 % of the time and the
-// gathers' address path about as much.  A work-group per group of 2 x 4
+// at three waves per SIMD (four spill: 250 -> 276 us): its 54 instructions a
+// pair fill 39 % of the issue slots, the LDS is busy 33 % of the time and the
+// address path 49 %.  A work-group per group of 2 x 4
 // A-scans computed six legs, a bounding box and nine shuffle sums per 32 pairs
 // of a lane, 110 instructions a pair: 48 x 48 over 30720 pixels, linear, FP32
-// took 352 us, now 250.
+// took 352 us, now 255.
 constexpr int kPartI = 64;                      // transmits of a part, at most
 
 template <typename DT, typename GT, int TYPE, int INTERP, bool APOD>

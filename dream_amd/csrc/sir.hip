@@ -27,11 +27,11 @@
 // run (sir_runs.hpp): a bin's edge and a closed-form sum of 1/r per run, about
 // 75 FP64-rate instructions whatever its length, against 19.5 for each
 // sub-element.  Each point takes the walk its run-length model prices lowest.
-// FP64 instruction issue bounds all three.  Measured, steps -> runs: 16384
-// points x 32 elements of 0.4 x 10 mm (7 sub-elements a run, 80 % of issue
-// slots) 630 -> 410 us; 24 uneven problems of 5 .. 15 mm elements, FP32 out,
-// 3.70 -> 2.45 ms; 9 discs of 3.5 .. 7.5 mm over 4096 points (18 a run) 1.20 ->
-// 0.83 ms.
+// FP64 instruction issue bounds all three.  Measured per call, steps -> runs:
+// 16384 points x 32 elements of 0.4 x 10 mm (7 sub-elements a run, the VALU
+// busy 88 % of its capacity) 668 -> 415 us; 24 uneven problems of 5 .. 15 mm
+// elements, FP32 out (78 %), 3.77 -> 2.5 ms; 9 discs of 3.5 .. 7.5 mm over 4096
+// points (18 a run, 85 %) 1.20 -> 0.58 ms in the kernel.
 //
 // Sample index.  The index must equal the reference's FP64 sequence bit for
 // bit.  A fast estimate u = r*c1 - d/dt (r from the hardware rsqrt, about

@@ -238,8 +238,9 @@ int dream_hip_arr_annu(double alpha, const double *Ro, int64_t No, double dx, do
                        const double *focal, const double *apod, int do_apod, int apod_met,
                        double apod_par, double *h, int err_level, int *sir_err);
 /* Device-pointer variant (conventions of dream_hip_arr_rect_dev; Gr, focal
- * and apod stay on the host).  Allocates num_radii x No x nt doubles of
- * device scratch for the disc responses during the call. */
+ * and apod stay on the host).  Takes num_radii x No x nt doubles of device
+ * scratch for the disc responses: kept per thread up to 128 MB, else allocated
+ * for the call. */
 int dream_hip_arr_annu_dev(const double *Ro, int64_t No, double dx, double dy, double dt,
                            int64_t nt, int delay_type, const double *delay, double v, double cp,
                            int64_t num_radii, const double *Gr, int foc_met, const double *focal,
