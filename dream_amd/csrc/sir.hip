@@ -31,7 +31,7 @@
 // 16384 points x 32 elements of 0.4 x 10 mm (7 sub-elements a run, the VALU
 // busy 88 % of its capacity) 668 -> 415 us; 24 uneven problems of 5 .. 15 mm
 // elements, FP32 out (78 %), 3.77 -> 2.5 ms; 9 discs of 3.5 .. 7.5 mm over 4096
-// points (18 a run, 85 %) 1.20 -> 0.58 ms in the kernel.
+// points (18 a run, 85 %) 1.20 -> 0.56 ms in the kernel.
 //
 // Sample index.  The index must equal the reference's FP64 sequence bit for
 // bit.  A fast estimate u = r*c1 - d/dt (r from the hardware rsqrt, about
